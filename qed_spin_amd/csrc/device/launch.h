@@ -112,7 +112,7 @@ struct CsrView {
     int xcd = 0;                   // contiguous row ranges per XCD (grid padded to a multiple of 8)
     int unroll = 1;                // single-vector SpMV: gathers issued 4 or 8 entries at a time (same sums)
     int dict_n = 0;                // dictionary entries (u8 / u16 ids)
-    int lds_dict = 1;              // u8 ids: stage the dictionary in LDS
+    int lds_dict = 1;              // stage the dictionary in LDS when it fits there
     int wg = 256;                  // single-vector SpMV: threads per workgroup (256, 512, 1024)
     // SELL-64 layout (sell_ptr non-null): col / vals hold the entries slice by slice in groups of
     // four, entry k of row 64 s + j at sell_ptr[s] + 256 (k / 4) + 4 j + k % 4 (slices padded to

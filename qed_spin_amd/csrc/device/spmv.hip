@@ -19,38 +19,66 @@ template <int NV> struct Ptrs {
     void* out[NV];
 };
 
-// The dictionary an entry's value id points into: u8 ids read it from LDS (staged at kernel start),
-// u16 ids from global memory.
-struct Dict {
+// The dictionary an entry's value id points into. LD: in LDS (staged at kernel start, a complex value
+// as one 16-byte word), else in global memory. A lookup is a gather over a handful of lines, and the
+// vector cache serves one line per clock to lanes that do not share theirs with a neighbour, so a
+// dictionary in global memory costs as much as the gather of x itself (twice that for a complex value,
+// whose parts lie apart). With u16 ids read from global memory, then from LDS: a 9.4M-row real sector
+// (609 values) 1.236 -> 1.105 ms an apply, four interleaved vectors on a 1.43M-row complex one (405
+// values) 0.399 -> 0.367 ms.
+template <bool LD> struct Dict {
     const double* re;
     const double* im;
 };
 
-template <int WIDTH, bool VREAL>
-__device__ __forceinline__ Dict stage_dict(const CsrView& A, double* sre, double* sim) {
-    if constexpr (WIDTH == 1 || WIDTH == 3) {
-        if (A.lds_dict) {
-            for (int i = threadIdx.x; i < A.dict_n; i += blockDim.x) {
-                sre[i] = A.dict_re[i];
-                if constexpr (!VREAL) sim[i] = A.dict_im[i];
+extern __shared__ __align__(16) double lds_dict[];
+
+/// LDS bytes a launch with the dictionary staged needs.
+inline std::size_t dict_lds_bytes(const CsrView& A) {
+    return A.width == 0 ? 0 : static_cast<std::size_t>(A.dict_n) * (A.values_real ? 8 : 16);
+}
+/// The largest staged dictionary: with 1024-thread workgroups two copies per compute unit, 32 waves.
+constexpr std::size_t kLdsDictMax = 64 * 1024;
+inline bool dict_in_lds(const CsrView& A) { return A.lds_dict && dict_lds_bytes(A) <= kLdsDictMax; }
+
+template <int WIDTH, bool VREAL, bool LD> __device__ __forceinline__ Dict<LD> stage_dict(const CsrView& A) {
+    if constexpr (LD && WIDTH != 0) {
+        for (int i = threadIdx.x; i < A.dict_n; i += blockDim.x) {
+            if constexpr (VREAL) {
+                lds_dict[i] = A.dict_re[i];
+            } else {
+                lds_dict[2 * i] = A.dict_re[i];
+                lds_dict[2 * i + 1] = A.dict_im[i];
             }
-            __syncthreads();
-            return Dict{sre, sim};
         }
+        __syncthreads();
     }
-    return Dict{A.dict_re, A.dict_im};
+    return Dict<LD>{A.dict_re, A.dict_im};
 }
 
-template <int WIDTH, bool VREAL>
-__device__ __forceinline__ void value_at(const CsrView& A, const Dict& d, u64 e, double& vr, double& vi) {
-    if constexpr (WIDTH == 1) {
-        const u32 id = A.nt ? __builtin_nontemporal_load(static_cast<const u8*>(A.vals) + e) : static_cast<const u8*>(A.vals)[e];
+template <bool VREAL, bool LD> __device__ __forceinline__ void dict_value(const Dict<LD>& d, u32 id, double& vr, double& vi) {
+    if constexpr (LD) {
+        if constexpr (VREAL) {
+            vr = lds_dict[id];
+        } else {
+            const Zd z = reinterpret_cast<const Zd*>(lds_dict)[id];
+            vr = z.re;
+            vi = z.im;
+        }
+    } else {
         vr = d.re[id];
         if constexpr (!VREAL) vi = d.im[id];
+    }
+}
+
+template <int WIDTH, bool VREAL, bool LD>
+__device__ __forceinline__ void value_at(const CsrView& A, const Dict<LD>& d, u64 e, double& vr, double& vi) {
+    if constexpr (WIDTH == 1) {
+        const u32 id = A.nt ? __builtin_nontemporal_load(static_cast<const u8*>(A.vals) + e) : static_cast<const u8*>(A.vals)[e];
+        dict_value<VREAL, LD>(d, id, vr, vi);
     } else if constexpr (WIDTH == 2) {
         const u32 id = A.nt ? __builtin_nontemporal_load(static_cast<const u16*>(A.vals) + e) : static_cast<const u16*>(A.vals)[e];
-        vr = A.dict_re[id];
-        if constexpr (!VREAL) vi = A.dict_im[id];
+        dict_value<VREAL, LD>(d, id, vr, vi);
     } else {
         if constexpr (VREAL) {
             vr = static_cast<const double*>(A.vals)[e];
@@ -71,7 +99,12 @@ __device__ __forceinline__ i64 row_block(const CsrView& A) {
     return static_cast<i64>(blockIdx.x & 7u) * per + (blockIdx.x >> 3);
 }
 
-inline unsigned block_threads(const CsrView& A) { return (A.wg == 512 || A.wg == 1024) ? A.wg : 256; }
+/// Threads per workgroup; 1024 where smaller workgroups' copies of the dictionary would leave a compute
+/// unit short of waves.
+inline unsigned block_threads(const CsrView& A) {
+    if (dict_in_lds(A) && dict_lds_bytes(A) > 16 * 1024) return 1024;
+    return (A.wg == 512 || A.wg == 1024) ? A.wg : 256;
+}
 
 inline unsigned grid_blocks(const CsrView& A, u64 threads) {
     const u64 t = block_threads(A);
@@ -82,24 +115,21 @@ inline unsigned grid_blocks(const CsrView& A, u64 threads) {
 
 // Column and value of entry e. WIDTH 3: the u8 id packed in the top byte of the column word
 // (columns below 2^24), one 4-byte load per entry.
-template <int WIDTH, bool VREAL>
-__device__ __forceinline__ void load_entry(const CsrView& A, const Dict& d, u64 e, u32& c, double& vr, double& vi) {
+template <int WIDTH, bool VREAL, bool LD>
+__device__ __forceinline__ void load_entry(const CsrView& A, const Dict<LD>& d, u64 e, u32& c, double& vr, double& vi) {
     if constexpr (WIDTH == 3) {
         const u32 w = A.nt ? __builtin_nontemporal_load(A.col + e) : A.col[e];
         c = w & 0xFFFFFFu;
-        const u32 id = w >> 24;
-        vr = d.re[id];
-        if constexpr (!VREAL) vi = d.im[id];
+        dict_value<VREAL, LD>(d, w >> 24, vr, vi);
     } else {
         c = A.nt ? __builtin_nontemporal_load(A.col + e) : A.col[e];
-        value_at<WIDTH, VREAL>(A, d, e, vr, vi);
+        value_at<WIDTH, VREAL, LD>(A, d, e, vr, vi);
     }
 }
 
-template <int WIDTH, bool VREAL, bool REAL, int L, int NV, int U>
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int L, int NV, int U>
 __global__ __launch_bounds__(1024) void k_spmv(CsrView A, Ptrs<NV> v) {
-    __shared__ double sre[(WIDTH == 1 || WIDTH == 3) ? 256 : 1], sim[(WIDTH == 1 || WIDTH == 3) && !VREAL ? 256 : 1];
-    const Dict d = stage_dict<WIDTH, VREAL>(A, sre, sim);
+    const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / L;
     const int lane = static_cast<int>(gid % L);
@@ -130,7 +160,7 @@ __global__ __launch_bounds__(1024) void k_spmv(CsrView A, Ptrs<NV> v) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     vi[u] = 0.0;
-                    load_entry<WIDTH, VREAL>(A, d, e + u * L, c[u], vr[u], vi[u]);
+                    load_entry<WIDTH, VREAL, LD>(A, d, e + u * L, c[u], vr[u], vi[u]);
                 }
                 if constexpr (REAL && NV == 1) {
                     double x[U];
@@ -147,7 +177,7 @@ __global__ __launch_bounds__(1024) void k_spmv(CsrView A, Ptrs<NV> v) {
         for (; e < e1; e += L) {
             u32 c;
             double vr, vi = 0.0;
-            load_entry<WIDTH, VREAL>(A, d, e, c, vr, vi);
+            load_entry<WIDTH, VREAL, LD>(A, d, e, c, vr, vi);
             accumulate(c, vr, vi);
         }
     }
@@ -169,10 +199,9 @@ __global__ __launch_bounds__(1024) void k_spmv(CsrView A, Ptrs<NV> v) {
 }
 
 // Block-interleaved vectors: X[row * NV + k].
-template <int WIDTH, bool VREAL, bool REAL, int L, int NV>
-__global__ __launch_bounds__(256) void k_spmv_block(CsrView A, const void* X, void* Y) {
-    __shared__ double sre[(WIDTH == 1 || WIDTH == 3) ? 256 : 1], sim[(WIDTH == 1 || WIDTH == 3) && !VREAL ? 256 : 1];
-    const Dict d = stage_dict<WIDTH, VREAL>(A, sre, sim);
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int L, int NV>
+__global__ __launch_bounds__(1024) void k_spmv_block(CsrView A, const void* X, void* Y) {
+    const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / L;
     const int lane = static_cast<int>(gid % L);
@@ -184,7 +213,7 @@ __global__ __launch_bounds__(256) void k_spmv_block(CsrView A, const void* X, vo
         for (u64 e = e0 + lane; e < e1; e += L) {
             u32 c32;
             double vr, vi = 0.0;
-            load_entry<WIDTH, VREAL>(A, d, e, c32, vr, vi);
+            load_entry<WIDTH, VREAL, LD>(A, d, e, c32, vr, vi);
             const u64 c = c32;
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
@@ -240,16 +269,14 @@ template <class V> __device__ __forceinline__ V load_vec(const CsrView& A, const
 }
 
 // The four entries of the group at e (a multiple of four): columns and values.
-template <int WIDTH, bool VREAL>
-__device__ __forceinline__ void load_quad(const CsrView& A, const Dict& d, u64 e, u32* c, double* vr, double* vi) {
+template <int WIDTH, bool VREAL, bool LD>
+__device__ __forceinline__ void load_quad(const CsrView& A, const Dict<LD>& d, u64 e, u32* c, double* vr, double* vi) {
     const u32x4 w = load_vec<u32x4>(A, A.col + e);
     if constexpr (WIDTH == 3) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             c[u] = w[u] & 0xFFFFFFu;
-            const u32 id = w[u] >> 24;
-            vr[u] = d.re[id];
-            if constexpr (!VREAL) vi[u] = d.im[id];
+            dict_value<VREAL, LD>(d, w[u] >> 24, vr[u], vi[u]);
         }
     } else {
 #pragma unroll
@@ -257,17 +284,11 @@ __device__ __forceinline__ void load_quad(const CsrView& A, const Dict& d, u64 e
         if constexpr (WIDTH == 1) {
             const u8x4 id = load_vec<u8x4>(A, static_cast<const u8*>(A.vals) + e);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                vr[u] = d.re[id[u]];
-                if constexpr (!VREAL) vi[u] = d.im[id[u]];
-            }
+            for (int u = 0; u < 4; ++u) dict_value<VREAL, LD>(d, id[u], vr[u], vi[u]);
         } else if constexpr (WIDTH == 2) {
             const u16x4 id = load_vec<u16x4>(A, static_cast<const u16*>(A.vals) + e);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                vr[u] = A.dict_re[id[u]];
-                if constexpr (!VREAL) vi[u] = A.dict_im[id[u]];
-            }
+            for (int u = 0; u < 4; ++u) dict_value<VREAL, LD>(d, id[u], vr[u], vi[u]);
         } else {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -290,8 +311,8 @@ template <int ACC> __device__ __forceinline__ double tree(const double* s) {
 
 /// Row `row` of the SELL layout applied to the NV vectors: ACC partial sums per vector, entries in
 /// groups of four, U per round.
-template <int WIDTH, bool VREAL, bool REAL, int NV, int U, int ACC>
-__device__ __forceinline__ void sell_row_sums(const CsrView& A, const Dict& d, i64 row, const Ptrs<NV>& v,
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int NV, int U, int ACC>
+__device__ __forceinline__ void sell_row_sums(const CsrView& A, const Dict<LD>& d, i64 row, const Ptrs<NV>& v,
                                               double (&ar)[NV][ACC], double (&ai)[NV][ACC]) {
     static_assert(U % 4 == 0, "whole groups of four entries per round");
     const u32 n = A.nt ? __builtin_nontemporal_load(A.sell_len + row) : A.sell_len[row];
@@ -320,7 +341,7 @@ __device__ __forceinline__ void sell_row_sums(const CsrView& A, const Dict& d, i
         for (int u = 0; u < U; ++u) vi[u] = 0.0;
 #pragma unroll
         for (int g = 0; g < U / 4; ++g)
-            load_quad<WIDTH, VREAL>(A, d, first + static_cast<u64>(k / 4 + g) * 256, c + 4 * g, vr + 4 * g, vi + 4 * g);
+            load_quad<WIDTH, VREAL, LD>(A, d, first + static_cast<u64>(k / 4 + g) * 256, c + 4 * g, vr + 4 * g, vi + 4 * g);
         if constexpr (REAL && NV == 1) {
             double x[U];
 #pragma unroll
@@ -335,21 +356,20 @@ __device__ __forceinline__ void sell_row_sums(const CsrView& A, const Dict& d, i
     for (; k < n; k += 4) {   // the last groups, entries below n (k stays a multiple of four)
         u32 c[4];
         double vr[4], vi[4] = {0.0, 0.0, 0.0, 0.0};
-        load_quad<WIDTH, VREAL>(A, d, first + static_cast<u64>(k / 4) * 256, c, vr, vi);
+        load_quad<WIDTH, VREAL, LD>(A, d, first + static_cast<u64>(k / 4) * 256, c, vr, vi);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             if (k + static_cast<u32>(u) < n) accumulate(u % ACC, c[u], vr[u], vi[u]);
     }
 }
 
-template <int WIDTH, bool VREAL, bool REAL, int NV, int U, int ACC>
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int NV, int U, int ACC>
 __global__ __launch_bounds__(1024) void k_sell(CsrView A, Ptrs<NV> v) {
-    __shared__ double sre[(WIDTH == 1 || WIDTH == 3) ? 256 : 1], sim[(WIDTH == 1 || WIDTH == 3) && !VREAL ? 256 : 1];
-    const Dict d = stage_dict<WIDTH, VREAL>(A, sre, sim);
+    const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 row = row_block(A) * blockDim.x + threadIdx.x;
     if (row >= A.rows) return;
     double ar[NV][ACC], ai[NV][ACC];
-    sell_row_sums<WIDTH, VREAL, REAL, NV, U, ACC>(A, d, row, v, ar, ai);
+    sell_row_sums<WIDTH, VREAL, REAL, LD, NV, U, ACC>(A, d, row, v, ar, ai);
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
         if constexpr (REAL) static_cast<double*>(v.out[q])[row] = tree<ACC>(ar[q]);
@@ -361,17 +381,16 @@ __global__ __launch_bounds__(1024) void k_sell(CsrView A, Ptrs<NV> v) {
 // first step) written, and the workgroup's partial of <v, w> (the wavefronts' xor trees, then the
 // wavefronts in order) into partial[workgroup] -- the apply followed by axpy_dot, without writing
 // and reading w in between. k_lanczos_finish sums the partials in workgroup order.
-template <int WIDTH, bool VREAL, bool REAL, int U, int ACC>
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int U, int ACC>
 __global__ __launch_bounds__(1024) void k_sell_lanczos(CsrView A, Ptrs<1> v, const void* vprev, double beta,
                                                        double* partial) {
-    __shared__ double sre[(WIDTH == 1 || WIDTH == 3) ? 256 : 1], sim[(WIDTH == 1 || WIDTH == 3) && !VREAL ? 256 : 1];
     __shared__ double wr[16], wi[16];
-    const Dict d = stage_dict<WIDTH, VREAL>(A, sre, sim);
+    const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 row = row_block(A) * blockDim.x + threadIdx.x;
     double pr = 0.0, pi = 0.0;
     if (row < A.rows) {
         double ar[1][ACC], ai[1][ACC];
-        sell_row_sums<WIDTH, VREAL, REAL, 1, U, ACC>(A, d, row, v, ar, ai);
+        sell_row_sums<WIDTH, VREAL, REAL, LD, 1, U, ACC>(A, d, row, v, ar, ai);
         if constexpr (REAL) {
             double w = tree<ACC>(ar[0]);
             if (vprev) w = w - beta * static_cast<const double*>(vprev)[row];
@@ -434,10 +453,9 @@ __global__ __launch_bounds__(256) void k_lanczos_finish(const double* partial, i
 // Block-interleaved vectors X[row * NV + k] on the SELL layout. ACC lanes share a row, lane l
 // taking entries k = l, l + ACC, ... in order (the single-vector kernel's partial sums), combined
 // by the xor butterfly whose order is that kernel's tree: the same bits as single applies.
-template <int WIDTH, bool VREAL, bool REAL, int NV, int ACC>
-__global__ __launch_bounds__(256) void k_sell_block(CsrView A, const void* X, void* Y) {
-    __shared__ double sre[(WIDTH == 1 || WIDTH == 3) ? 256 : 1], sim[(WIDTH == 1 || WIDTH == 3) && !VREAL ? 256 : 1];
-    const Dict d = stage_dict<WIDTH, VREAL>(A, sre, sim);
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int NV, int ACC>
+__global__ __launch_bounds__(1024) void k_sell_block(CsrView A, const void* X, void* Y) {
+    const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / ACC;
     const int lane = static_cast<int>(gid % ACC);
@@ -451,7 +469,7 @@ __global__ __launch_bounds__(256) void k_sell_block(CsrView A, const void* X, vo
         for (u32 k = static_cast<u32>(lane); k < n; k += ACC) {
             u32 c32;
             double vr, vi = 0.0;
-            load_entry<WIDTH, VREAL>(A, d, sell_at(slice, j, k), c32, vr, vi);
+            load_entry<WIDTH, VREAL, LD>(A, d, sell_at(slice, j, k), c32, vr, vi);
             const u64 c = c32;
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
@@ -482,49 +500,84 @@ __global__ __launch_bounds__(256) void k_sell_block(CsrView A, const void* X, vo
     }
 }
 
-template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& A, const VecSet& v, hipStream_t st) {
-    const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows))), block(block_threads(A));
+/// Launch with the dictionary in LDS when it fits there (dict_in_lds), else from global memory: tag
+/// is std::true_type / std::false_type, lds the dynamic LDS bytes.
+template <int WIDTH, class F> void by_dict(const CsrView& A, F&& f) {
+    if constexpr (WIDTH == 0) {
+        f(std::false_type{}, std::size_t{0});
+    } else {
+        if (dict_in_lds(A)) f(std::true_type{}, dict_lds_bytes(A));
+        else f(std::false_type{}, std::size_t{0});
+    }
+}
+
+/// The vectors of the set in launches of 8, 4, 2 and 1: go(std::integral_constant<int, NV>, Ptrs<NV>).
+template <class F> void by_vectors(const VecSet& v, F&& go) {
     int done = 0;
+    auto next = [&](auto tag) {
+        constexpr int NV = decltype(tag)::value;
+        Ptrs<NV> p;
+        for (int k = 0; k < NV; ++k) {
+            p.in[k] = v.in[done + k];
+            p.out[k] = v.out[done + k];
+        }
+        go(tag, p);
+        done += NV;
+    };
     while (done < v.k) {
         const int rest = v.k - done;
-        const int nv = rest >= 8 ? 8 : rest >= 4 ? 4 : rest >= 2 ? 2 : 1;
-        auto go = [&](auto tag) {
-            constexpr int NV = decltype(tag)::value;
-            Ptrs<NV> p;
-            for (int k = 0; k < NV; ++k) {
-                p.in[k] = v.in[done + k];
-                p.out[k] = v.out[done + k];
-            }
-            if (A.sell_acc == 4) {
-                if (NV == 1 && A.unroll >= 16) hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 16, 4>), grid, block, 0, st, A, p);
-                else if (NV == 1 && A.unroll >= 8) hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 8, 4>), grid, block, 0, st, A, p);
-                else hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 4, 4>), grid, block, 0, st, A, p);
-            } else {
-                if (NV == 1 && A.unroll >= 16) hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 16, 1>), grid, block, 0, st, A, p);
-                else if (NV == 1 && A.unroll >= 8) hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 8, 1>), grid, block, 0, st, A, p);
-                else hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, NV, 4, 1>), grid, block, 0, st, A, p);
-            }
-        };
-        if (nv == 8) go(std::integral_constant<int, 8>{});
-        else if (nv == 4) go(std::integral_constant<int, 4>{});
-        else if (nv == 2) go(std::integral_constant<int, 2>{});
-        else go(std::integral_constant<int, 1>{});
-        done += nv;
+        if (rest >= 8) next(std::integral_constant<int, 8>{});
+        else if (rest >= 4) next(std::integral_constant<int, 4>{});
+        else if (rest >= 2) next(std::integral_constant<int, 2>{});
+        else next(std::integral_constant<int, 1>{});
     }
+}
+
+template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& A, const VecSet& v, hipStream_t st) {
+    const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows))), block(block_threads(A));
+    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+        by_vectors(v, [&](auto tag, const auto& p) {
+            constexpr int NV = decltype(tag)::value;
+#define QSA_SELL(U, ACC) hipLaunchKernelGGL((k_sell<WIDTH, VREAL, REAL, LD, NV, U, ACC>), grid, block, lds, st, A, p)
+            if (A.sell_acc == 4) {
+                if (NV == 1 && A.unroll >= 16) QSA_SELL((NV == 1 ? 16 : 4), 4);
+                else if (NV == 1 && A.unroll >= 8) QSA_SELL((NV == 1 ? 8 : 4), 4);
+                else QSA_SELL(4, 4);
+            } else {
+                if (NV == 1 && A.unroll >= 16) QSA_SELL((NV == 1 ? 16 : 4), 1);
+                else if (NV == 1 && A.unroll >= 8) QSA_SELL((NV == 1 ? 8 : 4), 1);
+                else QSA_SELL(4, 1);
+            }
+#undef QSA_SELL
+        });
+    });
+}
+
+/// Workgroup of the block kernels: 256 threads, or 1024 where a workgroup's copy of the dictionary is
+/// worth more than a few of its rows (2 KB).
+inline CsrView block_view(const CsrView& A) {
+    CsrView B = A;
+    B.wg = dict_in_lds(A) && dict_lds_bytes(A) > 2048 ? 1024 : 256;
+    return B;
 }
 
 template <int WIDTH, bool VREAL, bool REAL, int ACC>
 void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    CsrView B = A;
-    B.wg = 256;
-    const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(256);
-    switch (nv) {
-    case 1: hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, 1, ACC>), grid, block, 0, st, B, X, Y); break;
-    case 2: hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, 2, ACC>), grid, block, 0, st, B, X, Y); break;
-    case 4: hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, 4, ACC>), grid, block, 0, st, B, X, Y); break;
-    case 8: hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, 8, ACC>), grid, block, 0, st, B, X, Y); break;
-    default: break;
-    }
+    const CsrView B = block_view(A);
+    const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(block_threads(B));
+    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+#define QSA_SELL_BLOCK(NV) hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, LD, NV, ACC>), grid, block, lds, st, B, X, Y)
+        switch (nv) {
+        case 1: QSA_SELL_BLOCK(1); break;
+        case 2: QSA_SELL_BLOCK(2); break;
+        case 4: QSA_SELL_BLOCK(4); break;
+        case 8: QSA_SELL_BLOCK(8); break;
+        default: break;
+        }
+#undef QSA_SELL_BLOCK
+    });
 }
 template <int WIDTH, bool VREAL, bool REAL>
 void launch_sell_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
@@ -533,30 +586,19 @@ void launch_sell_block(const CsrView& A, int nv, const void* X, void* Y, hipStre
 }
 
 template <int WIDTH, bool VREAL, bool REAL, int L> void launch_set(const CsrView& A, const VecSet& v, hipStream_t st) {
-    const u64 threads = static_cast<u64>(A.rows) * L;
-    const dim3 grid(grid_blocks(A, threads)), block(block_threads(A));
-    int done = 0;
-    while (done < v.k) {
-        const int rest = v.k - done;
-        const int nv = rest >= 8 ? 8 : rest >= 4 ? 4 : rest >= 2 ? 2 : 1;
-        auto go = [&](auto tag) {
+    const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows) * L)), block(block_threads(A));
+    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+        by_vectors(v, [&](auto tag, const auto& p) {
             constexpr int NV = decltype(tag)::value;
-            Ptrs<NV> p;
-            for (int k = 0; k < NV; ++k) {
-                p.in[k] = v.in[done + k];
-                p.out[k] = v.out[done + k];
-            }
-            if (NV == 1 && A.unroll >= 8) hipLaunchKernelGGL((k_spmv<WIDTH, VREAL, REAL, L, NV, 8>), grid, block, 0, st, A, p);
-            else if (NV == 1 && A.unroll >= 4) hipLaunchKernelGGL((k_spmv<WIDTH, VREAL, REAL, L, NV, 4>), grid, block, 0, st, A, p);
-            else if (NV == 1 && A.unroll > 1) hipLaunchKernelGGL((k_spmv<WIDTH, VREAL, REAL, L, NV, 2>), grid, block, 0, st, A, p);
-            else hipLaunchKernelGGL((k_spmv<WIDTH, VREAL, REAL, L, NV, 1>), grid, block, 0, st, A, p);
-        };
-        if (nv == 8) go(std::integral_constant<int, 8>{});
-        else if (nv == 4) go(std::integral_constant<int, 4>{});
-        else if (nv == 2) go(std::integral_constant<int, 2>{});
-        else go(std::integral_constant<int, 1>{});
-        done += nv;
-    }
+#define QSA_SPMV(U) hipLaunchKernelGGL((k_spmv<WIDTH, VREAL, REAL, LD, L, NV, U>), grid, block, lds, st, A, p)
+            if (NV == 1 && A.unroll >= 8) QSA_SPMV((NV == 1 ? 8 : 1));
+            else if (NV == 1 && A.unroll >= 4) QSA_SPMV((NV == 1 ? 4 : 1));
+            else if (NV == 1 && A.unroll > 1) QSA_SPMV((NV == 1 ? 2 : 1));
+            else QSA_SPMV(1);
+#undef QSA_SPMV
+        });
+    });
 }
 
 template <int WIDTH, bool VREAL, bool REAL> void pick_lanes(const CsrView& A, const VecSet& v, hipStream_t st) {
@@ -571,17 +613,20 @@ template <int WIDTH, bool VREAL, bool REAL> void pick_lanes(const CsrView& A, co
 
 template <int WIDTH, bool VREAL, bool REAL, int L>
 void launch_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    CsrView B = A;
-    B.wg = 256;
-    const u64 threads = static_cast<u64>(A.rows) * L;
-    const dim3 grid(grid_blocks(B, threads)), block(256);
-    switch (nv) {
-    case 1: hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, L, 1>), grid, block, 0, st, A, X, Y); break;
-    case 2: hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, L, 2>), grid, block, 0, st, A, X, Y); break;
-    case 4: hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, L, 4>), grid, block, 0, st, A, X, Y); break;
-    case 8: hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, L, 8>), grid, block, 0, st, A, X, Y); break;
-    default: break;
-    }
+    const CsrView B = block_view(A);
+    const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * L)), block(block_threads(B));
+    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+#define QSA_SPMV_BLOCK(NV) hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, LD, L, NV>), grid, block, lds, st, B, X, Y)
+        switch (nv) {
+        case 1: QSA_SPMV_BLOCK(1); break;
+        case 2: QSA_SPMV_BLOCK(2); break;
+        case 4: QSA_SPMV_BLOCK(4); break;
+        case 8: QSA_SPMV_BLOCK(8); break;
+        default: break;
+        }
+#undef QSA_SPMV_BLOCK
+    });
 }
 
 template <int WIDTH, bool VREAL, bool REAL> void pick_lanes_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
@@ -731,15 +776,21 @@ bool sell_lanczos(const CsrView& A, bool real, const void* v, const void* vprev,
     auto go = [&](auto wd, auto vr, auto xr) {
         constexpr int W = decltype(wd)::value;
         constexpr bool VR = decltype(vr)::value, XR = decltype(xr)::value;
-        if (A.sell_acc == 4) {
-            if (A.unroll >= 16) hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 16, 4>), grid, block, 0, st, A, p, vprev, beta, partial);
-            else if (A.unroll >= 8) hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 8, 4>), grid, block, 0, st, A, p, vprev, beta, partial);
-            else hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 4, 4>), grid, block, 0, st, A, p, vprev, beta, partial);
-        } else {
-            if (A.unroll >= 16) hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 16, 1>), grid, block, 0, st, A, p, vprev, beta, partial);
-            else if (A.unroll >= 8) hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 8, 1>), grid, block, 0, st, A, p, vprev, beta, partial);
-            else hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, 4, 1>), grid, block, 0, st, A, p, vprev, beta, partial);
-        }
+        by_dict<W>(A, [&](auto in_lds, std::size_t lds) {
+            constexpr bool LD = decltype(in_lds)::value;
+#define QSA_SELL_LANCZOS(U, ACC) \
+    hipLaunchKernelGGL((k_sell_lanczos<W, VR, XR, LD, U, ACC>), grid, block, lds, st, A, p, vprev, beta, partial)
+            if (A.sell_acc == 4) {
+                if (A.unroll >= 16) QSA_SELL_LANCZOS(16, 4);
+                else if (A.unroll >= 8) QSA_SELL_LANCZOS(8, 4);
+                else QSA_SELL_LANCZOS(4, 4);
+            } else {
+                if (A.unroll >= 16) QSA_SELL_LANCZOS(16, 1);
+                else if (A.unroll >= 8) QSA_SELL_LANCZOS(8, 1);
+                else QSA_SELL_LANCZOS(4, 1);
+            }
+#undef QSA_SELL_LANCZOS
+        });
     };
     using T = std::true_type;
     using F = std::false_type;
