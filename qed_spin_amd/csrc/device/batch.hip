@@ -15,9 +15,9 @@
 // other blocks share the batch.
 //
 // SpMV: for R >= 8 one thread per (row, vector), the R threads of a row reading the same column and
-// value and gathering one contiguous line of R entries; for R < 8, 16 threads per row (R rounded
-// up to a power of two, 16 / that many lanes per (row, vector)) splitting the row's entries, summed
-// by a fixed xor butterfly.
+// value and gathering one contiguous line of R entries; for 1 < R < 8 a group of 2, 4 or 8 threads
+// per row (R rounded up), one vector each, that share the row's columns and value ids; for R = 1 eight
+// threads per row splitting its entries, summed by a fixed xor butterfly.
 //
 // The Lanczos scalars alpha, beta, the local-reorthogonalisation overlap, the active flags and the
 // step counter live on the device; a step needs no host synchronisation, so it is captured once
@@ -70,38 +70,137 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_wide(BatchView B, const
     }
 }
 
-// R < 8: RP = R rounded up to a power of two, LR = 16 / RP lanes per (row, vector), 16 threads per
-// row; lane l of a vector takes entries e0 + l, e0 + l + LR, ... (four lanes per (row, vector) at
-// R = 1 measured the same on the N = 28 continued fractions).
-template <int RP, int LR>
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_narrow(BatchView B, const Zd* X, Zd* Y) {
-    constexpr int TPR = RP * LR;
-    constexpr int slots = kThreads / TPR;
-    const Tile t = B.tiles[tile_id(B)];
-    const int R = B.R;
-    const int slot = threadIdx.x / TPR, w = threadIdx.x % TPR;
-    const int s = w / LR, lane = w % LR;
-    const bool live = s < R && pair_live(B, t.block, s);
-    // every thread of a row group runs the same rounds (the butterfly needs all of them)
-    for (u64 base = t.row_begin; base < t.row_end; base += slots) {
-        const u64 r = base + slot;
-        double ar = 0.0, ai = 0.0;
-        if (live && r < t.row_end) {
-            const u64 e0 = B.row_ptr[r], e1 = B.row_ptr[r + 1];
-            for (u64 e = e0 + lane; e < e1; e += LR) {
-                const u64 c = B.col[e];
-                const Zd v = entry_value(B, e);
-                const Zd x = X[c * R + s];
-                ar += v.re * x.re - v.im * x.im;
-                ai += v.re * x.im + v.im * x.re;
-            }
+/// A stored entry times its pair's factor.
+__device__ __forceinline__ Zd scaled(Zd v, double f) { return Zd{v.re * f, v.im * f}; }
+
+// 1 < R < 8: a row's group of RP = 2, 4 or 8 lanes (R rounded up), lane s holding vector s. The lanes
+// load the row's columns and value ids together, eight entries a round (each pair or quad of lanes
+// reads consecutive entries once), and pass them on by DPP; every lane then gathers its vector's entry,
+// a group's lanes one contiguous line, eight gathers in flight. The block's dictionary is in LDS. Each
+// lane keeps 16 / RP partial sums, entry k of the row in sum k mod (16 / RP), combined as an xor
+// butterfly over that many lanes would.
+//
+// What bounds it is the vector cache's address rate, one line per clock for lanes that do not share one
+// with a neighbour: with every lane of a row reading every column, id, and both halves of the value
+// from global memory (five loads per entry and lane, lanes splitting the row) the step's SpMV at
+// N = 24, R = 4 (9.07M rows, 2.2e8 entries) took 2.83 ms; so 1.68 ms, the first recurrence pass included.
+constexpr int kBatchDictMax = 1024;   // LDS dictionary entries of a tile's block (16 KB)
+
+/// The value of lane J of the caller's pair (Q = 2) or quad (Q = 4) of lanes.
+template <int Q, int J> __device__ __forceinline__ u32 group_lane(u32 v) {
+    constexpr int ctrl = Q == 2 ? (J == 0 ? 0xA0 : 0xF5) : J * 0x55;   // quad_perm
+    return static_cast<u32>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), ctrl, 0xF, 0xF, true));
+}
+template <int Q, int J> __device__ __forceinline__ double group_lane(double v) {
+    const u64 b = static_cast<u64>(__double_as_longlong(v));
+    const u64 lo = group_lane<Q, J>(static_cast<u32>(b)), hi = group_lane<Q, J>(static_cast<u32>(b >> 32));
+    return __longlong_as_double(static_cast<long long>(lo | (hi << 32)));
+}
+
+/// The dictionary of the tile's block into LDS (every thread of the workgroup calls it; the caller
+/// synchronises). Returns the block's first id.
+__device__ __forceinline__ u32 stage_block_dict(const BatchView& B, u32 block, Zd* dict) {
+    const u32 d0 = B.dict_begin[block], n = B.dict_begin[block + 1] - d0;
+    for (u32 i = threadIdx.x; i < n; i += blockDim.x) dict[i] = Zd{B.dict_re[d0 + i], B.dict_im[d0 + i]};
+    return d0;
+}
+
+/// The row offsets of the tile's rows, from its first entry (every thread calls it; the caller
+/// synchronises). Returns that first entry.
+__device__ __forceinline__ u64 stage_rows(const BatchView& B, const Tile& t, u32* rp) {
+    const u64 first = B.row_ptr[t.row_begin];
+    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
+    for (u32 i = threadIdx.x; i <= n; i += blockDim.x) rp[i] = static_cast<u32>(B.row_ptr[t.row_begin + i] - first);
+    return first;
+}
+
+extern __shared__ __align__(16) Zd batch_dict[];
+
+/// One row of the narrow SpMV for the caller's vector: entries [b0, b1) past `first`, x = stored X
+/// times fc.
+template <int RP, int J>
+__device__ __forceinline__ void narrow_gather(const BatchView& B, const Zd* X, const u32 (&c)[8 / (RP == 2 ? 2 : 4)],
+                                              u32 left, int s, bool live, Zd (&x)[8]) {
+    constexpr int Q = RP == 2 ? 2 : 4;
+    const u32 cj = group_lane<Q, J % Q>(c[J / Q]);
+    if (static_cast<u32>(J) < left && live) x[J] = X[static_cast<u64>(cj) * B.R + s];
+    if constexpr (J + 1 < 8) narrow_gather<RP, J + 1>(B, X, c, left, s, live, x);
+}
+template <int RP, bool LD, int J, int LR>
+__device__ __forceinline__ void narrow_sum(const u32 (&id)[8 / (RP == 2 ? 2 : 4)], const Zd (&v)[8 / (RP == 2 ? 2 : 4)],
+                                           u32 left, const Zd (&stored)[8], double fc, double (&ar)[LR],
+                                           double (&ai)[LR]) {
+    constexpr int Q = RP == 2 ? 2 : 4;
+    Zd w;
+    if constexpr (LD) {
+        w = batch_dict[group_lane<Q, J % Q>(id[J / Q])];
+    } else {
+        w = Zd{group_lane<Q, J % Q>(v[J / Q].re), group_lane<Q, J % Q>(v[J / Q].im)};
+    }
+    if (static_cast<u32>(J) < left) {
+        const Zd x = scaled(stored[J], fc);
+        ar[J % LR] += w.re * x.re - w.im * x.im;
+        ai[J % LR] += w.re * x.im + w.im * x.re;
+    }
+    if constexpr (J + 1 < 8) narrow_sum<RP, LD, J + 1, LR>(id, v, left, stored, fc, ar, ai);
+}
+
+template <int RP, bool LD>
+__device__ __forceinline__ Zd narrow_row(const BatchView& B, const Zd* X, u64 first, u32 d0, u32 b0, u32 b1, int s,
+                                         bool live, double fc) {
+    constexpr int Q = RP == 2 ? 2 : 4, NL = 8 / Q, LR = 16 / RP;
+    const u32 p = threadIdx.x & (Q - 1);
+    double ar[LR], ai[LR];
+#pragma unroll
+    for (int k = 0; k < LR; ++k) ar[k] = ai[k] = 0.0;
+    for (u32 e = b0; e < b1; e += 8) {   // one trip count for all lanes of the row
+        const u32 left = b1 - e;
+        u32 c[NL], id[NL];
+        Zd v[NL], x[8];
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const u32 k = static_cast<u32>(q * Q) + p;
+            const u64 at = first + e + (k < left ? k : left - 1);
+            c[q] = B.col[at];
+            id[q] = 0;
+            if constexpr (LD) id[q] = B.vid[at] - d0;
+            else v[q] = entry_value(B, at);
         }
 #pragma unroll
-        for (int off = LR / 2; off > 0; off >>= 1) {
-            ar += __shfl_xor(ar, off, LR);
-            ai += __shfl_xor(ai, off, LR);
+        for (int j = 0; j < 8; ++j) x[j] = Zd{0.0, 0.0};
+        narrow_gather<RP, 0>(B, X, c, left, s, live, x);
+        narrow_sum<RP, LD, 0, LR>(id, v, left, x, fc, ar, ai);
+    }
+    if constexpr (LR == 8) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            ar[k] += ar[k + 4];
+            ai[k] += ai[k + 4];
         }
-        if (live && r < t.row_end && lane == 0) Y[r * R + s] = Zd{ar, ai};
+    }
+    if constexpr (LR >= 4) {
+        ar[0] += ar[2];
+        ai[0] += ai[2];
+        ar[1] += ar[3];
+        ai[1] += ai[3];
+    }
+    return Zd{ar[0] + ar[1], ai[0] + ai[1]};
+}
+
+template <int RP, bool LD>
+__global__ __launch_bounds__(kThreads) void k_batch_spmv_narrow(BatchView B, const Zd* X, Zd* Y, const double* scur) {
+    __shared__ u32 rp[kBatchTileRows + 1];
+    const Tile t = B.tiles[tile_id(B)];
+    const u64 first = stage_rows(B, t, rp);
+    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
+    __syncthreads();
+    const int s = static_cast<int>(threadIdx.x % RP);
+    const bool live = s < B.R && pair_live(B, t.block, s);
+    const double fc = scur && live ? scur[static_cast<u64>(t.block) * B.R + s] : 1.0;
+    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
+    for (u32 r = threadIdx.x / RP; r < n; r += kThreads / RP) {
+        const Zd y = narrow_row<RP, LD>(B, X, first, d0, rp[r], rp[r + 1], s, live, fc);
+        if (live) Y[(t.row_begin + r) * B.R + s] = y;
     }
 }
 
@@ -134,7 +233,6 @@ __device__ __forceinline__ void tile_partial(const BatchView& B, double pr, doub
 // f (1 / beta of the step that made it): every read multiplies by f, which rounds exactly as the
 // stored product of a separate scaling pass would, so the results are the same bit for bit and the
 // pass is saved.
-__device__ __forceinline__ Zd scaled(Zd v, double f) { return Zd{v.re * f, v.im * f}; }
 
 __global__ __launch_bounds__(kThreads) void k_batch_spmv_wide_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
                                                                     Zd* W, const double* beta, double* partial,
@@ -174,20 +272,59 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_wide_fused(BatchView B,
     tile_partial(B, pr, pi, partial);
 }
 
-// The same for R = 1 (the continued fractions: one vector per block), THREADS threads per tile.
-// Each row's entries go to L lanes (lane l: entries e0 + l, e0 + l + L, ... in order) and the
-// lanes' sums meet in an xor butterfly; with L = 8 that is the arithmetic of the sector SpMV that
-// batch_spmv uses at R = 1, so W equals its product followed by batch_vec mode 0 bit for bit. The
-// partial of <V_cur, W> sums the tile's rows in row order, as mode 0 does with one row per
-// thread. Workgroups take the tiles in XCD-contiguous runs (workgroup w: tile (w mod 8) * per +
-// w / 8) unless a schedule is given, so each XCD's L2 sees neighbouring rows, as the sector SpMV's
-// row ranges do.
-template <int L, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_batch_spmv_one_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
-                                                                  Zd* W, const double* beta, double* partial,
-                                                                  const double* sprev, const double* scur) {
-    static_assert(THREADS % L == 0 && THREADS >= kBatchTileRows, "whole row groups; one LDS cell per row");
-    __shared__ double sr[kBatchTileRows], si[kBatchTileRows];
+// The same for R = 2 and 4, on the narrow SpMV: the group's lanes are the slots of batch_vec mode 0,
+// so the partials are its partials bit for bit. (R = 3, 5, 6 and 7 keep the separate pass: their
+// slots are not the groups' rows.)
+template <int RP, bool LD>
+__global__ __launch_bounds__(kThreads) void k_batch_spmv_narrow_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
+                                                                      Zd* W, const double* beta, double* partial,
+                                                                      const double* sprev, const double* scur) {
+    __shared__ u32 rp[kBatchTileRows + 1];
+    const Tile t = B.tiles[tile_id(B)];
+    const u64 first = stage_rows(B, t, rp);
+    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
+    __syncthreads();
+    const int s = static_cast<int>(threadIdx.x % RP);
+    const bool live = pair_live(B, t.block, s);
+    const u64 bs = static_cast<u64>(t.block) * RP + s;
+    const int step = *B.step;
+    const double b = beta[bs], fp = sprev ? sprev[bs] : 1.0, fc = scur ? scur[bs] : 1.0;
+    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
+    double pr = 0.0, pi = 0.0;
+    for (u32 r = threadIdx.x / RP; r < n; r += kThreads / RP) {
+        const u64 i = (t.row_begin + r) * RP + s;
+        Zd w = narrow_row<RP, LD>(B, Vcur, first, d0, rp[r], rp[r + 1], s, live, fc);
+        if (!live) continue;
+        if (step > 0) {
+            const Zd p = scaled(Vprev[i], fp);
+            w = Zd{w.re - b * p.re, w.im - b * p.im};
+        }
+        W[i] = w;
+        const Zd d = cdot(scaled(Vcur[i], fc), w);
+        pr += d.re;
+        pi += d.im;
+    }
+    tile_partial(B, pr, pi, partial);
+}
+
+// The same for R = 1 (the continued fractions: one vector per block). Each row's entries go to 8
+// lanes (lane l: entries e0 + l, e0 + l + 8, ... in order) and the lanes' sums meet in an xor
+// butterfly, the arithmetic of the sector SpMV that batch_spmv uses at R = 1. Two rows and two
+// entries of each are in flight per lane, the block's dictionary in LDS. The partial of <V_cur, W>
+// sums each group's rows in order, then the 32 groups by a fixed tree. Workgroups take the tiles in
+// XCD-contiguous runs (workgroup w: tile (w mod 8) * per + w / 8) unless a schedule is given, so each
+// XCD's L2 sees neighbouring rows, as the sector SpMV's row ranges do.
+//
+// With the value's two halves read from a dictionary in global memory (three gathers per entry in
+// place of one, each lane its own line) and one entry in flight, the step's SpMV at N = 26 (10.4M rows,
+// 1.5e8 entries) took 0.906 ms; so 0.785 ms.
+template <bool LD>
+__global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
+                                                                   Zd* W, const double* beta, double* partial,
+                                                                   const double* sprev, const double* scur) {
+    constexpr int L = 8, groups = kThreads / L, P = 2, U = 2;
+    __shared__ u32 rp[kBatchTileRows + 1];
+    __shared__ double sr[groups], si[groups];
     u32 tile;
     if (B.sched) {
         tile = B.sched[blockIdx.x];
@@ -197,58 +334,103 @@ __global__ __launch_bounds__(THREADS) void k_batch_spmv_one_fused(BatchView B, c
         if (tile >= B.n_tiles) return;   // the whole workgroup: the grid is rounded up to 8
     }
     const Tile t = B.tiles[tile];
-    constexpr int rows_per_pass = THREADS / L;
-    const int g = threadIdx.x / L, lane = threadIdx.x % L;
-    if (threadIdx.x < kBatchTileRows) {
-        sr[threadIdx.x] = 0.0;
-        si[threadIdx.x] = 0.0;
-    }
+    const u64 first = stage_rows(B, t, rp);
+    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
     __syncthreads();
+    const u32 g = threadIdx.x / L, lane = threadIdx.x % L;
+    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
+    double pr = 0.0, pi = 0.0;
     if (pair_live(B, t.block, 0)) {
         const int step = *B.step;
         const double b = beta[t.block];
         const double fp = sprev ? sprev[t.block] : 1.0, fc = scur ? scur[t.block] : 1.0;
-        // every thread of a row group runs the same rounds (the butterfly needs all of them)
-        for (u64 base = t.row_begin; base < t.row_end; base += rows_per_pass) {
-            const u64 r = base + g;
-            double ar = 0.0, ai = 0.0;
-            if (r < t.row_end) {
-                const u64 e0 = B.row_ptr[r], e1 = B.row_ptr[r + 1];
-                for (u64 e = e0 + lane; e < e1; e += L) {
-                    const u64 c = B.col[e];
-                    const Zd v = entry_value(B, e);
-                    const Zd x = scaled(Vcur[c], fc);
-                    ar += v.re * x.re - v.im * x.im;
-                    ai += v.re * x.im + v.im * x.re;
+        // every thread of the workgroup runs the same passes (the butterfly needs whole groups)
+        for (u32 base = 0; base < n; base += P * groups) {
+            u32 e[P], end[P];
+            double ar[P], ai[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const u32 r = base + static_cast<u32>(p * groups) + g;
+                e[p] = r < n ? rp[r] + lane : 0u;
+                end[p] = r < n ? rp[r + 1] : 0u;
+                ar[p] = ai[p] = 0.0;
+            }
+            bool more = true;
+            while (more) {
+                u32 c[P][U], id[P][U];
+                Zd v[P][U], x[P][U];
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const u32 k = e[p] + static_cast<u32>(u * L);
+                        c[p][u] = id[p][u] = 0;
+                        v[p][u] = x[p][u] = Zd{0.0, 0.0};
+                        if (k < end[p]) {
+                            c[p][u] = B.col[first + k];
+                            if constexpr (LD) id[p][u] = B.vid[first + k] - d0;
+                            else v[p][u] = entry_value(B, first + k);
+                        }
+                    }
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (e[p] + static_cast<u32>(u * L) < end[p]) x[p][u] = Vcur[c[p][u]];
+                more = false;
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (e[p] + static_cast<u32>(u * L) < end[p]) {
+                            if constexpr (LD) v[p][u] = batch_dict[id[p][u]];
+                            const Zd xs = scaled(x[p][u], fc);
+                            ar[p] += v[p][u].re * xs.re - v[p][u].im * xs.im;
+                            ai[p] += v[p][u].re * xs.im + v[p][u].im * xs.re;
+                        }
+                    e[p] += U * L;
+                    more = more || e[p] < end[p];
                 }
             }
 #pragma unroll
-            for (int off = L / 2; off > 0; off >>= 1) {
-                ar += __shfl_xor(ar, off, L);
-                ai += __shfl_xor(ai, off, L);
-            }
-            if (r < t.row_end && lane == 0) {
-                Zd w{ar, ai};
-                if (step > 0) {
-                    const Zd p = scaled(Vprev[r], fp);
-                    w = Zd{w.re - b * p.re, w.im - b * p.im};
+            for (int p = 0; p < P; ++p) {
+#pragma unroll
+                for (int off = L / 2; off > 0; off >>= 1) {
+                    ar[p] += __shfl_xor(ar[p], off, L);
+                    ai[p] += __shfl_xor(ai[p], off, L);
                 }
-                W[r] = w;
-                const Zd d = cdot(scaled(Vcur[r], fc), w);
-                sr[r - t.row_begin] = d.re;
-                si[r - t.row_begin] = d.im;
+                const u32 q = base + static_cast<u32>(p * groups) + g;
+                if (q < n && lane == 0) {
+                    const u64 r = t.row_begin + q;
+                    Zd w{ar[p], ai[p]};
+                    if (step > 0) {
+                        const Zd pv = scaled(Vprev[r], fp);
+                        w = Zd{w.re - b * pv.re, w.im - b * pv.im};
+                    }
+                    W[r] = w;
+                    const Zd d = cdot(scaled(Vcur[r], fc), w);
+                    pr += d.re;
+                    pi += d.im;
+                }
             }
         }
     }
+    if (lane == 0) {
+        sr[g] = pr;
+        si[g] = pi;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = 0.0, c = 0.0;
-        for (int q = 0; q < kBatchTileRows; ++q) {
-            a += sr[q];
-            c += si[q];
+    if (threadIdx.x < static_cast<u32>(groups)) {
+        double a = sr[threadIdx.x], c = si[threadIdx.x];
+#pragma unroll
+        for (int off = groups / 2; off > 0; off >>= 1) {
+            a += __shfl_xor(a, off, groups);
+            c += __shfl_xor(c, off, groups);
         }
-        partial[static_cast<u64>(tile) * 64 * 2] = a;
-        partial[static_cast<u64>(tile) * 64 * 2 + 1] = c;
+        if (threadIdx.x == 0) {
+            partial[static_cast<u64>(tile) * 64 * 2] = a;
+            partial[static_cast<u64>(tile) * 64 * 2 + 1] = c;
+        }
     }
 }
 
@@ -263,7 +445,8 @@ __global__ __launch_bounds__(THREADS) void k_batch_spmv_one_fused(BatchView B, c
 // Pairs no longer running are left alone.
 __global__ __launch_bounds__(kThreads) void k_batch_vec(BatchView B, int mode, const Zd* Vprev, const Zd* Vcur, Zd* W,
                                                         const double* coef, const Zd* zcoef, double threshold,
-                                                        double* partial, double* partial2, const double* vscale) {
+                                                        double* partial, double* partial2, const double* vscale,
+                                                        const double* pscale) {
     const Tile t = B.tiles[tile_id(B)];
     const int R = B.R, slots = kThreads / R;
     const int slot = threadIdx.x / R, s = threadIdx.x % R;
@@ -285,7 +468,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_vec(BatchView B, int mode, c
             if (mode == 0) {
                 if (step > 0) {
                     const double b = coef[bs];
-                    const Zd p = Vprev[i];
+                    const Zd p = scaled(Vprev[i], pscale ? pscale[bs] : 1.0);
                     w = Zd{w.re - b * p.re, w.im - b * p.im};
                     W[i] = w;
                 }
@@ -720,7 +903,17 @@ unsigned grid_for(u64 n) {
 
 }  // namespace
 
-void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st) {
+namespace {
+/// f(whether the blocks' dictionaries fit LDS one at a time, the dynamic LDS bytes).
+template <class F> void by_block_dict(const BatchView& B, F&& f) {
+    if (B.vid && B.dict_begin && B.dict_max > 0 && B.dict_max <= static_cast<u32>(kBatchDictMax))
+        f(std::true_type{}, static_cast<std::size_t>(B.dict_max) * sizeof(Zd));
+    else
+        f(std::false_type{}, std::size_t{0});
+}
+}  // namespace
+
+void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st, const double* scur) {
     if (!B.n_tiles) return;
     if (B.R == 1) {
         // one vector per block: the packed matrix is an ordinary CSR, applied by the sector SpMV
@@ -752,39 +945,49 @@ void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st) {
         return;
     }
     const dim3 grid(B.n_tiles), block(kThreads);
-    if (B.R >= 8) hipLaunchKernelGGL(k_batch_spmv_wide, grid, block, 0, st, B, X, Y);
-    else if (B.R == 1) hipLaunchKernelGGL((k_batch_spmv_narrow<1, 16>), grid, block, 0, st, B, X, Y);
-    else if (B.R == 2) hipLaunchKernelGGL((k_batch_spmv_narrow<2, 8>), grid, block, 0, st, B, X, Y);
-    else if (B.R <= 4) hipLaunchKernelGGL((k_batch_spmv_narrow<4, 4>), grid, block, 0, st, B, X, Y);
-    else hipLaunchKernelGGL((k_batch_spmv_narrow<8, 2>), grid, block, 0, st, B, X, Y);
+    if (B.R >= 8) {
+        hipLaunchKernelGGL(k_batch_spmv_wide, grid, block, 0, st, B, X, Y);
+        return;
+    }
+    by_block_dict(B, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+        if (B.R == 2) hipLaunchKernelGGL((k_batch_spmv_narrow<2, LD>), grid, block, lds, st, B, X, Y, scur);
+        else if (B.R <= 4) hipLaunchKernelGGL((k_batch_spmv_narrow<4, LD>), grid, block, lds, st, B, X, Y, scur);
+        else hipLaunchKernelGGL((k_batch_spmv_narrow<8, LD>), grid, block, lds, st, B, X, Y, scur);
+    });
 }
 
 bool batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
                       hipStream_t st, const double* sprev, const double* scur) {
-    // 1 < R < 8: a fused form of the narrow kernel (the terms of alpha through LDS to keep mode 0's
-    // summation order) made the chain24 T > 0 Lanczos runs slower (3.0 -> 3.7 s); the two kernels stay
-    if (B.R > 1 && B.R < 8) return false;
+    if (B.R == 3 || (B.R > 4 && B.R < 8)) return false;
     if (!B.n_tiles) return true;
-    if (B.R == 1) {
-        // 8 lanes per row (the lane count of the sector SpMV that batch_spmv uses at R = 1), 256
-        // threads: on the N = 28 continued fractions 1024 threads (two passes per tile) took 0.99 s
-        // for the 200 steps against 0.87 s, and 4 lanes per row 0.89 s
-        const u32 grid = B.sched ? B.n_tiles : (B.n_tiles + 7u) / 8u * 8u;
-        hipLaunchKernelGGL((k_batch_spmv_one_fused<8, kThreads>), dim3(grid), dim3(kThreads), 0, st, B, Vprev, Vcur, W,
-                           beta, partial, sprev, scur);
+    if (B.R >= 8) {
+        hipLaunchKernelGGL(k_batch_spmv_wide_fused, dim3(B.n_tiles), dim3(kThreads), 0, st, B, Vprev, Vcur, W, beta,
+                           partial, sprev, scur);
         return true;
     }
-    hipLaunchKernelGGL(k_batch_spmv_wide_fused, dim3(B.n_tiles), dim3(kThreads), 0, st, B, Vprev, Vcur, W, beta,
-                       partial, sprev, scur);
+    const dim3 grid(B.R > 1 || B.sched ? B.n_tiles : (B.n_tiles + 7u) / 8u * 8u), block(kThreads);
+    by_block_dict(B, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+        if (B.R == 1)
+            hipLaunchKernelGGL((k_batch_spmv_one_fused<LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta, partial,
+                               sprev, scur);
+        else if (B.R == 2)
+            hipLaunchKernelGGL((k_batch_spmv_narrow_fused<2, LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta,
+                               partial, sprev, scur);
+        else
+            hipLaunchKernelGGL((k_batch_spmv_narrow_fused<4, LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta,
+                               partial, sprev, scur);
+    });
     return true;
 }
 
 void batch_vec(const BatchView& B, int mode, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* coef,
                const Zd* zcoef, double threshold, double* partial, hipStream_t st, double* partial2,
-               const double* vscale) {
+               const double* vscale, const double* pscale) {
     if (!B.n_tiles) return;
     hipLaunchKernelGGL(k_batch_vec, dim3(B.n_tiles), dim3(kThreads), 0, st, B, mode, Vprev, Vcur, W, coef, zcoef,
-                       threshold, partial, partial2, vscale);
+                       threshold, partial, partial2, vscale, pscale);
 }
 
 void batch_finish(const BatchView& B, int kind, const double* partial, double* alpha_hist, double* beta_hist, Zd* ov,

@@ -94,7 +94,7 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     // and when every block stores dictionary ids and the dictionaries hold at most 2^16 values
     // together, 16-bit ids into their concatenation (2 bytes per entry instead of 16); else in full
     // (with 8 or more vectors the gathers dominate and a full value is one broadcast load).
-    std::vector<std::uint32_t> dict_off(ops_.size(), 0);
+    std::vector<std::uint32_t> dict_off(ops_.size() + 1, 0);
     bool ids = R_ < 8;
     std::uint64_t dict_total = 0;
     for (std::size_t b = 0; ids && b < ops_.size(); ++b) {
@@ -105,10 +105,13 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
         }
         dict_off[b] = static_cast<std::uint32_t>(dict_total);
         dict_total += static_cast<std::uint64_t>(A.dict_n);
+        dict_max_ = std::max(dict_max_, static_cast<std::uint32_t>(A.dict_n));
     }
     if (dict_total > (std::uint64_t{1} << 16)) ids = false;
     if (ids) {
         dict_n_ = static_cast<std::uint32_t>(dict_total);
+        dict_off.back() = dict_n_;
+        put(dict_begin_, dict_off, st);
         vid_.reset(std::max<std::uint64_t>(nnz_, 1) * 2);
         dict_re_.reset(dict_total * 8);
         dict_im_.reset(dict_total * 8);
@@ -262,6 +265,8 @@ dev::BatchView BatchedLanczos::view() const {
         B.dict_re = dict_re_.get<double>();
         B.dict_im = dict_im_.get<double>();
         B.dict_n = dict_n_;
+        B.dict_begin = dict_begin_.get<std::uint32_t>();
+        B.dict_max = dict_max_;
     }
     B.step = step_d_.get<int>();
     B.active = active_d_.get<int>();
@@ -375,23 +380,21 @@ void BatchedLanczos::run(int M, const std::vector<double>& breakdown_tol, bool l
     double* ib = inv_b_.get<double>();
     const double* tol = tol_d_.get<double>();
     const double thr = 1.49011611938476562e-08;   // sqrt(eps): LocalDGKS3's overlap threshold
-    // With the fused SpMV (R = 1 or R >= 8) the next vector is never scaled in place: each of the three
-    // buffers keeps a per-pair factor (1 / beta of the step that wrote it; 1 for the normalised
-    // start) that every read applies, which rounds as the scaling pass would (same results, one
-    // pass over the vectors fewer per step).
-    const bool defer = R_ == 1 || R_ >= 8;
+    // The next vector is never scaled in place: each of the three buffers keeps a per-pair factor
+    // (1 / beta of the step that wrote it; 1 for the normalised start) that every read applies, which
+    // rounds as a scaling pass would (same results, one pass over the vectors fewer per step).
     const std::size_t np = pairs;
     double* S[3] = {scale_.get<double>(), scale_.get<double>() + np, scale_.get<double>() + 2 * np};
     auto step = [&](int phase) {
         dev::Zd* p = V[phase % 3];
         dev::Zd* c = V[(phase + 1) % 3];
         dev::Zd* w = V[(phase + 2) % 3];
-        const double* sp = defer ? S[phase % 3] : nullptr;
-        const double* sc = defer ? S[(phase + 1) % 3] : nullptr;
-        double* sw = defer ? S[(phase + 2) % 3] : ib;
+        const double* sp = S[phase % 3];
+        const double* sc = S[(phase + 1) % 3];
+        double* sw = S[(phase + 2) % 3];
         if (!dev::batch_spmv_fused(B, p, c, w, cb, partial, st, sp, sc)) {
-            dev::batch_spmv(B, c, w, st);
-            dev::batch_vec(B, 0, p, c, w, cb, nullptr, 0.0, partial, st);
+            dev::batch_spmv(B, c, w, st, sc);
+            dev::batch_vec(B, 0, p, c, w, cb, nullptr, 0.0, partial, st, nullptr, sc, sp);
         }
         dev::batch_finish(B, 0, partial, ah, bh, ov, ca, cb, ib, tol, st);
         if (local) {
@@ -405,7 +408,6 @@ void BatchedLanczos::run(int M, const std::vector<double>& breakdown_tol, bool l
             dev::batch_vec(B, 4, nullptr, c, w, ca, nullptr, 0.0, partial, st, nullptr, sc);
             dev::batch_finish(B, 2, partial, ah, bh, ov, ca, cb, sw, tol, st);
         }
-        if (!defer) dev::batch_vec(B, 3, nullptr, nullptr, w, ib, nullptr, 0.0, partial, st);
         dev::batch_advance(B, st);
     };
     const int Mrun = *std::max_element(cap.begin(), cap.end());

@@ -96,7 +96,8 @@ private:
     std::vector<std::uint32_t> tile_begin_;
     DeviceBuffer row_ptr_, col_, val_, vid_, dict_re_, dict_im_, tiles_d_, tile_begin_d_, cap_d_, active_d_, steps_d_,
         step_d_;
-    std::uint32_t dict_n_ = 0;
+    std::uint32_t dict_n_ = 0, dict_max_ = 0;
+    DeviceBuffer dict_begin_;
     int sched_kind_ = 0;
     DeviceBuffer sched_d_;
     DeviceBuffer V0_, V1_, W_, partial_, partial2_, fix_, scale_, alpha_h_, beta_h_, ov_, cur_a_, cur_b_, inv_b_,
