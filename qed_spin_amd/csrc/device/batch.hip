@@ -14,14 +14,20 @@
 // order (LDS), then the block's tile sums by a fixed tree: deterministic, and independent of which
 // other blocks share the batch.
 //
-// SpMV: for R >= 8 one thread per (row, vector), the R threads of a row reading the same column and
-// value and gathering one contiguous line of R entries; for 1 < R < 8 a group of 2, 4 or 8 threads
-// per row (R rounded up), one vector each, that share the row's columns and value ids; for R = 1 eight
-// threads per row splitting its entries, summed by a fixed xor butterfly.
+// SpMV: for R > 1 a group of 2, 4 or 8 threads per row, one vector each, that share the row's columns
+// and value ids; above 8 vectors a work item is a tile and a run of eight of its vectors. For R = 1
+// eight threads per row splitting its entries, summed by a fixed xor butterfly.
+//
+// The order of a block's rows is the engine's own: blocks whose vectors (eight of them at most) do not
+// fit an XCD's L2 are stored by breadth-first level of their matrix's graph, the blocks' states'
+// order within a level. A row's columns then lie in its own and the two neighbouring levels, so with
+// the tiles of a block run in order on one XCD each entry of X comes from memory once.
 //
 // The Lanczos scalars alpha, beta, the local-reorthogonalisation overlap, the active flags and the
 // step counter live on the device; a step needs no host synchronisation, so it is captured once
 // as a hipGraph and replayed.
+#include <hipcub/hipcub.hpp>
+
 #include "dev_common.h"
 #include "launch.h"
 
@@ -31,12 +37,26 @@ namespace {
 
 constexpr int kThreads = 256;
 
+typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+typedef u16 u16x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ Zd cmul(Zd a, Zd b) { return Zd{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 __device__ __forceinline__ Zd cdot(Zd a, Zd b) { return Zd{a.re * b.re + a.im * b.im, a.re * b.im - a.im * b.re}; }
 
-/// The tile this workgroup runs: the schedule's entry (a permutation of the tiles), else its own
-/// index. Every tile's work and partial sums are the same whichever workgroup runs it.
-__device__ __forceinline__ u32 tile_id(const BatchView& B) { return B.sched ? B.sched[blockIdx.x] : blockIdx.x; }
+/// The SpMV work of a workgroup: a tile and a run of at most eight vectors (`chunk`), by the schedule's
+/// entry (tile * chunks + chunk, ~0: none) or, without one, in order. An item's work and partial sums
+/// are the same whichever workgroup runs it.
+struct Work {
+    u32 tile;
+    int chunk;
+    bool any;
+};
+__device__ __forceinline__ Work work_item(const BatchView& B, int chunks) {
+    const u32 id = B.sched ? B.sched[blockIdx.x] : blockIdx.x;
+    if (id == ~0u) return Work{0, 0, false};
+    if (chunks == 1) return Work{id, 0, true};
+    return Work{id / static_cast<u32>(chunks), static_cast<int>(id % static_cast<u32>(chunks)), true};
+}
 
 __device__ __forceinline__ bool pair_live(const BatchView& B, u32 block, int s) {
     return !B.active || B.active[static_cast<u64>(block) * B.R + s] != 0;
@@ -50,40 +70,24 @@ __device__ __forceinline__ Zd entry_value(const BatchView& B, u64 e) {
     return B.val[e];
 }
 
-// One thread per (row, vector), R >= 8.
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_wide(BatchView B, const Zd* X, Zd* Y) {
-    const Tile t = B.tiles[tile_id(B)];
-    const int R = B.R, slots = kThreads / R;
-    const int slot = threadIdx.x / R, s = threadIdx.x % R;
-    if (slot >= slots || !pair_live(B, t.block, s)) return;
-    for (u64 r = t.row_begin + slot; r < t.row_end; r += slots) {
-        const u64 e0 = B.row_ptr[r], e1 = B.row_ptr[r + 1];
-        double ar = 0.0, ai = 0.0;
-        for (u64 e = e0; e < e1; ++e) {
-            const u64 c = B.col[e];
-            const Zd v = entry_value(B, e);
-            const Zd x = X[c * R + s];
-            ar += v.re * x.re - v.im * x.im;
-            ai += v.re * x.im + v.im * x.re;
-        }
-        Y[r * R + s] = Zd{ar, ai};
-    }
-}
-
 /// A stored entry times its pair's factor.
 __device__ __forceinline__ Zd scaled(Zd v, double f) { return Zd{v.re * f, v.im * f}; }
 
-// 1 < R < 8: a row's group of RP = 2, 4 or 8 lanes (R rounded up), lane s holding vector s. The lanes
+// R > 1: a row's group of RP = 2, 4 or 8 lanes, lane s holding vector s of the item's run. The lanes
 // load the row's columns and value ids together, eight entries a round (each pair or quad of lanes
 // reads consecutive entries once), and pass them on by DPP; every lane then gathers its vector's entry,
 // a group's lanes one contiguous line, eight gathers in flight. The block's dictionary is in LDS. Each
-// lane keeps 16 / RP partial sums, entry k of the row in sum k mod (16 / RP), combined as an xor
-// butterfly over that many lanes would.
+// lane keeps two partial sums.
 //
-// What bounds it is the vector cache's address rate, one line per clock for lanes that do not share one
-// with a neighbour: with every lane of a row reading every column, id, and both halves of the value
-// from global memory (five loads per entry and lane, lanes splitting the row) the step's SpMV at
-// N = 24, R = 4 (9.07M rows, 2.2e8 entries) took 2.83 ms; so 1.68 ms, the first recurrence pass included.
+// What bounds it: with every lane of a row reading every column, id, and both halves of the value from
+// global memory, the vector cache's address rate (one line per clock for lanes that do not share one
+// with a neighbour); so it took 2.83 ms a step at N = 24, R = 4 (9.07M rows, 2.2e8 entries), and
+// 1.68 ms (the first recurrence pass included) with the group's lanes sharing their loads and the L2
+// missing on 77M lines a step: X fetched again and again, 870 bytes a row of 64. In level order the
+// misses are 27M (what the matrix and the vectors are) and the step 1.59 ms: the L1 fetches, a line
+// for almost every entry at 2.5 clocks, are left. At R = 40 a row's 640 bytes times the rows of the
+// tiles in flight fit an L2 in no order, hence the runs of eight vectors (a line): N = 22 (2.29M rows)
+// 3.54 -> 1.99 ms a step, 6.6 GB of memory traffic at 3.3 TB/s.
 constexpr int kBatchDictMax = 1024;   // LDS dictionary entries of a tile's block (16 KB)
 
 /// The value of lane J of the caller's pair (Q = 2) or quad (Q = 4) of lanes.
@@ -97,110 +101,310 @@ template <int Q, int J> __device__ __forceinline__ double group_lane(double v) {
     return __longlong_as_double(static_cast<long long>(lo | (hi << 32)));
 }
 
-/// The dictionary of the tile's block into LDS (every thread of the workgroup calls it; the caller
-/// synchronises). Returns the block's first id.
-__device__ __forceinline__ u32 stage_block_dict(const BatchView& B, u32 block, Zd* dict) {
+/// The dictionary of the tile's block into LDS, a zero after its last value (every thread of the
+/// workgroup calls it; the caller synchronises): the block's first id, and the zero's.
+struct BlockDict {
+    u32 first, zero;
+};
+__device__ __forceinline__ BlockDict stage_block_dict(const BatchView& B, u32 block, Zd* dict) {
     const u32 d0 = B.dict_begin[block], n = B.dict_begin[block + 1] - d0;
     for (u32 i = threadIdx.x; i < n; i += blockDim.x) dict[i] = Zd{B.dict_re[d0 + i], B.dict_im[d0 + i]};
-    return d0;
-}
-
-/// The row offsets of the tile's rows, from its first entry (every thread calls it; the caller
-/// synchronises). Returns that first entry.
-__device__ __forceinline__ u64 stage_rows(const BatchView& B, const Tile& t, u32* rp) {
-    const u64 first = B.row_ptr[t.row_begin];
-    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
-    for (u32 i = threadIdx.x; i <= n; i += blockDim.x) rp[i] = static_cast<u32>(B.row_ptr[t.row_begin + i] - first);
-    return first;
+    if (threadIdx.x == 0) dict[n] = Zd{0.0, 0.0};
+    return BlockDict{d0, n};
 }
 
 extern __shared__ __align__(16) Zd batch_dict[];
 
-/// One row of the narrow SpMV for the caller's vector: entries [b0, b1) past `first`, x = stored X
-/// times fc.
-template <int RP, int J>
-__device__ __forceinline__ void narrow_gather(const BatchView& B, const Zd* X, const u32 (&c)[8 / (RP == 2 ? 2 : 4)],
-                                              u32 left, int s, bool live, Zd (&x)[8]) {
-    constexpr int Q = RP == 2 ? 2 : 4;
-    const u32 cj = group_lane<Q, J % Q>(c[J / Q]);
-    if (static_cast<u32>(J) < left && live) x[J] = X[static_cast<u64>(cj) * B.R + s];
-    if constexpr (J + 1 < 8) narrow_gather<RP, J + 1>(B, X, c, left, s, live, x);
-}
-template <int RP, bool LD, int J, int LR>
-__device__ __forceinline__ void narrow_sum(const u32 (&id)[8 / (RP == 2 ? 2 : 4)], const Zd (&v)[8 / (RP == 2 ? 2 : 4)],
-                                           u32 left, const Zd (&stored)[8], double fc, double (&ar)[LR],
-                                           double (&ai)[LR]) {
-    constexpr int Q = RP == 2 ? 2 : 4;
-    Zd w;
-    if constexpr (LD) {
-        w = batch_dict[group_lane<Q, J % Q>(id[J / Q])];
-    } else {
-        w = Zd{group_lane<Q, J % Q>(v[J / Q].re), group_lane<Q, J % Q>(v[J / Q].im)};
-    }
-    if (static_cast<u32>(J) < left) {
-        const Zd x = scaled(stored[J], fc);
-        ar[J % LR] += w.re * x.re - w.im * x.im;
-        ai[J % LR] += w.re * x.im + w.im * x.re;
-    }
-    if constexpr (J + 1 < 8) narrow_sum<RP, LD, J + 1, LR>(id, v, left, stored, fc, ar, ai);
+// ar + i ai += v x, by fused multiply-adds.
+__device__ __forceinline__ void zfma(Zd v, Zd x, double& ar, double& ai) {
+    ar = __builtin_fma(v.re, x.re, ar);
+    ai = __builtin_fma(v.re, x.im, ai);
+    ar = __builtin_fma(-v.im, x.im, ar);
+    ai = __builtin_fma(v.im, x.re, ai);
 }
 
-template <int RP, bool LD>
-__device__ __forceinline__ Zd narrow_row(const BatchView& B, const Zd* X, u64 first, u32 d0, u32 b0, u32 b1, int s,
-                                         bool live, double fc) {
-    constexpr int Q = RP == 2 ? 2 : 4, NL = 8 / Q, LR = 16 / RP;
-    const u32 p = threadIdx.x & (Q - 1);
-    double ar[LR], ai[LR];
-#pragma unroll
-    for (int k = 0; k < LR; ++k) ar[k] = ai[k] = 0.0;
-    for (u32 e = b0; e < b1; e += 8) {   // one trip count for all lanes of the row
-        const u32 left = b1 - e;
-        u32 c[NL], id[NL];
-        Zd v[NL], x[8];
+/// Four entries of the caller's row: their columns and value ids (values), one to each lane of a quad
+/// (RP = 2: two to each lane of a pair). Past the row's end, its last entry with value zero.
+template <int RP, bool LD> struct Quad {
+    static constexpr int Q = RP == 2 ? 2 : 4, NL = 4 / Q;
+    u32 c[NL], id[NL];
+    Zd v[NL];
+    __device__ __forceinline__ void load(const BatchView& B, u64 first, u32 d0, u32 zero, u32 e, u32 b1) {
+        const u32 p = threadIdx.x & (Q - 1);
 #pragma unroll
         for (int q = 0; q < NL; ++q) {
-            const u32 k = static_cast<u32>(q * Q) + p;
-            const u64 at = first + e + (k < left ? k : left - 1);
+            const u32 k = e + static_cast<u32>(q * Q) + p;
+            const u64 at = first + (k < b1 ? k : b1 - 1);
             c[q] = B.col[at];
-            id[q] = 0;
-            if constexpr (LD) id[q] = B.vid[at] - d0;
-            else v[q] = entry_value(B, at);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = Zd{0.0, 0.0};
-        narrow_gather<RP, 0>(B, X, c, left, s, live, x);
-        narrow_sum<RP, LD, 0, LR>(id, v, left, x, fc, ar, ai);
-    }
-    if constexpr (LR == 8) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            ar[k] += ar[k + 4];
-            ai[k] += ai[k + 4];
+            if constexpr (LD) {
+                const u32 i = B.vid[at] - d0;
+                id[q] = k < b1 ? i : zero;
+            } else {
+                const Zd w = entry_value(B, at);
+                v[q] = k < b1 ? w : Zd{0.0, 0.0};
+            }
         }
     }
-    if constexpr (LR >= 4) {
-        ar[0] += ar[2];
-        ai[0] += ai[2];
-        ar[1] += ar[3];
-        ai[1] += ai[3];
+    template <int J> __device__ __forceinline__ Zd gather(const char* X, u32 stride) const {
+        return *reinterpret_cast<const Zd*>(X + static_cast<u64>(group_lane<Q, J % Q>(c[J / Q])) * stride);
     }
-    return Zd{ar[0] + ar[1], ai[0] + ai[1]};
+    template <int J> __device__ __forceinline__ Zd value() const {
+        if constexpr (LD) return batch_dict[group_lane<Q, J % Q>(id[J / Q])];
+        else return Zd{group_lane<Q, J % Q>(v[J / Q].re), group_lane<Q, J % Q>(v[J / Q].im)};
+    }
+};
+
+/// One row of the SpMV for the caller's vector: entries [b0, b1) past `first`; X at the vector's first
+/// entry, `stride` bytes between rows, `zero` the dictionary's zero. Eight gathers in flight, the next
+/// eight entries' columns and ids loaded behind them. Two partial sums (entries 0 to 3 and 4 to 7 of
+/// each round).
+template <int RP, bool LD>
+__device__ __forceinline__ Zd group_row(const BatchView& B, const char* X, u32 stride, u64 first, u32 d0, u32 zero, u32 b0,
+                                        u32 b1) {
+    double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0;
+    if (b0 >= b1) return Zd{0.0, 0.0};   // one answer, and one trip count below, for all lanes of the row
+    Quad<RP, LD> lo, hi;
+    lo.load(B, first, d0, zero, b0, b1);
+    hi.load(B, first, d0, zero, b0 + 4, b1);
+    for (u32 e = b0;;) {
+        const Zd x0 = lo.template gather<0>(X, stride), x1 = lo.template gather<1>(X, stride),
+                 x2 = lo.template gather<2>(X, stride), x3 = lo.template gather<3>(X, stride);
+        Zd x4{0.0, 0.0}, x5{0.0, 0.0}, x6{0.0, 0.0}, x7{0.0, 0.0};
+        const Quad<RP, LD> a = lo, b = hi;
+        if (e + 4 < b1) {
+            x4 = b.template gather<0>(X, stride);
+            x5 = b.template gather<1>(X, stride);
+            x6 = b.template gather<2>(X, stride);
+            x7 = b.template gather<3>(X, stride);
+        }
+        e += 8;
+        const bool more = e < b1;
+        if (more) {
+            lo.load(B, first, d0, zero, e, b1);
+            hi.load(B, first, d0, zero, e + 4, b1);
+        }
+        zfma(a.template value<0>(), x0, ar, ai);
+        zfma(a.template value<1>(), x1, ar, ai);
+        zfma(a.template value<2>(), x2, ar, ai);
+        zfma(a.template value<3>(), x3, ar, ai);
+        zfma(b.template value<0>(), x4, br, bi);
+        zfma(b.template value<1>(), x5, br, bi);
+        zfma(b.template value<2>(), x6, br, bi);
+        zfma(b.template value<3>(), x7, br, bi);
+        if (!more) break;
+    }
+    return Zd{ar + br, ai + bi};
 }
 
-template <int RP, bool LD>
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_narrow(BatchView B, const Zd* X, Zd* Y, const double* scur) {
+/// Threads of the grouped SpMV: more rows per pass in fewer workgroups keep the rows in flight on an XCD
+/// (resident workgroups times a tile) close together.
+constexpr int kGroupThreads = 512;
+
+/// Y = A X, or (FUSED) the first recurrence pass with it: W = H V_cur - beta V_prev (beta of this step;
+/// skipped at step 0) and the partial of <V_cur, W> (a group's lanes' rows in order, the wave's groups
+/// by an xor tree, then the waves in order).
+///
+/// With sprev / scur the stored vectors are the unnormalised ones and V = U f with the pair's factor
+/// f (1 / beta of the step that made it), applied to the row's sum and to V_prev: no separate scaling
+/// pass over the vectors.
+template <int RP, bool LD, bool FUSED>
+__global__ __launch_bounds__(kGroupThreads) void k_batch_spmv_group(BatchView B, int chunks, const Zd* Vprev,
+                                                                    const Zd* X, Zd* Y, const double* beta,
+                                                                    double* partial, const double* sprev,
+                                                                    const double* scur) {
     __shared__ u32 rp[kBatchTileRows + 1];
-    const Tile t = B.tiles[tile_id(B)];
-    const u64 first = stage_rows(B, t, rp);
-    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
-    __syncthreads();
-    const int s = static_cast<int>(threadIdx.x % RP);
-    const bool live = s < B.R && pair_live(B, t.block, s);
-    const double fc = scur && live ? scur[static_cast<u64>(t.block) * B.R + s] : 1.0;
+    __shared__ double sr[FUSED ? kGroupThreads / 64 * RP : 1], si[FUSED ? kGroupThreads / 64 * RP : 1];
+    const Work w = work_item(B, chunks);
+    if (!w.any) return;   // the whole workgroup
+    const Tile t = B.tiles[w.tile];
+    const u64 first = B.row_ptr[t.row_begin];
     const u32 n = static_cast<u32>(t.row_end - t.row_begin);
-    for (u32 r = threadIdx.x / RP; r < n; r += kThreads / RP) {
-        const Zd y = narrow_row<RP, LD>(B, X, first, d0, rp[r], rp[r + 1], s, live, fc);
-        if (live) Y[(t.row_begin + r) * B.R + s] = y;
+    for (u32 i = threadIdx.x; i <= n; i += kGroupThreads) rp[i] = static_cast<u32>(B.row_ptr[t.row_begin + i] - first);
+    BlockDict dict{0, 0};
+    if constexpr (LD) dict = stage_block_dict(B, t.block, batch_dict);
+    __syncthreads();
+    const int R = B.R, lane = static_cast<int>(threadIdx.x % RP), s = w.chunk * 8 + lane;
+    const bool live = s < R && pair_live(B, t.block, s);
+    const int sv = s < R ? s : R - 1;   // idle lanes gather what a neighbour does
+    const u64 bs = static_cast<u64>(t.block) * R + sv;
+    const double fc = scur ? scur[bs] : 1.0;
+    const bool sub = FUSED && *B.step > 0;
+    const double b = sub ? beta[bs] * (sprev ? sprev[bs] : 1.0) : 0.0;
+    const u32 stride = static_cast<u32>(R) * 16u;
+    const char* Xs = reinterpret_cast<const char*>(X + sv);
+    double pr = 0.0, pi = 0.0;
+    for (u32 r = threadIdx.x / RP; r < n; r += kGroupThreads / RP) {
+        const u64 i = (t.row_begin + r) * R + sv;
+        Zd p{0.0, 0.0}, x{0.0, 0.0};
+        if constexpr (FUSED) {
+            if (sub) p = Vprev[i];
+            x = X[i];
+        }
+        Zd y = scaled(group_row<RP, LD>(B, Xs, stride, first, dict.first, dict.zero, rp[r], rp[r + 1]), fc);
+        if (!live) continue;
+        if constexpr (FUSED) {
+            y = Zd{y.re - b * p.re, y.im - b * p.im};
+            const Zd d = cdot(scaled(x, fc), y);
+            pr += d.re;
+            pi += d.im;
+        }
+        Y[i] = y;
+    }
+    if constexpr (FUSED) {
+#pragma unroll
+        for (int off = 32; off >= RP; off >>= 1) {
+            pr += __shfl_xor(pr, off, 64);
+            pi += __shfl_xor(pi, off, 64);
+        }
+        const u32 wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63u) < static_cast<u32>(RP)) {
+            sr[wave * RP + lane] = pr;
+            si[wave * RP + lane] = pi;
+        }
+        __syncthreads();
+        if (threadIdx.x < static_cast<u32>(RP) && s < R) {
+            double a = 0.0, c = 0.0;
+            for (int q = 0; q < kGroupThreads / 64; ++q) {
+                a += sr[q * RP + lane];
+                c += si[q * RP + lane];
+            }
+            partial[(static_cast<u64>(w.tile) * 64 + s) * 2] = a;
+            partial[(static_cast<u64>(w.tile) * 64 + s) * 2 + 1] = c;
+        }
+    }
+}
+
+// The fused pass for R = 1 (the continued fractions: one vector per block), on slices of 64 rows of a
+// tile: one lane per row, its entries in groups of four (OneView), eight gathers in flight and two
+// partial sums. With eight lanes per row on the packed CSR, the value's two halves read from a
+// dictionary in global memory and one entry in flight, the step at N = 26 (10.4M rows, 1.5e8 entries)
+// took 0.906 ms; with the dictionary in LDS and four entries in flight 0.785 ms, in level order
+// (L2 misses 26.7M -> 10.7M lines) 0.769 ms: latency, every row being a chain of loads for a couple of
+// entries per lane. So: 0.626 ms.
+template <bool LD>
+__global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, const Zd* Vprev,
+                                                                   const Zd* Vcur, Zd* W, const double* beta,
+                                                                   double* partial, const double* sprev,
+                                                                   const double* scur) {
+    static_assert(kThreads == kBatchTileRows, "a thread per row of a tile");
+    __shared__ double sr[kThreads / 64], si[kThreads / 64];
+    const OneView& S = B.one;
+    const Work w = work_item(B, 1);
+    if (!w.any) return;   // the whole workgroup
+    const Tile t = B.tiles[w.tile];
+    const u64 r = t.row_begin + threadIdx.x;
+    const bool on = r < t.row_end && pair_live(B, t.block, 0);
+    const u32 n = on ? S.len[r] : 0u;
+    const u64 at = S.ptr[static_cast<u64>(w.tile) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] + (threadIdx.x & 63u) * 4u;
+    if constexpr (LD) {
+        (void)stage_block_dict(B, t.block, batch_dict);
+        __syncthreads();
+    }
+    double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0;
+    for (u32 k = 0; k < n; k += 8) {
+        u32x4 c[2];
+        u16x4 id[2];
+        Zd v[8], x[8];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const u64 e = at + static_cast<u64>(k / 4 + static_cast<u32>(g)) * 256;
+            c[g] = *reinterpret_cast<const u32x4*>(S.col + e);
+            if constexpr (LD) {
+                id[g] = *reinterpret_cast<const u16x4*>(S.vid + e);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[4 * g + u] = S.val[e + static_cast<u64>(u)];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = Vcur[c[u / 4][u % 4]];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if constexpr (LD) v[u] = batch_dict[id[u / 4][u % 4]];
+            if (u < 4) zfma(v[u], x[u], ar, ai);
+            else zfma(v[u], x[u], br, bi);
+        }
+    }
+    double pr = 0.0, pi = 0.0;
+    if (on) {
+        const double fc = scur ? scur[t.block] : 1.0;
+        Zd y = scaled(Zd{ar + br, ai + bi}, fc);
+        if (*B.step > 0) {
+            const double b = beta[t.block] * (sprev ? sprev[t.block] : 1.0);
+            const Zd p = Vprev[r];
+            y = Zd{y.re - b * p.re, y.im - b * p.im};
+        }
+        W[r] = y;
+        const Zd d = cdot(scaled(Vcur[r], fc), y);
+        pr = d.re;
+        pi = d.im;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        pr += __shfl_xor(pr, off, 64);
+        pi += __shfl_xor(pi, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) {
+        sr[threadIdx.x >> 6] = pr;
+        si[threadIdx.x >> 6] = pi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a = 0.0, c = 0.0;
+        for (int q = 0; q < kThreads / 64; ++q) {
+            a += sr[q];
+            c += si[q];
+        }
+        partial[static_cast<u64>(w.tile) * 64 * 2] = a;
+        partial[static_cast<u64>(w.tile) * 64 * 2 + 1] = c;
+    }
+}
+
+// The slices of the R = 1 layout: entries of each slice (64 lanes times its longest row in whole groups
+// of eight), the rows' lengths, then the entries; past a row's end its own row with value zero.
+__global__ __launch_bounds__(kThreads) void k_one_lengths(BatchView B, u32* len, u64* slice) {
+    const Tile t = B.tiles[blockIdx.x];
+    const u64 r = t.row_begin + threadIdx.x;
+    u32 n = 0;
+    if (r < t.row_end) {
+        n = static_cast<u32>(B.row_ptr[r + 1] - B.row_ptr[r]);
+        len[r] = n;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const u32 o = static_cast<u32>(__shfl_xor(static_cast<int>(n), off, 64));
+        n = o > n ? o : n;
+    }
+    if ((threadIdx.x & 63u) == 0)
+        slice[static_cast<u64>(blockIdx.x) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] = static_cast<u64>((n + 7u) & ~7u) * 64;
+}
+
+__global__ __launch_bounds__(kThreads) void k_one_fill(BatchView B, const u64* slice, u32* col, u16* vid, Zd* val) {
+    const Tile t = B.tiles[blockIdx.x];
+    const u64 r = t.row_begin + threadIdx.x;
+    if (r >= t.row_end) return;
+    const u64 from = B.row_ptr[r];
+    const u32 n = static_cast<u32>(B.row_ptr[r + 1] - from), end = (n + 7u) & ~7u;
+    const u64 at = slice[static_cast<u64>(blockIdx.x) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] + (threadIdx.x & 63u) * 4u;
+    const u32 d0 = vid ? B.dict_begin[t.block] : 0u, zero = vid ? B.dict_begin[t.block + 1] - d0 : 0u;
+    for (u32 k = 0; k < end; k += 4) {
+        u32x4 c;
+        u16x4 id;
+        Zd v[4];
+#pragma unroll
+        for (u32 u = 0; u < 4; ++u) {
+            const bool in = k + u < n;
+            c[u] = in ? B.col[from + k + u] : static_cast<u32>(r);
+            if (vid) id[u] = static_cast<u16>(in ? B.vid[from + k + u] - d0 : zero);
+            else v[u] = in ? entry_value(B, from + k + u) : Zd{0.0, 0.0};
+        }
+        const u64 e = at + static_cast<u64>(k / 4) * 256;
+        *reinterpret_cast<u32x4*>(col + e) = c;
+        if (vid) {
+            *reinterpret_cast<u16x4*>(vid + e) = id;
+        } else {
+            for (u32 u = 0; u < 4; ++u) val[e + u] = v[u];
+        }
     }
 }
 
@@ -214,227 +418,17 @@ __device__ __forceinline__ void tile_partial(const BatchView& B, double pr, doub
     si[threadIdx.x] = pi;
     __syncthreads();
     if (static_cast<int>(threadIdx.x) < R &&
-        (!only || only[static_cast<u64>(B.tiles[tile_id(B)].block) * R + threadIdx.x])) {
+        (!only || only[static_cast<u64>(B.tiles[blockIdx.x].block) * R + threadIdx.x])) {
         double a = 0.0, b = 0.0;
         for (int q = 0; q < slots; ++q) {
             a += sr[q * R + threadIdx.x];
             b += si[q * R + threadIdx.x];
         }
-        partial[(static_cast<u64>(tile_id(B)) * 64 + threadIdx.x) * 2] = a;
-        partial[(static_cast<u64>(tile_id(B)) * 64 + threadIdx.x) * 2 + 1] = b;
+        partial[(static_cast<u64>(blockIdx.x) * 64 + threadIdx.x) * 2] = a;
+        partial[(static_cast<u64>(blockIdx.x) * 64 + threadIdx.x) * 2 + 1] = b;
     }
 }
 
-// The SpMV of R >= 8 with the first recurrence pass in its epilogue: W = H V_cur - beta V_prev
-// (beta of this step; skipped at step 0) and the partial of <V_cur, W>, the same arithmetic as
-// batch_spmv followed by batch_vec mode 0, without writing and re-reading W in between.
-//
-// With sprev / scur the stored vectors are the unnormalised ones and V = U f with the pair's factor
-// f (1 / beta of the step that made it): every read multiplies by f, which rounds exactly as the
-// stored product of a separate scaling pass would, so the results are the same bit for bit and the
-// pass is saved.
-
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_wide_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
-                                                                    Zd* W, const double* beta, double* partial,
-                                                                    const double* sprev, const double* scur) {
-    const Tile t = B.tiles[tile_id(B)];
-    const int R = B.R, slots = kThreads / R;
-    const int slot = threadIdx.x / R, s = threadIdx.x % R;
-    const bool live = slot < slots && pair_live(B, t.block, s);
-    double pr = 0.0, pi = 0.0;
-    if (live) {
-        const int step = *B.step;
-        const u64 bs = static_cast<u64>(t.block) * R + s;
-        const double b = beta[bs];
-        const double fp = sprev ? sprev[bs] : 1.0, fc = scur ? scur[bs] : 1.0;
-        for (u64 r = t.row_begin + slot; r < t.row_end; r += slots) {
-            const u64 e0 = B.row_ptr[r], e1 = B.row_ptr[r + 1];
-            double ar = 0.0, ai = 0.0;
-            for (u64 e = e0; e < e1; ++e) {
-                const u64 c = B.col[e];
-                const Zd v = entry_value(B, e);
-                const Zd x = scaled(Vcur[c * R + s], fc);
-                ar += v.re * x.re - v.im * x.im;
-                ai += v.re * x.im + v.im * x.re;
-            }
-            const u64 i = r * R + s;
-            Zd w{ar, ai};
-            if (step > 0) {
-                const Zd p = scaled(Vprev[i], fp);
-                w = Zd{w.re - b * p.re, w.im - b * p.im};
-            }
-            W[i] = w;
-            const Zd d = cdot(scaled(Vcur[i], fc), w);
-            pr += d.re;
-            pi += d.im;
-        }
-    }
-    tile_partial(B, pr, pi, partial);
-}
-
-// The same for R = 2 and 4, on the narrow SpMV: the group's lanes are the slots of batch_vec mode 0,
-// so the partials are its partials bit for bit. (R = 3, 5, 6 and 7 keep the separate pass: their
-// slots are not the groups' rows.)
-template <int RP, bool LD>
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_narrow_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
-                                                                      Zd* W, const double* beta, double* partial,
-                                                                      const double* sprev, const double* scur) {
-    __shared__ u32 rp[kBatchTileRows + 1];
-    const Tile t = B.tiles[tile_id(B)];
-    const u64 first = stage_rows(B, t, rp);
-    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
-    __syncthreads();
-    const int s = static_cast<int>(threadIdx.x % RP);
-    const bool live = pair_live(B, t.block, s);
-    const u64 bs = static_cast<u64>(t.block) * RP + s;
-    const int step = *B.step;
-    const double b = beta[bs], fp = sprev ? sprev[bs] : 1.0, fc = scur ? scur[bs] : 1.0;
-    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
-    double pr = 0.0, pi = 0.0;
-    for (u32 r = threadIdx.x / RP; r < n; r += kThreads / RP) {
-        const u64 i = (t.row_begin + r) * RP + s;
-        Zd w = narrow_row<RP, LD>(B, Vcur, first, d0, rp[r], rp[r + 1], s, live, fc);
-        if (!live) continue;
-        if (step > 0) {
-            const Zd p = scaled(Vprev[i], fp);
-            w = Zd{w.re - b * p.re, w.im - b * p.im};
-        }
-        W[i] = w;
-        const Zd d = cdot(scaled(Vcur[i], fc), w);
-        pr += d.re;
-        pi += d.im;
-    }
-    tile_partial(B, pr, pi, partial);
-}
-
-// The same for R = 1 (the continued fractions: one vector per block). Each row's entries go to 8
-// lanes (lane l: entries e0 + l, e0 + l + 8, ... in order) and the lanes' sums meet in an xor
-// butterfly, the arithmetic of the sector SpMV that batch_spmv uses at R = 1. Two rows and two
-// entries of each are in flight per lane, the block's dictionary in LDS. The partial of <V_cur, W>
-// sums each group's rows in order, then the 32 groups by a fixed tree. Workgroups take the tiles in
-// XCD-contiguous runs (workgroup w: tile (w mod 8) * per + w / 8) unless a schedule is given, so each
-// XCD's L2 sees neighbouring rows, as the sector SpMV's row ranges do.
-//
-// With the value's two halves read from a dictionary in global memory (three gathers per entry in
-// place of one, each lane its own line) and one entry in flight, the step's SpMV at N = 26 (10.4M rows,
-// 1.5e8 entries) took 0.906 ms; so 0.785 ms.
-template <bool LD>
-__global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, const Zd* Vprev, const Zd* Vcur,
-                                                                   Zd* W, const double* beta, double* partial,
-                                                                   const double* sprev, const double* scur) {
-    constexpr int L = 8, groups = kThreads / L, P = 2, U = 2;
-    __shared__ u32 rp[kBatchTileRows + 1];
-    __shared__ double sr[groups], si[groups];
-    u32 tile;
-    if (B.sched) {
-        tile = B.sched[blockIdx.x];
-    } else {
-        const u32 per = gridDim.x >> 3;
-        tile = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-        if (tile >= B.n_tiles) return;   // the whole workgroup: the grid is rounded up to 8
-    }
-    const Tile t = B.tiles[tile];
-    const u64 first = stage_rows(B, t, rp);
-    const u32 d0 = LD ? stage_block_dict(B, t.block, batch_dict) : 0u;
-    __syncthreads();
-    const u32 g = threadIdx.x / L, lane = threadIdx.x % L;
-    const u32 n = static_cast<u32>(t.row_end - t.row_begin);
-    double pr = 0.0, pi = 0.0;
-    if (pair_live(B, t.block, 0)) {
-        const int step = *B.step;
-        const double b = beta[t.block];
-        const double fp = sprev ? sprev[t.block] : 1.0, fc = scur ? scur[t.block] : 1.0;
-        // every thread of the workgroup runs the same passes (the butterfly needs whole groups)
-        for (u32 base = 0; base < n; base += P * groups) {
-            u32 e[P], end[P];
-            double ar[P], ai[P];
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const u32 r = base + static_cast<u32>(p * groups) + g;
-                e[p] = r < n ? rp[r] + lane : 0u;
-                end[p] = r < n ? rp[r + 1] : 0u;
-                ar[p] = ai[p] = 0.0;
-            }
-            bool more = true;
-            while (more) {
-                u32 c[P][U], id[P][U];
-                Zd v[P][U], x[P][U];
-#pragma unroll
-                for (int p = 0; p < P; ++p)
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        const u32 k = e[p] + static_cast<u32>(u * L);
-                        c[p][u] = id[p][u] = 0;
-                        v[p][u] = x[p][u] = Zd{0.0, 0.0};
-                        if (k < end[p]) {
-                            c[p][u] = B.col[first + k];
-                            if constexpr (LD) id[p][u] = B.vid[first + k] - d0;
-                            else v[p][u] = entry_value(B, first + k);
-                        }
-                    }
-#pragma unroll
-                for (int p = 0; p < P; ++p)
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (e[p] + static_cast<u32>(u * L) < end[p]) x[p][u] = Vcur[c[p][u]];
-                more = false;
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (e[p] + static_cast<u32>(u * L) < end[p]) {
-                            if constexpr (LD) v[p][u] = batch_dict[id[p][u]];
-                            const Zd xs = scaled(x[p][u], fc);
-                            ar[p] += v[p][u].re * xs.re - v[p][u].im * xs.im;
-                            ai[p] += v[p][u].re * xs.im + v[p][u].im * xs.re;
-                        }
-                    e[p] += U * L;
-                    more = more || e[p] < end[p];
-                }
-            }
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-#pragma unroll
-                for (int off = L / 2; off > 0; off >>= 1) {
-                    ar[p] += __shfl_xor(ar[p], off, L);
-                    ai[p] += __shfl_xor(ai[p], off, L);
-                }
-                const u32 q = base + static_cast<u32>(p * groups) + g;
-                if (q < n && lane == 0) {
-                    const u64 r = t.row_begin + q;
-                    Zd w{ar[p], ai[p]};
-                    if (step > 0) {
-                        const Zd pv = scaled(Vprev[r], fp);
-                        w = Zd{w.re - b * pv.re, w.im - b * pv.im};
-                    }
-                    W[r] = w;
-                    const Zd d = cdot(scaled(Vcur[r], fc), w);
-                    pr += d.re;
-                    pi += d.im;
-                }
-            }
-        }
-    }
-    if (lane == 0) {
-        sr[g] = pr;
-        si[g] = pi;
-    }
-    __syncthreads();
-    if (threadIdx.x < static_cast<u32>(groups)) {
-        double a = sr[threadIdx.x], c = si[threadIdx.x];
-#pragma unroll
-        for (int off = groups / 2; off > 0; off >>= 1) {
-            a += __shfl_xor(a, off, groups);
-            c += __shfl_xor(c, off, groups);
-        }
-        if (threadIdx.x == 0) {
-            partial[static_cast<u64>(tile) * 64 * 2] = a;
-            partial[static_cast<u64>(tile) * 64 * 2 + 1] = c;
-        }
-    }
-}
-
-// mode 0: W -= beta V_prev (skipped at step 0), then partial of <V_cur, W> (alpha);
 // mode 1: W -= alpha V_cur, then partial of <V_cur, W> (the local overlap);
 // mode 5: mode 1, and the partial of ||W||^2 into partial2 as well (what mode 2 sums when it does
 //         not correct W);
@@ -443,11 +437,10 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, 
 //         B.fix (after mode 5) only the pairs flagged there, their norms into partial2;
 // mode 3: W *= 1 / beta_next (the next basis vector).
 // Pairs no longer running are left alone.
-__global__ __launch_bounds__(kThreads) void k_batch_vec(BatchView B, int mode, const Zd* Vprev, const Zd* Vcur, Zd* W,
+__global__ __launch_bounds__(kThreads) void k_batch_vec(BatchView B, int mode, const Zd* Vcur, Zd* W,
                                                         const double* coef, const Zd* zcoef, double threshold,
-                                                        double* partial, double* partial2, const double* vscale,
-                                                        const double* pscale) {
-    const Tile t = B.tiles[tile_id(B)];
+                                                        double* partial, double* partial2, const double* vscale) {
+    const Tile t = B.tiles[blockIdx.x];
     const int R = B.R, slots = kThreads / R;
     const int slot = threadIdx.x / R, s = threadIdx.x % R;
     const u64 bs = static_cast<u64>(t.block) * R + s;
@@ -465,17 +458,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_vec(BatchView B, int mode, c
         for (u64 r = t.row_begin + slot; r < t.row_end; r += slots) {
             const u64 i = r * R + s;
             Zd w = W[i];
-            if (mode == 0) {
-                if (step > 0) {
-                    const double b = coef[bs];
-                    const Zd p = scaled(Vprev[i], pscale ? pscale[bs] : 1.0);
-                    w = Zd{w.re - b * p.re, w.im - b * p.im};
-                    W[i] = w;
-                }
-                const Zd d = cdot(scaled(Vcur[i], fc), w);
-                pr += d.re;
-                pi += d.im;
-            } else if (mode == 1 || mode == 4 || mode == 5) {
+            if (mode == 1 || mode == 4 || mode == 5) {
                 const double a = coef[bs];
                 const Zd v = scaled(Vcur[i], fc);
                 w = Zd{w.re - a * v.re, w.im - a * v.im};
@@ -590,7 +573,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_finish(BatchView B, int kind
 
 // ||V||^2 per pair, then V scaled by 1 / ||V||: the normalisation of the start vectors.
 __global__ __launch_bounds__(kThreads) void k_batch_norm_partial(BatchView B, const Zd* V, double* partial) {
-    const Tile t = B.tiles[tile_id(B)];
+    const Tile t = B.tiles[blockIdx.x];
     const int R = B.R, slots = kThreads / R;
     const int slot = threadIdx.x / R, s = threadIdx.x % R;
     double p = 0.0;
@@ -614,7 +597,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_norm_finish(BatchView B, con
 }
 
 __global__ __launch_bounds__(kThreads) void k_batch_scale(BatchView B, Zd* V, const double* inv) {
-    const Tile t = B.tiles[tile_id(B)];
+    const Tile t = B.tiles[blockIdx.x];
     const int R = B.R, slots = kThreads / R;
     const int slot = threadIdx.x / R, s = threadIdx.x % R;
     if (slot >= slots) return;
@@ -625,10 +608,91 @@ __global__ __launch_bounds__(kThreads) void k_batch_scale(BatchView B, Zd* V, co
     }
 }
 
-// V[(row0 + i) R + s] = src[i], i < n: one vector placed into the batch layout.
-__global__ void k_batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n) {
+// One vector placed into the batch layout: state i of the block at packed row row0 + i, or, with the
+// engine's row order, place[row0 + i].
+__global__ void k_batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n, const u32* place) {
+    for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * blockDim.x) {
+        const u64 r = place ? place[row0 + i] : row0 + i;
+        V[r * R + s] = src[i];
+    }
+}
+
+// The whole batch vector from the states' order into the engine's: out[place[r] R + s] = in[r R + s].
+__global__ void k_batch_reorder(const Zd* in, u64 rows, int R, const u32* place, Zd* out) {
+    const u64 n = rows * static_cast<u64>(R);
     for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * blockDim.x)
-        V[(row0 + i) * R + s] = src[i];
+        out[place[i / R] * static_cast<u64>(R) + i % R] = in[i];
+}
+
+// ---- the engine's row order ---------------------------------------------------------------------
+// Breadth-first levels of the blocks flagged in `reorder`, from each block's first row: a sweep takes the
+// rows of level l and marks their unmarked columns l + 1 (several rows may mark one, with the same
+// value; the matrix is Hermitian, so its pattern is symmetric). 255: not reached.
+constexpr u32 kLevelNone = 255;
+
+__global__ __launch_bounds__(kThreads) void k_level_init(BatchView B, const u8* reorder, u8* level) {
+    const Tile t = B.tiles[blockIdx.x];
+    const bool on = reorder[t.block] != 0;
+    const u64 first = B.tiles[B.tile_begin[t.block]].row_begin;
+    for (u64 r = t.row_begin + threadIdx.x; r < t.row_end; r += kThreads)
+        level[r] = static_cast<u8>(on && r != first ? kLevelNone : 0u);
+}
+
+__global__ __launch_bounds__(kThreads) void k_level_sweep(BatchView B, const u8* reorder, u32 l, u8* level, u32* marked) {
+    const Tile t = B.tiles[blockIdx.x];
+    if (!reorder[t.block]) return;
+    const u64 n = t.row_end - t.row_begin;
+    bool any = false;
+    for (u64 r = threadIdx.x >> 3; r < n; r += kThreads / 8) {
+        if (level[t.row_begin + r] != l) continue;
+        const u64 e1 = B.row_ptr[t.row_begin + r + 1];
+        for (u64 e = B.row_ptr[t.row_begin + r] + (threadIdx.x & 7u); e < e1; e += 8) {
+            const u32 c = B.col[e];
+            if (level[c] == kLevelNone) {
+                level[c] = static_cast<u8>(l + 1);
+                any = true;
+            }
+        }
+    }
+    if (any) marked[l] = 1u;
+}
+
+__global__ __launch_bounds__(kThreads) void k_level_keys(BatchView B, const u8* level, u32* key, u32* row) {
+    const Tile t = B.tiles[blockIdx.x];
+    for (u64 r = t.row_begin + threadIdx.x; r < t.row_end; r += kThreads) {
+        key[r] = (t.block << 8) | level[r];
+        row[r] = static_cast<u32>(r);
+    }
+}
+
+__global__ void k_order_invert(const u32* order, u64 n, u32* place) {
+    for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * blockDim.x)
+        place[order[i]] = static_cast<u32>(i);
+}
+
+__global__ void k_order_lengths(const u64* row_ptr, const u32* order, u64 n, u32* len) {
+    for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * blockDim.x) {
+        const u64 r = order ? order[i] : i;
+        len[i] = static_cast<u32>(row_ptr[r + 1] - row_ptr[r]);
+    }
+}
+
+// Row i of the new matrix is row order[i] of the old one (null: i), its entries in the same order, their
+// columns moved to place[column] (null: kept); eight lanes per row.
+__global__ __launch_bounds__(kThreads) void k_order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val,
+                                                         const u32* order, const u32* place, u64 n, const u64* new_ptr,
+                                                         u32* new_col, u16* new_vid, Zd* new_val) {
+    const u64 stride = static_cast<u64>(gridDim.x) * (kThreads / 8);
+    for (u64 i = blockIdx.x * static_cast<u64>(kThreads / 8) + (threadIdx.x >> 3); i < n; i += stride) {
+        const u64 r = order ? order[i] : i;
+        const u64 from = row_ptr[r], m = row_ptr[r + 1] - from, to = new_ptr[i];
+        for (u64 k = threadIdx.x & 7u; k < m; k += 8) {
+            const u32 c = col[from + k];
+            new_col[to + k] = place ? place[c] : c;
+            if (vid) new_vid[to + k] = vid[from + k];
+            else new_val[to + k] = val[from + k];
+        }
+    }
 }
 
 __global__ void k_batch_advance(BatchView B) {
@@ -762,7 +826,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_gs_coef(BatchView B, const Z
 // W -= sum_{k < K} coef_k V_k on the tiles of the flagged blocks, k ascending.
 __global__ __launch_bounds__(kThreads) void k_batch_gs_update(BatchView B, const Zd* basis, u64 layer, int K, int kmax,
                                                               Zd* W, const int* full, const int* on, const Zd* coef) {
-    const Tile t = B.tiles[tile_id(B)];
+    const Tile t = B.tiles[blockIdx.x];
     if (!gs_block(B, t.block, full, on)) return;
     const int R = B.R, slots = kThreads / R;
     const int slot = threadIdx.x / R, s = threadIdx.x % R;
@@ -903,91 +967,67 @@ unsigned grid_for(u64 n) {
 
 }  // namespace
 
+bool batch_dict_in_lds(const BatchView& B) {
+    return B.dict_begin && B.dict_max > 0 && B.dict_max <= static_cast<u32>(kBatchDictMax);
+}
+
 namespace {
 /// f(whether the blocks' dictionaries fit LDS one at a time, the dynamic LDS bytes).
-template <class F> void by_block_dict(const BatchView& B, F&& f) {
-    if (B.vid && B.dict_begin && B.dict_max > 0 && B.dict_max <= static_cast<u32>(kBatchDictMax))
-        f(std::true_type{}, static_cast<std::size_t>(B.dict_max) * sizeof(Zd));
-    else
-        f(std::false_type{}, std::size_t{0});
+template <class F> void by_block_dict(const BatchView& B, bool ids, F&& f) {
+    if (ids && batch_dict_in_lds(B)) f(std::true_type{}, (static_cast<std::size_t>(B.dict_max) + 1) * sizeof(Zd));
+    else f(std::false_type{}, std::size_t{0});
+}
+
+template <bool FUSED>
+void launch_group(const BatchView& B, const Zd* Vprev, const Zd* X, Zd* Y, const double* beta, double* partial,
+                  const double* sprev, const double* scur, hipStream_t st) {
+    const int chunks = batch_chunks(B.R);
+    const dim3 grid(B.sched ? B.n_sched : B.n_tiles * static_cast<u32>(chunks)), block(kGroupThreads);
+    by_block_dict(B, B.vid != nullptr, [&](auto in_lds, std::size_t lds) {
+        constexpr bool LD = decltype(in_lds)::value;
+#define QSA_GROUP(RP)                                                                                                  \
+    hipLaunchKernelGGL((k_batch_spmv_group<RP, LD, FUSED>), grid, block, lds, st, B, chunks, Vprev, X, Y, beta, partial, \
+                       sprev, scur)
+        if (B.R <= 2) QSA_GROUP(2);
+        else if (B.R <= 4) QSA_GROUP(4);
+        else QSA_GROUP(8);
+#undef QSA_GROUP
+    });
 }
 }  // namespace
 
-void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st, const double* scur) {
-    if (!B.n_tiles) return;
-    if (B.R == 1) {
-        // one vector per block: the packed matrix is an ordinary CSR, applied by the sector SpMV
-        // (8 lanes per row, gathers four entries at a time, a contiguous row range per XCD); pairs
-        // that finished still compute their rows, which nothing reads
-        CsrView A;
-        A.rows = static_cast<i64>(B.rows);
-        A.row_ptr = B.row_ptr;
-        A.col = B.col;
-        if (B.vid) {
-            A.vals = B.vid;
-            A.width = 2;
-            A.dict_re = B.dict_re;
-            A.dict_im = B.dict_im;
-            A.dict_n = static_cast<int>(B.dict_n);
-        } else {
-            A.vals = B.val;
-            A.width = 0;
-        }
-        A.values_real = false;
-        A.lanes = 8;
-        A.xcd = 1;
-        A.unroll = 4;
-        VecSet v;
-        v.k = 1;
-        v.in[0] = X;
-        v.out[0] = Y;
-        csr_spmv(A, false, v, st);
-        return;
-    }
-    const dim3 grid(B.n_tiles), block(kThreads);
-    if (B.R >= 8) {
-        hipLaunchKernelGGL(k_batch_spmv_wide, grid, block, 0, st, B, X, Y);
-        return;
-    }
-    by_block_dict(B, [&](auto in_lds, std::size_t lds) {
-        constexpr bool LD = decltype(in_lds)::value;
-        if (B.R == 2) hipLaunchKernelGGL((k_batch_spmv_narrow<2, LD>), grid, block, lds, st, B, X, Y, scur);
-        else if (B.R <= 4) hipLaunchKernelGGL((k_batch_spmv_narrow<4, LD>), grid, block, lds, st, B, X, Y, scur);
-        else hipLaunchKernelGGL((k_batch_spmv_narrow<8, LD>), grid, block, lds, st, B, X, Y, scur);
-    });
+void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st) {
+    if (B.n_tiles) launch_group<false>(B, nullptr, X, Y, nullptr, nullptr, nullptr, nullptr, st);
 }
 
-bool batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
+void batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
                       hipStream_t st, const double* sprev, const double* scur) {
-    if (B.R == 3 || (B.R > 4 && B.R < 8)) return false;
-    if (!B.n_tiles) return true;
-    if (B.R >= 8) {
-        hipLaunchKernelGGL(k_batch_spmv_wide_fused, dim3(B.n_tiles), dim3(kThreads), 0, st, B, Vprev, Vcur, W, beta,
-                           partial, sprev, scur);
-        return true;
+    if (!B.n_tiles) return;
+    if (B.R > 1) {
+        launch_group<true>(B, Vprev, Vcur, W, beta, partial, sprev, scur, st);
+        return;
     }
-    const dim3 grid(B.R > 1 || B.sched ? B.n_tiles : (B.n_tiles + 7u) / 8u * 8u), block(kThreads);
-    by_block_dict(B, [&](auto in_lds, std::size_t lds) {
+    const dim3 grid(B.sched ? B.n_sched : B.n_tiles), block(kThreads);
+    by_block_dict(B, B.one.vid != nullptr, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
-        if (B.R == 1)
-            hipLaunchKernelGGL((k_batch_spmv_one_fused<LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta, partial,
-                               sprev, scur);
-        else if (B.R == 2)
-            hipLaunchKernelGGL((k_batch_spmv_narrow_fused<2, LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta,
-                               partial, sprev, scur);
-        else
-            hipLaunchKernelGGL((k_batch_spmv_narrow_fused<4, LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta,
-                               partial, sprev, scur);
+        hipLaunchKernelGGL((k_batch_spmv_one_fused<LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta, partial,
+                           sprev, scur);
     });
-    return true;
 }
 
-void batch_vec(const BatchView& B, int mode, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* coef,
-               const Zd* zcoef, double threshold, double* partial, hipStream_t st, double* partial2,
-               const double* vscale, const double* pscale) {
+void one_lengths(const BatchView& B, u32* len, u64* slice, hipStream_t st) {
+    if (B.n_tiles) hipLaunchKernelGGL(k_one_lengths, dim3(B.n_tiles), dim3(kThreads), 0, st, B, len, slice);
+}
+
+void one_fill(const BatchView& B, const u64* slice, u32* col, u16* vid, Zd* val, hipStream_t st) {
+    if (B.n_tiles) hipLaunchKernelGGL(k_one_fill, dim3(B.n_tiles), dim3(kThreads), 0, st, B, slice, col, vid, val);
+}
+
+void batch_vec(const BatchView& B, int mode, const Zd* Vcur, Zd* W, const double* coef, const Zd* zcoef,
+               double threshold, double* partial, hipStream_t st, double* partial2, const double* vscale) {
     if (!B.n_tiles) return;
-    hipLaunchKernelGGL(k_batch_vec, dim3(B.n_tiles), dim3(kThreads), 0, st, B, mode, Vprev, Vcur, W, coef, zcoef,
-                       threshold, partial, partial2, vscale, pscale);
+    hipLaunchKernelGGL(k_batch_vec, dim3(B.n_tiles), dim3(kThreads), 0, st, B, mode, Vcur, W, coef, zcoef, threshold,
+                       partial, partial2, vscale);
 }
 
 void batch_finish(const BatchView& B, int kind, const double* partial, double* alpha_hist, double* beta_hist, Zd* ov,
@@ -1005,9 +1045,51 @@ void batch_normalize(const BatchView& B, Zd* V, double* partial, double* inv, do
     hipLaunchKernelGGL(k_batch_scale, dim3(B.n_tiles), dim3(kThreads), 0, st, B, V, inv);
 }
 
-void batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n, hipStream_t st) {
+void batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n, const u32* place, hipStream_t st) {
     if (!n) return;
-    hipLaunchKernelGGL(k_batch_place, dim3(grid_for(n)), dim3(256), 0, st, V, R, row0, s, src, n);
+    hipLaunchKernelGGL(k_batch_place, dim3(grid_for(n)), dim3(256), 0, st, V, R, row0, s, src, n, place);
+}
+
+void batch_reorder(const Zd* in, u64 rows, int R, const u32* place, Zd* out, hipStream_t st) {
+    if (!rows) return;
+    hipLaunchKernelGGL(k_batch_reorder, dim3(grid_for(rows * static_cast<u64>(R))), dim3(256), 0, st, in, rows, R, place, out);
+}
+
+void level_init(const BatchView& B, const u8* reorder, u8* level, hipStream_t st) {
+    if (B.n_tiles) hipLaunchKernelGGL(k_level_init, dim3(B.n_tiles), dim3(kThreads), 0, st, B, reorder, level);
+}
+
+void level_sweep(const BatchView& B, const u8* reorder, u32 l, u8* level, u32* marked, hipStream_t st) {
+    if (B.n_tiles) hipLaunchKernelGGL(k_level_sweep, dim3(B.n_tiles), dim3(kThreads), 0, st, B, reorder, l, level, marked);
+}
+
+std::size_t level_sort_temp_bytes(u64 rows) {
+    std::size_t bytes = 0;
+    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, static_cast<const u32*>(nullptr), static_cast<u32*>(nullptr),
+                                             static_cast<const u32*>(nullptr), static_cast<u32*>(nullptr),
+                                             static_cast<unsigned>(rows));
+    return bytes;
+}
+
+void level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
+                 std::size_t temp_bytes, hipStream_t st) {
+    if (!B.n_tiles) return;
+    hipLaunchKernelGGL(k_level_keys, dim3(B.n_tiles), dim3(kThreads), 0, st, B, level, key, row);
+    int bits = 8;
+    while (bits < 32 && (static_cast<u64>(B.n_blocks) >> (bits - 8)) != 0) ++bits;
+    (void)hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, key, key2, row, order, static_cast<unsigned>(B.rows), 0, bits, st);
+    hipLaunchKernelGGL(k_order_invert, dim3(grid_for(B.rows)), dim3(256), 0, st, order, B.rows, place);
+}
+
+void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hipStream_t st) {
+    if (rows) hipLaunchKernelGGL(k_order_lengths, dim3(grid_for(rows)), dim3(256), 0, st, row_ptr, order, rows, len);
+}
+
+void order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val, const u32* order, const u32* place,
+                u64 rows, const u64* new_ptr, u32* new_col, u16* new_vid, Zd* new_val, hipStream_t st) {
+    if (rows)
+        hipLaunchKernelGGL(k_order_rows, dim3(grid_for(rows * 8)), dim3(kThreads), 0, st, row_ptr, col, vid, val, order,
+                           place, rows, new_ptr, new_col, new_vid, new_val);
 }
 
 void csr_to_dense(const CsrView& A, Zd* out, hipStream_t st) {

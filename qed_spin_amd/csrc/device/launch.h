@@ -208,13 +208,25 @@ struct Tile {
     u64 row_begin, row_end;
     u32 block, pad;
 };
+/// The matrix for R = 1: slices of 64 rows of a tile (kBatchTileRows / 64 per tile), entry k of the slice's
+/// lane j at ptr[slice] + 256 (k / 4) + 4 j + k % 4; every row filled up to whole groups of eight with
+/// its own row and value zero. Ids count from the block's first; vid null: full values.
+struct OneView {
+    const u64* ptr = nullptr;
+    const u32* len = nullptr;           // per row
+    const u32* col = nullptr;
+    const u16* vid = nullptr;
+    const Zd* val = nullptr;
+};
 struct BatchView {
     u64 rows = 0;                       // packed rows
     u32 n_blocks = 0, n_tiles = 0;
     int R = 0;                          // vectors per block (<= 64), X[row R + s]
     const Tile* tiles = nullptr;        // n_tiles, blocks contiguous
-    const u32* sched = nullptr;         // n_tiles: workgroup w runs tile sched[w] (null: tile w)
+    const u32* sched = nullptr;         // n_sched: workgroup w's SpMV work, tile * chunks + chunk (~0: none);
+    u32 n_sched = 0;                    // null: in order
     const u32* tile_begin = nullptr;    // n_blocks + 1
+    OneView one;                        // R = 1: the matrix batch_spmv_fused reads
     const u64* row_ptr = nullptr;       // packed block-diagonal CSR
     const u32* col = nullptr;
     const Zd* val = nullptr;            // the values in full, or (vid set) ids into the dictionary
@@ -232,21 +244,26 @@ struct BatchView {
 };
 constexpr int kBatchTileRows = 256;
 constexpr int kBatchMaxR = 64;
-/// Y = A X; scur (1 < R < 8 only, or null): X = stored X times its per-pair factor.
-void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st, const double* scur = nullptr);
-/// W = H V_cur - beta V_prev with the partials of <V_cur, W> (batch_spmv + batch_vec mode 0 in one
-/// kernel, the same arithmetic; bit for bit except for the order of the partials at R = 1); false
-/// (nothing launched) when R is 3, 5, 6 or 7. sprev / scur: per-pair factors of the stored vectors
-/// (V = stored times factor), or null (1).
-bool batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
+/// Work items of a tile in the SpMV: one up to eight vectors, above that one per run of eight.
+constexpr int batch_chunks(int R) { return R > 8 ? (R + 7) / 8 : 1; }
+void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st);
+/// Whether a block's dictionary fits the SpMV's LDS (else the R = 1 layout holds full values).
+bool batch_dict_in_lds(const BatchView& B);
+/// The R = 1 layout (OneView) of a packed matrix: the rows' lengths and the slices' entries
+/// (kBatchTileRows / 64 per tile; sell_scan gives their offsets), then the entries (vid or val null).
+void one_lengths(const BatchView& B, u32* len, u64* slice, hipStream_t st);
+void one_fill(const BatchView& B, const u64* slice, u32* col, u16* vid, Zd* val, hipStream_t st);
+/// W = H V_cur - beta V_prev with the partials of <V_cur, W>. sprev / scur: per-pair factors of the
+/// stored vectors (V = stored times factor), or null (1).
+void batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
                       hipStream_t st, const double* sprev = nullptr, const double* scur = nullptr);
-/// mode 0: W -= beta V_prev, <V_cur, W>; 1: W -= alpha V_cur, <V_cur, W>; 5: mode 1 and ||W||^2
-/// into partial2; 4: W -= alpha V_cur, ||W||^2; 2: local reorthogonalisation, ||W||^2 (with B.fix:
-/// only the flagged pairs, into partial2); 3: W *= 1 / beta. Partials per tile and vector. vscale:
-/// per-pair factor of the stored V_cur, or null (1); pscale: V_prev's (mode 0).
-void batch_vec(const BatchView& B, int mode, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* coef,
-               const Zd* zcoef, double threshold, double* partial, hipStream_t st, double* partial2 = nullptr,
-               const double* vscale = nullptr, const double* pscale = nullptr);
+/// mode 1: W -= alpha V_cur, <V_cur, W>; 5: mode 1 and ||W||^2 into partial2; 4: W -= alpha V_cur,
+/// ||W||^2; 2: local reorthogonalisation, ||W||^2 (with B.fix: only the flagged pairs, into partial2);
+/// 3: W *= 1 / beta. Partials per tile and vector. vscale: per-pair factor of the stored V_cur, or
+/// null (1).
+void batch_vec(const BatchView& B, int mode, const Zd* Vcur, Zd* W, const double* coef, const Zd* zcoef,
+               double threshold, double* partial, hipStream_t st, double* partial2 = nullptr,
+               const double* vscale = nullptr);
 /// kind 0: alpha; 1: the overlap (and, with B.fix, the flag of the pairs whose |overlap| exceeds
 /// threshold from step 1 on); 2: beta (ends breaking-down or capped pairs). The step is read from
 /// B.step on the device.
@@ -255,15 +272,34 @@ void batch_finish(const BatchView& B, int kind, const double* partial, double* a
                   double threshold = 0.0);
 /// V scaled to unit norm per (block, vector); inv = 1 / norm, norm2 (may be null) = norm^2.
 void batch_normalize(const BatchView& B, Zd* V, double* partial, double* inv, double* norm2, hipStream_t st);
-/// V[(row0 + i) R + s] = src[i] for i < n.
-void batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n, hipStream_t st);
+/// One vector into the batch layout: V[r R + s] = src[i] for i < n, r = row0 + i or place[row0 + i].
+void batch_place(Zd* V, int R, u64 row0, int s, const Zd* src, u64 n, const u32* place, hipStream_t st);
+/// A whole batch vector moved into the engine's row order: out[place[r] R + s] = in[r R + s].
+void batch_reorder(const Zd* in, u64 rows, int R, const u32* place, Zd* out, hipStream_t st);
+/// Breadth-first levels (0..254, 255: not reached) of the blocks flagged in reorder, from each block's
+/// first row; the other blocks' rows all get level 0. level_sweep marks level l + 1 from level l and
+/// sets marked[l] when it marked any row.
+void level_init(const BatchView& B, const u8* reorder, u8* level, hipStream_t st);
+void level_sweep(const BatchView& B, const u8* reorder, u32 l, u8* level, u32* marked, hipStream_t st);
+std::size_t level_sort_temp_bytes(u64 rows);
+/// order[i] = the row at place i when every block's rows go by level, then by row; place: its inverse.
+/// key, key2, row: rows words each.
+void level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
+                 std::size_t temp_bytes, hipStream_t st);
+/// A packed matrix with its rows in `order` (null: kept) and its columns at `place` (null: kept), each
+/// row's entries in their order: the new rows' lengths, then (new_ptr from their scan) the entries.
+void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hipStream_t st);
+void order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val, const u32* order, const u32* place,
+                u64 rows, const u64* new_ptr, u32* new_col, u16* new_vid, Zd* new_val, hipStream_t st);
 void batch_fill_zero(Zd* x, u64 n, hipStream_t st);
 
 // ---- sample.hip ------------------------------------------------------------------------------
 /// Gaussian start vectors: vector p (block p / R, slot p % R) of std::mt19937(seeds[p]) ->
 /// std::normal_distribution<double>, entry i = (n_2i, n_2i+1) written to
-/// V[(row_begin[p / R] + i) R + p % R] for i < dims[p / R]; `vectors` workgroups. Not normalised.
-void sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims, const u32* seeds, u32 vectors, hipStream_t st);
+/// V[r R + p % R], r = row_begin[p / R] + i or place[row_begin[p / R] + i], for i < dims[p / R];
+/// `vectors` workgroups. Not normalised.
+void sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims, const u32* seeds, u32 vectors,
+                  const u32* place, hipStream_t st);
 /// One block's CSR into the packed one: rows and columns offset, values in full into val, or (vid
 /// set, the block's CSR holding dictionary ids) the ids offset by dict_off into vid.
 void pack_csr(const CsrView& A, u64 row_off, u64 col_off, u64 nnz_off, u64* row_ptr, u32* col, Zd* val, u16* vid,

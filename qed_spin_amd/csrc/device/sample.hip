@@ -49,10 +49,10 @@ __device__ __forceinline__ double canonical(u32 lo, u32 hi) {
     return r >= 1.0 ? 0x1.fffffffffffffp-1 : r;
 }
 
-// Vector p of a batch: block b = p / R, slot s = p % R; entries go to V[(row_begin[b] + i) * R + s]
-// for i < dims[b].
+// Vector p of a batch: block b = p / R, slot s = p % R; entry i < dims[b] goes to V[r * R + s] with
+// r = row_begin[b] + i, or place[row_begin[b] + i].
 __global__ __launch_bounds__(kSampleThreads) void k_sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims,
-                                                                 const u32* seeds) {
+                                                                 const u32* seeds, const u32* place) {
     __shared__ u32 state[2][kMtN];
     __shared__ u64 kept[kSampleThreads / 64];
     const u32 p = blockIdx.x;
@@ -109,7 +109,10 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample_gauss(Zd* V, int R, c
             if (wv < wave) before += c;
             total += c;
         }
-        if (keep && done + before < n) V[(row0 + done + before) * static_cast<u64>(R) + s] = Zd{re, im};
+        if (keep && done + before < n) {
+            const u64 r = row0 + done + before;
+            V[(place ? place[r] : r) * static_cast<u64>(R) + s] = Zd{re, im};
+        }
         done += total;
         __syncthreads();
     }
@@ -117,9 +120,11 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample_gauss(Zd* V, int R, c
 
 }  // namespace
 
-void sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims, const u32* seeds, u32 vectors, hipStream_t st) {
+void sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims, const u32* seeds, u32 vectors,
+                  const u32* place, hipStream_t st) {
     if (!vectors) return;
-    hipLaunchKernelGGL(k_sample_gauss, dim3(vectors), dim3(kSampleThreads), 0, st, V, R, row_begin, dims, seeds);
+    hipLaunchKernelGGL(k_sample_gauss, dim3(vectors), dim3(kSampleThreads), 0, st, V, R, row_begin, dims, seeds,
+                       place);
 }
 
 }  // namespace qsa::dev

@@ -90,12 +90,10 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     const hipStream_t st = engine_stream();
     row_ptr_.reset((rows_ + 1) * 8);
     col_.reset(std::max<std::uint64_t>(nnz_, 1) * 4);
-    // Values: with fewer than 8 vectors per block (the value stream is a large share of the bytes)
-    // and when every block stores dictionary ids and the dictionaries hold at most 2^16 values
-    // together, 16-bit ids into their concatenation (2 bytes per entry instead of 16); else in full
-    // (with 8 or more vectors the gathers dominate and a full value is one broadcast load).
+    // Values: when every block stores dictionary ids and the dictionaries hold at most 2^16 values
+    // together, 16-bit ids into their concatenation (2 bytes per entry instead of 16); else in full.
     std::vector<std::uint32_t> dict_off(ops_.size() + 1, 0);
-    bool ids = R_ < 8;
+    bool ids = true;
     std::uint64_t dict_total = 0;
     for (std::size_t b = 0; ids && b < ops_.size(); ++b) {
         const dev::CsrView A = ops_[b]->device_csr();
@@ -146,6 +144,12 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     }
     put(tiles_d_, tiles_, st);
     put(tile_begin_d_, tile_begin_, st);
+    const auto t_order = clock_t_::now();
+    order_rows();
+    if (R_ == 1) slice_rows();
+    const char* pinned = std::getenv("QED_SPIN_AMD_BATCH_SCHEDULE");   // 0 or 1
+    set_schedule(pinned ? (std::atoi(pinned) == 1 ? 1 : 0) : 1);
+    order_s_ = secs(t_order, clock_t_::now());
     const std::size_t vec_bytes = rows_ * static_cast<std::size_t>(R_) * sizeof(dev::Zd);
     V0_.reset(vec_bytes);
     V1_.reset(vec_bytes);
@@ -169,83 +173,126 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     QSA_HIP(hipStreamSynchronize(st));
 }
 
+// A row's columns are gathered R at a time, so an XCD's L2 should hold the part of X that the rows in
+// flight on it read. In the order of a momentum sector's states that is nearly the whole block: at
+// N = 24, R = 4 (112,632 states, 7.2 MB) the counters gave 870 bytes of X fetched per row of 64. In
+// breadth-first level order a row's columns lie within one level of its own (21 to 42 levels on
+// rings of 22 to 26 sites, the widest 6 to 14% of a block). Blocks below 2 MB fit an L2 as they are.
+// (Rows of a level by their least column of the level before, so that neighbours share columns in the
+// L1, took a fifth of the L1's misses at R = 1 for 2% of the step, and made the J1-J2 rings' step at
+// R = 4 9% slower.)
+void BatchedLanczos::order_rows() {
+    const std::uint64_t wide = static_cast<std::uint64_t>(std::min(R_, 8)) * sizeof(dev::Zd);
+    std::vector<std::uint8_t> reorder(ops_.size(), 0);
+    bool any = false;
+    for (std::size_t b = 0; b < ops_.size(); ++b) {
+        reorder[b] = dim(static_cast<int>(b)) * wide > kOrderMinBytes ? 1 : 0;
+        any = any || reorder[b];
+    }
+    if (!any || ops_.size() >= (std::size_t{1} << 24)) return;
+    const hipStream_t st = engine_stream();
+    dev::BatchView B = view();
+    DeviceBuffer flags, level(rows_), marked(256 * 4);
+    put(flags, reorder, st);
+    const auto* on = flags.get<std::uint8_t>();
+    dev::level_init(B, on, level.get<std::uint8_t>(), st);
+    dev::fill_zero(false, marked.get(), marked.bytes() / 8, st);
+    std::vector<std::uint32_t> hit(256, 0);
+    constexpr std::uint32_t kSweeps = 16;   // between looks at whether the last ones marked anything
+    for (std::uint32_t l = 0; l + 1 < 255;) {
+        const std::uint32_t end = std::min<std::uint32_t>(l + kSweeps, 254);
+        for (; l < end; ++l) dev::level_sweep(B, on, l, level.get<std::uint8_t>(), marked.get<std::uint32_t>(), st);
+        QSA_HIP(hipGetLastError());
+        copy_to_host(hit.data(), marked.get(), marked.bytes());
+        if (!hit[l - 1]) break;
+    }
+    order_.reset(rows_ * 4);
+    place_.reset(rows_ * 4);
+    {
+        DeviceBuffer key(rows_ * 4), key2(rows_ * 4), row(rows_ * 4);
+        const std::size_t tb = dev::level_sort_temp_bytes(rows_);
+        DeviceBuffer temp(tb ? tb : 8);
+        dev::level_order(B, level.get<std::uint8_t>(), key.get<std::uint32_t>(), key2.get<std::uint32_t>(),
+                         row.get<std::uint32_t>(), order_.get<std::uint32_t>(), place_.get<std::uint32_t>(), temp.get(), tb,
+                         st);
+        QSA_HIP(hipGetLastError());
+    }
+    reorder_matrix(rows_, order_.get<std::uint32_t>(), place_.get<std::uint32_t>(), row_ptr_, col_, vid_, val_);
+}
+
+/// The packed matrix in the R = 1 layout, in place of the CSR.
+void BatchedLanczos::slice_rows() {
+    const hipStream_t st = engine_stream();
+    const dev::BatchView B = view();
+    const std::int64_t slices = static_cast<std::int64_t>(tiles_.size()) * (dev::kBatchTileRows / 64);
+    DeviceBuffer words(static_cast<std::size_t>(slices + 1) * 8);
+    one_len_.reset(rows_ * 4);
+    one_ptr_.reset(static_cast<std::size_t>(slices + 1) * 8);
+    dev::fill_zero(false, words.get(), static_cast<std::size_t>(slices + 1), st);
+    dev::one_lengths(B, one_len_.get<std::uint32_t>(), words.get<std::uint64_t>(), st);
+    const std::size_t tb = dev::sell_scan_temp_bytes(slices);
+    DeviceBuffer temp(tb ? tb : 8);
+    dev::sell_scan(words.get<std::uint64_t>(), slices, one_ptr_.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(hipGetLastError());
+    std::uint64_t total = 0;
+    copy_to_host(&total, one_ptr_.get<std::uint64_t>() + slices, 8);
+    const bool ids = B.vid && dev::batch_dict_in_lds(B);
+    DeviceBuffer col(std::max<std::uint64_t>(total, 1) * 4), vid(ids ? total * 2 : 0),
+        val(ids ? 0 : std::max<std::uint64_t>(total, 1) * sizeof(dev::Zd));
+    dev::one_fill(B, one_ptr_.get<std::uint64_t>(), col.get<std::uint32_t>(), vid.get<std::uint16_t>(), val.get<dev::Zd>(), st);
+    QSA_HIP(hipGetLastError());
+    col_ = std::move(col);
+    vid_ = std::move(vid);
+    val_ = std::move(val);
+    row_ptr_.release();
+    one_ = true;
+}
+
+void reorder_matrix(std::uint64_t rows, const std::uint32_t* order, const std::uint32_t* place, DeviceBuffer& row_ptr,
+                    DeviceBuffer& col, DeviceBuffer& vid, DeviceBuffer& val) {
+    const hipStream_t st = engine_stream();
+    DeviceBuffer len(rows * 4), ptr((rows + 1) * 8);
+    dev::order_lengths(row_ptr.get<std::uint64_t>(), order, rows, len.get<std::uint32_t>(), st);
+    const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows));
+    DeviceBuffer temp(tb ? tb : 8);
+    dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows), ptr.get<std::uint64_t>(), temp.get(), tb, st);
+    DeviceBuffer ncol(col.bytes()), nvid(vid.bytes()), nval(val.bytes());
+    dev::order_rows(row_ptr.get<std::uint64_t>(), col.get<std::uint32_t>(), vid.get<std::uint16_t>(), val.get<dev::Zd>(), order,
+                    place, rows, ptr.get<std::uint64_t>(), ncol.get<std::uint32_t>(), nvid.get<std::uint16_t>(),
+                    nval.get<dev::Zd>(), st);
+    QSA_HIP(hipGetLastError());
+    row_ptr = std::move(ptr);   // the old ones are freed on this stream, after the kernels that read them
+    col = std::move(ncol);
+    vid = std::move(nvid);
+    val = std::move(nval);
+}
+
 void BatchedLanczos::set_schedule(int kind) {
     sched_kind_ = 0;
     sched_d_.release();
+    n_sched_ = 0;
     if (kind != 1 || tiles_.empty()) return;
-    // blocks to XCDs, largest first onto the XCD with the fewest rows so far; workgroup w runs on XCD
-    // w % 8, so it takes the next tile of that XCD's blocks (of the longest remaining queue when that
-    // XCD has none left)
-    constexpr int kXcd = 8;
-    std::vector<std::size_t> order(ops_.size());
-    for (std::size_t b = 0; b < order.size(); ++b) order[b] = b;
-    std::stable_sort(order.begin(), order.end(), [&](std::size_t a, std::size_t b) { return dim(a) > dim(b); });
-    std::uint64_t load[kXcd] = {};
-    std::vector<std::uint32_t> queue[kXcd];
-    for (const std::size_t b : order) {
-        int x = 0;
-        for (int y = 1; y < kXcd; ++y)
-            if (load[y] < load[x]) x = y;
-        load[x] += dim(static_cast<int>(b));
-        for (std::uint32_t t = tile_begin_[b]; t < tile_begin_[b + 1]; ++t) queue[x].push_back(t);
-    }
-    std::size_t head[kXcd] = {};
-    std::vector<std::uint32_t> sched(tiles_.size());
-    for (std::size_t w = 0; w < sched.size(); ++w) {
-        int x = static_cast<int>(w % kXcd);
-        if (head[x] == queue[x].size()) {
-            for (int y = 0; y < kXcd; ++y)
-                if (queue[y].size() - head[y] > queue[x].size() - head[x]) x = y;
+    // Workgroup w runs on XCD w % 8: each XCD gets one eighth of the tiles, neighbours in order, so that
+    // the columns of the rows in flight share its L2; with several runs of vectors, a block's tiles
+    // take one run after the other.
+    constexpr std::size_t kXcd = 8;
+    const std::size_t nt = tiles_.size(), chunks = static_cast<std::size_t>(dev::batch_chunks(R_));
+    const std::size_t longest = (nt + kXcd - 1) / kXcd * chunks;
+    std::vector<std::uint32_t> sched(longest * kXcd, ~0u);
+    for (std::size_t x = 0; x < kXcd; ++x) {
+        const std::size_t t0 = x * nt / kXcd, t1 = (x + 1) * nt / kXcd;
+        std::size_t w = x;
+        for (std::size_t a = t0; a < t1;) {
+            std::size_t b = a;
+            while (b < t1 && tiles_[b].block == tiles_[a].block) ++b;
+            for (std::size_t c = 0; c < chunks; ++c)
+                for (std::size_t t = a; t < b; ++t, w += kXcd) sched[w] = static_cast<std::uint32_t>(t * chunks + c);
+            a = b;
         }
-        sched[w] = queue[x][head[x]++];
     }
     put(sched_d_, sched, engine_stream());
-    QSA_HIP(hipStreamSynchronize(engine_stream()));
+    n_sched_ = static_cast<std::uint32_t>(sched.size());
     sched_kind_ = 1;
-}
-
-int BatchedLanczos::tune_schedule() {
-    if (const char* e = std::getenv("QED_SPIN_AMD_BATCH_SCHEDULE")) {   // pinned: 0 or 1
-        set_schedule(std::atoi(e) == 1 ? 1 : 0);
-        return sched_kind_;
-    }
-    // small engines finish a step in microseconds either way; above 65536 tiles the two schedules
-    // measured alike and a timed apply costs tens of milliseconds. R = 1 keeps the in-order schedule,
-    // which its fused step kernel runs in XCD-contiguous runs of tiles (the plain apply timed here
-    // is the sector SpMV, which takes no schedule)
-    if (R_ == 1 || tiles_.size() < 4096 || tiles_.size() > 65536) {
-        set_schedule(0);
-        return 0;
-    }
-    // one warm-up apply, then the two schedules alternately (0, 1, 0, 1), each apply timed
-    const hipStream_t st = engine_stream();
-    hipEvent_t ev[5];
-    for (auto& e : ev) QSA_HIP(hipEventCreate(&e));
-    set_schedule(1);
-    const std::uint32_t* grouped = sched_d_.get<std::uint32_t>();
-    DeviceBuffer keep = std::move(sched_d_);
-    dev::BatchView B = packed_view();
-    B.sched = nullptr;
-    dev::batch_spmv(B, V1_.get<dev::Zd>(), W_.get<dev::Zd>(), st);
-    QSA_HIP(hipEventRecord(ev[0], st));
-    for (int i = 0; i < 4; ++i) {
-        B.sched = (i & 1) ? grouped : nullptr;
-        dev::batch_spmv(B, V1_.get<dev::Zd>(), W_.get<dev::Zd>(), st);
-        QSA_HIP(hipEventRecord(ev[i + 1], st));
-    }
-    QSA_HIP(hipEventSynchronize(ev[4]));
-    float ms[2] = {0.0f, 0.0f};
-    for (int i = 0; i < 4; ++i) {
-        float m = 0.0f;
-        QSA_HIP(hipEventElapsedTime(&m, ev[i], ev[i + 1]));
-        ms[i & 1] += m;
-    }
-    for (auto& e : ev) (void)hipEventDestroy(e);
-    const int best = ms[1] < ms[0] ? 1 : 0;
-    dev::batch_fill_zero(W_.get<dev::Zd>(), rows_ * R_, st);
-    QSA_HIP(hipStreamSynchronize(st));
-    set_schedule(best);
-    return best;
 }
 
 dev::BatchView BatchedLanczos::view() const {
@@ -256,12 +303,21 @@ dev::BatchView BatchedLanczos::view() const {
     B.R = R_;
     B.tiles = tiles_d_.get<dev::Tile>();
     B.sched = sched_d_ ? sched_d_.get<std::uint32_t>() : nullptr;
+    B.n_sched = n_sched_;
     B.tile_begin = tile_begin_d_.get<std::uint32_t>();
-    B.row_ptr = row_ptr_.get<std::uint64_t>();
-    B.col = col_.get<std::uint32_t>();
-    B.val = val_.get<dev::Zd>();
-    if (dict_n_) {
+    if (one_) {
+        B.one.ptr = one_ptr_.get<std::uint64_t>();
+        B.one.len = one_len_.get<std::uint32_t>();
+        B.one.col = col_.get<std::uint32_t>();
+        B.one.vid = vid_.get<std::uint16_t>();
+        B.one.val = val_.get<dev::Zd>();
+    } else {
+        B.row_ptr = row_ptr_.get<std::uint64_t>();
+        B.col = col_.get<std::uint32_t>();
+        B.val = val_.get<dev::Zd>();
         B.vid = vid_.get<std::uint16_t>();
+    }
+    if (dict_n_) {
         B.dict_re = dict_re_.get<double>();
         B.dict_im = dict_im_.get<double>();
         B.dict_n = dict_n_;
@@ -277,7 +333,13 @@ dev::BatchView BatchedLanczos::view() const {
 }
 
 void BatchedLanczos::set_start(const cplx* host) {
-    copy_to_device(V0_.get(), host, rows_ * R_ * sizeof(dev::Zd));
+    if (place_) {   // through W, into the engine's row order
+        copy_to_device(W_.get(), host, rows_ * R_ * sizeof(dev::Zd));
+        dev::batch_reorder(W_.get<dev::Zd>(), rows_, R_, place_.get<std::uint32_t>(), V0_.get<dev::Zd>(), engine_stream());
+        QSA_HIP(hipGetLastError());
+    } else {
+        copy_to_device(V0_.get(), host, rows_ * R_ * sizeof(dev::Zd));
+    }
     normalize(nullptr);
 }
 
@@ -289,7 +351,7 @@ void BatchedLanczos::clear_start() {
 void BatchedLanczos::place(int b, int s, const cplx* device_vector) {
     if (b < 0 || b >= n_blocks() || s < 0 || s >= R_) throw Error(kInvalid, "batched lanczos: no such pair");
     dev::batch_place(V0_.get<dev::Zd>(), R_, row_off_[b], s, reinterpret_cast<const dev::Zd*>(device_vector), dim(b),
-                     engine_stream());
+                     place_.get<std::uint32_t>(), engine_stream());
     QSA_HIP(hipGetLastError());
 }
 
@@ -320,16 +382,9 @@ void BatchedLanczos::sample_start(const std::vector<std::uint32_t>& seeds) {
     put(dim_d, dims, st);
     put(seed_d, seeds, st);
     dev::sample_gauss(V0_.get<dev::Zd>(), R_, rb_d.get<std::uint64_t>(), dim_d.get<std::uint64_t>(),
-                      seed_d.get<std::uint32_t>(), static_cast<std::uint32_t>(pairs), st);
+                      seed_d.get<std::uint32_t>(), static_cast<std::uint32_t>(pairs), place_.get<std::uint32_t>(), st);
     QSA_HIP(hipGetLastError());
     normalize(nullptr);
-}
-
-void BatchedLanczos::apply(const cplx* X, cplx* Y) const {
-    dev::BatchView B = view();
-    B.active = nullptr;
-    dev::batch_spmv(B, reinterpret_cast<const dev::Zd*>(X), reinterpret_cast<dev::Zd*>(Y), engine_stream());
-    QSA_HIP(hipGetLastError());
 }
 
 void BatchedLanczos::run(int M, const std::vector<double>& breakdown_tol, bool local, bool use_graph,
@@ -392,20 +447,17 @@ void BatchedLanczos::run(int M, const std::vector<double>& breakdown_tol, bool l
         const double* sp = S[phase % 3];
         const double* sc = S[(phase + 1) % 3];
         double* sw = S[(phase + 2) % 3];
-        if (!dev::batch_spmv_fused(B, p, c, w, cb, partial, st, sp, sc)) {
-            dev::batch_spmv(B, c, w, st, sc);
-            dev::batch_vec(B, 0, p, c, w, cb, nullptr, 0.0, partial, st, nullptr, sc, sp);
-        }
+        dev::batch_spmv_fused(B, p, c, w, cb, partial, st, sp, sc);
         dev::batch_finish(B, 0, partial, ah, bh, ov, ca, cb, ib, tol, st);
         if (local) {
             // W -= alpha V with the local overlap and ||W||^2 in one pass; the correction pass then
             // touches only the pairs whose overlap asks for one (their norms are summed again)
-            dev::batch_vec(B, 5, nullptr, c, w, ca, nullptr, 0.0, partial, st, partial2, sc);
+            dev::batch_vec(B, 5, c, w, ca, nullptr, 0.0, partial, st, partial2, sc);
             dev::batch_finish(B, 1, partial, ah, bh, ov, ca, cb, ib, tol, st, thr);
-            dev::batch_vec(B, 2, nullptr, c, w, nullptr, ov, thr, partial, st, partial2, sc);
+            dev::batch_vec(B, 2, c, w, nullptr, ov, thr, partial, st, partial2, sc);
             dev::batch_finish(B, 2, partial2, ah, bh, ov, ca, cb, sw, tol, st);
         } else {
-            dev::batch_vec(B, 4, nullptr, c, w, ca, nullptr, 0.0, partial, st, nullptr, sc);
+            dev::batch_vec(B, 4, c, w, ca, nullptr, 0.0, partial, st, nullptr, sc);
             dev::batch_finish(B, 2, partial, ah, bh, ov, ca, cb, sw, tol, st);
         }
         dev::batch_advance(B, st);
@@ -523,14 +575,11 @@ void BatchedLanczos::run_kept(int M, const std::vector<double>& breakdown_tol, c
         dev::Zd* W = basis + static_cast<std::uint64_t>(j + 1) * layer;
         // the kept layers are stored normalised (the overlaps read them later), so only the first
         // recurrence pass is fused here, not the deferred scaling of run()
-        if (!dev::batch_spmv_fused(B, Vp, Vc, W, cb, partial, st)) {
-            dev::batch_spmv(B, Vc, W, st);
-            dev::batch_vec(B, 0, Vp, Vc, W, cb, nullptr, 0.0, partial, st);
-        }
+        dev::batch_spmv_fused(B, Vp, Vc, W, cb, partial, st);
         dev::batch_finish(B, 0, partial, ah, bh, ov, ca, cb, ib, tol, st);
-        dev::batch_vec(B, 5, nullptr, Vc, W, ca, nullptr, 0.0, partial, st, partial2);
+        dev::batch_vec(B, 5, Vc, W, ca, nullptr, 0.0, partial, st, partial2);
         dev::batch_finish(B, 1, partial, ah, bh, ov, ca, cb, ib, tol, st, thr);
-        dev::batch_vec(B, 2, nullptr, Vc, W, nullptr, ov, thr, partial, st, partial2);
+        dev::batch_vec(B, 2, Vc, W, nullptr, ov, thr, partial, st, partial2);
         if (any_full) {
             // CGS2 against every kept layer; the second pass only where the first removed more than
             // 1 - kappa of ||W|| (DGKS, as the reference's FullCGS2 gates it): partial2 holds the
@@ -543,7 +592,7 @@ void BatchedLanczos::run_kept(int M, const std::vector<double>& breakdown_tol, c
             dev::batch_norm_partial(B, W, partial2, st);
         }
         dev::batch_finish(B, 2, partial2, ah, bh, ov, ca, cb, ib, tol, st);
-        dev::batch_vec(B, 3, nullptr, nullptr, W, ib, nullptr, 0.0, partial, st);
+        dev::batch_vec(B, 3, nullptr, W, ib, nullptr, 0.0, partial, st);
         dev::batch_advance(B, st);
     }
     QSA_HIP(hipGetLastError());
@@ -573,9 +622,8 @@ std::vector<Curves> batched_ftlm(const std::vector<std::shared_ptr<const SectorO
     const int R = std::min(o.samples, dev::kBatchMaxR);
     BatchedLanczos L(blocks, R);
     t.pack_s += secs(t_pack, clock_t_::now());
-    const auto t_tune = clock_t_::now();
-    t.schedule = L.tune_schedule();
-    t.tune_s += secs(t_tune, clock_t_::now());
+    t.schedule = L.schedule();
+    t.order_s = L.order_seconds();
     std::vector<RitzPool> pools(nb);
     std::vector<double> alpha, beta;
     std::vector<int> steps;

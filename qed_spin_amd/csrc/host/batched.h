@@ -20,8 +20,8 @@ struct BatchedTimings {
     std::uint64_t rows = 0, nnz = 0;
     int steps = 0;
     bool graph = false;
-    int schedule = 0;               ///< the tile schedule the autotuner chose (BatchedLanczos::set_schedule)
-    double tune_s = 0.0;
+    int schedule = 0;               ///< the tile schedule (BatchedLanczos::set_schedule)
+    double order_s = 0.0;           ///< ordering the rows (within pack_s)
 };
 
 /// The packed engine: blocks (square sector operators on the CSR lane) x R complex vectors.
@@ -65,29 +65,27 @@ public:
     void run_kept(int M, const std::vector<double>& breakdown_tol, const std::vector<int>& full, cplx* basis,
                   std::vector<double>& alpha, std::vector<double>& beta, std::vector<int>& steps, BatchedTimings& t,
                   const std::vector<int>* live = nullptr);
-    /// Y = H X on batch vectors (device pointers, rows() x R complex each).
-    void apply(const cplx* X, cplx* Y) const;
     /// The start vectors (rows() x R, device): written by the caller, then normalize().
     cplx* start_buffer() { return V0_.get<cplx>(); }
-    /// Which workgroup runs which tile: 0 in order, 1 grouped by XCD (the tiles of a block on one
-    /// XCD, blocks spread over the XCDs by rows, so a block's gathers share that XCD's L2). Every
-    /// schedule gives the same results bit for bit: a tile's work and partial sums do not depend on
-    /// the workgroup that runs it.
+    /// Which workgroup runs which part of the SpMV: 0 in order over all XCDs, 1 (the default;
+    /// QED_SPIN_AMD_BATCH_SCHEDULE pins either) each XCD one run of neighbouring tiles. Both give the
+    /// same results bit for bit: a tile's work and partial sums do not depend on the workgroup.
     void set_schedule(int kind);
     int schedule() const { return sched_kind_; }
-    /// The schedule of the faster packed matvec, timed over a few applies of each (the engine's
-    /// autotuner); returns the chosen kind. Engines of fewer than 4096 or more than 65536 tiles keep
-    /// schedule 0.
-    int tune_schedule();
-    /// The packed layout as the kernels read it (tiles, R); every pair live.
-    dev::BatchView packed_view() const {
-        dev::BatchView B = view();
-        B.active = nullptr;
-        return B;
-    }
+    /// Host seconds the row order and the schedule took.
+    double order_seconds() const { return order_s_; }
+    /// The engine's row order (device, rows() words each, null: the states' order): the packed row of
+    /// the states' order at place i, and the place of each such row.
+    const std::uint32_t* order() const { return order_.get<std::uint32_t>(); }
+    const std::uint32_t* place() const { return place_.get<std::uint32_t>(); }
 
 private:
     dev::BatchView view() const;
+    void order_rows();
+    void slice_rows();
+    /// Blocks whose vectors (eight at most) take more than this are stored in level order: half an
+    /// XCD's L2.
+    static constexpr std::uint64_t kOrderMinBytes = 2u << 20;
     std::vector<std::shared_ptr<const SectorOperator>> ops_;
     int R_;
     std::uint64_t rows_ = 0, nnz_ = 0;
@@ -99,11 +97,20 @@ private:
     std::uint32_t dict_n_ = 0, dict_max_ = 0;
     DeviceBuffer dict_begin_;
     int sched_kind_ = 0;
-    DeviceBuffer sched_d_;
+    std::uint32_t n_sched_ = 0;
+    double order_s_ = 0.0;
+    DeviceBuffer sched_d_, order_, place_;
+    bool one_ = false;   // R = 1: col_ and vid_ / val_ are the sliced layout's
+    DeviceBuffer one_ptr_, one_len_;
     DeviceBuffer V0_, V1_, W_, partial_, partial2_, fix_, scale_, alpha_h_, beta_h_, ov_, cur_a_, cur_b_, inv_b_,
         tol_d_;
     friend struct BatchedAccess;
 };
+
+/// A packed matrix with its rows in `order` (null: kept) and its columns moved to `place` (null: kept),
+/// each row's entries in their order; vid or val may be empty.
+void reorder_matrix(std::uint64_t rows, const std::uint32_t* order, const std::uint32_t* place, DeviceBuffer& row_ptr,
+                    DeviceBuffer& col, DeviceBuffer& vid, DeviceBuffer& val);
 
 struct BatchedFtlmOptions {
     int samples = 40, krylov = 100;

@@ -125,7 +125,7 @@ extern "C" int qedh_ftlm_batched(const qedh_matvec* blocks, int n_blocks, int sa
             stats[6] = static_cast<double>(t.rows);
             stats[7] = static_cast<double>(t.nnz);
             stats[8] = static_cast<double>(t.schedule);
-            stats[9] = t.tune_s;
+            stats[9] = t.order_s;
         }
     });
 }
@@ -263,9 +263,8 @@ extern "C" int qedh_cf_batched(const qedh_matvec* blocks, int n_blocks, int R, c
         const auto t0 = std::chrono::steady_clock::now();
         qsa::BatchedTimings t;
         qsa::BatchedLanczos L(ops, R);
-        const auto t_tune = std::chrono::steady_clock::now();
-        t.schedule = L.tune_schedule();
-        t.tune_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_tune).count();
+        t.schedule = L.schedule();
+        t.order_s = L.order_seconds();
         L.clear_start();
         const std::size_t pairs = static_cast<std::size_t>(n_blocks) * static_cast<std::size_t>(R);
         for (int b = 0; b < n_blocks; ++b)
@@ -314,7 +313,7 @@ extern "C" int qedh_cf_batched(const qedh_matvec* blocks, int n_blocks, int R, c
             stats[5] = static_cast<double>(t.rows);
             stats[6] = static_cast<double>(t.nnz);
             stats[7] = static_cast<double>(t.schedule);
-            stats[8] = t.tune_s;
+            stats[8] = t.order_s;
         }
     });
 }
@@ -482,7 +481,7 @@ extern "C" int qedh_gaussian_vectors(uint64_t base, uint64_t first_sample, int c
         qsa::copy_to_device(dim_d.get(), dims.data(), c * 8);
         qsa::copy_to_device(seed_d.get(), seeds.data(), c * 4);
         qsa::dev::sample_gauss(reinterpret_cast<qsa::dev::Zd*>(out), 1, rb_d.get<std::uint64_t>(),
-                               dim_d.get<std::uint64_t>(), seed_d.get<std::uint32_t>(), static_cast<std::uint32_t>(c), st);
+                               dim_d.get<std::uint64_t>(), seed_d.get<std::uint32_t>(), static_cast<std::uint32_t>(c), nullptr, st);
         QSA_HIP(hipGetLastError());
         QSA_HIP(hipStreamSynchronize(st));
     });

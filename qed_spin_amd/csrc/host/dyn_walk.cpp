@@ -24,7 +24,8 @@ double since(clk::time_point a) { return std::chrono::duration<double>(clk::now(
 class PackedProbe {
 public:
     PackedProbe(const std::vector<const SectorOperator*>& probes, const std::vector<std::uint64_t>& row_off,
-                const std::vector<std::uint64_t>& col_off, int R)
+                const std::vector<std::uint64_t>& col_off, int R, const std::uint32_t* row_order,
+                const std::uint32_t* col_place)
         : R_(R) {
         const hipStream_t st = engine_stream();
         std::vector<std::uint64_t> nnz_off(1, 0);
@@ -40,6 +41,10 @@ public:
             dev::pack_csr(probes[c]->device_csr(), row_off[c], col_off[c], nnz_off[c], row_ptr_.get<std::uint64_t>(),
                           col_.get<std::uint32_t>(), val_.get<dev::Zd>(), nullptr, 0, st);
         QSA_HIP(hipGetLastError());
+        if (row_order || col_place) {   // into the engines' row orders
+            DeviceBuffer no_ids;
+            reorder_matrix(rows_, row_order, col_place, row_ptr_, col_, no_ids, val_);
+        }
         std::vector<dev::Tile> tiles;
         std::vector<std::uint32_t> begin(1, 0);
         for (std::size_t c = 0; c < probes.size(); ++c) {
@@ -268,8 +273,8 @@ DynWalkResult ftlm_dynamics_walk(const std::vector<std::shared_ptr<const SectorO
                     tol_c.push_back(o.breakdown_tol[channels[c].source]);
                     full_c.push_back(static_cast<std::size_t>(channels[c].H->dim()) <= full_limit ? 1 : 0);
                 }
-                const PackedProbe P(probes, crow, colo, R);
                 BatchedLanczos T(wtgt, R);
+                const PackedProbe P(probes, crow, colo, R, T.order(), S.place());
                 P.apply(Vs, reinterpret_cast<dev::Zd*>(T.start_buffer()));
                 T.normalize(&n2);
                 std::vector<int> live(nc * static_cast<std::size_t>(R));
