@@ -166,15 +166,19 @@ struct Cols {
     }
 };
 
-// dot_many: block b owns a row range; the rows come in tiles of kTile staged in LDS (the w tile),
-// wavefront v owns the columns j = v, v + 4, ...: its lanes read 64 consecutive rows of column j
-// per load (coalesced), sum, and the wave total accumulates into the column's LDS slot (one owner:
-// no race). Partials are written column-major [j][b] so the finish reads them contiguously.
+// dot_many: block (b, g) owns a row range and a group of `per` columns; the rows come in tiles of kTile
+// staged in LDS (the w tile), wavefront v owns the columns j = v, v + 4, ... of the group: its lanes read
+// 64 consecutive rows of column j per load (coalesced), sum, and the wave total accumulates into the
+// column's LDS slot (one owner: no race). Partials are written column-major [j][b] so the finish
+// reads them contiguously. Few rows leave the card idle with every block taking every column (n = 9252:
+// 10 blocks of 100 columns took 50 us): there the columns go to several blocks (dot_columns, 7 us;
+// 112,632 complex rows and 25 columns 22 -> 13 us). Four loads in flight per lane: eight are slower where
+// HBM bounds it (2.6M rows and 50 columns 224 us for 200).
 constexpr int kManyCols = 256;   // columns per launch
 constexpr int kTile = 1024;      // rows per LDS tile
 
 template <bool C>
-__global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, const void* w,
+__global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, int per, const void* w,
                                                        std::size_t n, std::size_t rows_per_block, double* partial,
                                                        int nb, int want_norm) {
     __shared__ Zd sw[kTile];
@@ -182,7 +186,9 @@ __global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, const voi
     const std::size_t r0 = blockIdx.x * rows_per_block;
     const std::size_t r1 = (r0 + rows_per_block < n) ? r0 + rows_per_block : n;
     const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    for (int j = threadIdx.x; j <= m; j += blockDim.x) acc[j] = Zd{0.0, 0.0};
+    const int j0 = static_cast<int>(blockIdx.y) * per, j1 = j0 + per < m ? j0 + per : m;
+    const bool norm = want_norm && blockIdx.y == 0;
+    for (int j = j0 + static_cast<int>(threadIdx.x); j < j1; j += blockDim.x) acc[j] = Zd{0.0, 0.0};
     double nrm = 0.0;
     __syncthreads();
     for (std::size_t t0 = r0; t0 < r1; t0 += kTile) {
@@ -190,10 +196,10 @@ __global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, const voi
         for (int i = threadIdx.x; i < cnt; i += blockDim.x) {
             const Zd v = V<C>::load(w, t0 + i);
             sw[i] = v;
-            if (want_norm) nrm += v.re * v.re + (C ? v.im * v.im : 0.0);
+            if (norm) nrm += v.re * v.re + (C ? v.im * v.im : 0.0);
         }
         __syncthreads();
-        for (int j = wv; j < m; j += kWaves) {
+        for (int j = j0 + wv; j < j1; j += kWaves) {
             const void* cj = Vb.at(j);
             double pr = 0.0, pi = 0.0;
 #pragma unroll 4
@@ -213,16 +219,27 @@ __global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, const voi
         }
         __syncthreads();
     }
-    if (want_norm) {
+    if (norm) {
         double dummy = 0.0;
         block_sum2(nrm, dummy);
-        if (threadIdx.x == 0) acc[m] = Zd{nrm, 0.0};
+        if (threadIdx.x == 0) {
+            partial[(static_cast<std::size_t>(m) * nb + blockIdx.x) * 2] = nrm;
+            partial[(static_cast<std::size_t>(m) * nb + blockIdx.x) * 2 + 1] = 0.0;
+        }
     }
-    __syncthreads();
-    for (int j = threadIdx.x; j <= m; j += blockDim.x) {
+    for (int j = j0 + static_cast<int>(threadIdx.x); j < j1; j += blockDim.x) {
         partial[(static_cast<std::size_t>(j) * nb + blockIdx.x) * 2] = acc[j].re;
         partial[(static_cast<std::size_t>(j) * nb + blockIdx.x) * 2 + 1] = acc[j].im;
     }
+}
+
+/// Columns per block of dot_many: all of them when the row blocks alone fill the card, else as few (four,
+/// one per wavefront, or more) as make about three blocks per compute unit.
+inline int dot_columns(int m, std::size_t row_blocks) {
+    const int most = (m + kWaves - 1) / kWaves;
+    const int groups = static_cast<int>(std::min<std::size_t>(static_cast<std::size_t>(most), (768 + row_blocks - 1) / row_blocks));
+    if (groups <= 1) return m;
+    return ((m + groups - 1) / groups + kWaves - 1) / kWaves * kWaves;
 }
 
 // One block per column: the sum of its nb block partials (contiguous) in a fixed order.
@@ -274,6 +291,72 @@ __global__ __launch_bounds__(kThreads) void k_axpy_many(const Zd* coeffs, Cols V
         block_sum2(s0, s1);
         if (threadIdx.x == 0) {
             partial[2 * blockIdx.x] = s0;
+            partial[2 * blockIdx.x + 1] = 0.0;
+        }
+    }
+}
+
+// axpy_many below kSplitRows rows: a block takes ROWS rows and its 512 / ROWS wavefront groups a share of
+// the columns each (column j to group j mod groups, four loads in flight per thread), the shares added
+// in group order. One thread per four rows and all columns, as above, is a chain of m / 4 rounds of
+// loads on n / 1024 blocks: 44 us for 9252 rows and 100 columns (so 7), 18 us for 112,632 complex rows and
+// 25 (so 9.6). From 2^19 rows on the threads alone keep enough loads in flight.
+constexpr std::size_t kSplitRows = std::size_t{1} << 19;
+constexpr int kSplitThreads = 512;
+
+template <bool C, int ROWS>
+__global__ __launch_bounds__(kSplitThreads) void k_axpy_many_split(const Zd* coeffs, Cols Vb, int m, void* w,
+                                                                   std::size_t n, double* partial, int want_norm,
+                                                                   double sign) {
+    constexpr int G = kSplitThreads / ROWS, U = 4;
+    __shared__ Zd sc[kManyCols];
+    __shared__ Zd share[G - 1][ROWS];
+    __shared__ double part[ROWS / 64];
+    for (int j = threadIdx.x; j < m; j += kSplitThreads) sc[j] = Zd{sign * coeffs[j].re, sign * coeffs[j].im};
+    __syncthreads();
+    const int row = static_cast<int>(threadIdx.x % ROWS), g = static_cast<int>(threadIdx.x / ROWS);
+    double s0 = 0.0;
+    for (std::size_t base = blockIdx.x * static_cast<std::size_t>(ROWS); base < n;
+         base += static_cast<std::size_t>(gridDim.x) * ROWS) {
+        const std::size_t i = base + row;
+        const bool in = i < n;
+        Zd acc{0.0, 0.0};
+        if (in) {
+            int j = g;
+            for (; j + (U - 1) * G < m; j += U * G) {
+                Zd v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = V<C>::load(Vb.at(j + u * G), i);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if constexpr (C) acc = cadd(acc, cmul(sc[j + u * G], v[u]));
+                    else acc.re += sc[j + u * G].re * v[u].re;
+                }
+            }
+            for (; j < m; j += G) {
+                const Zd vj = V<C>::load(Vb.at(j), i);
+                acc = C ? cadd(acc, cmul(sc[j], vj)) : Zd{acc.re + sc[j].re * vj.re, 0.0};
+            }
+        }
+        if (g > 0) share[g - 1][row] = acc;
+        __syncthreads();
+        if (g == 0 && in) {
+            acc = cadd(V<C>::load(w, i), acc);
+#pragma unroll
+            for (int q = 0; q < G - 1; ++q) acc = cadd(acc, share[q][row]);
+            V<C>::store(w, i, acc);
+            s0 += acc.re * acc.re + (C ? acc.im * acc.im : 0.0);
+        }
+        __syncthreads();   // before the next rows' shares
+    }
+    if (want_norm) {   // the rows' threads are the first ROWS / 64 wavefronts
+        s0 = wave_sum(s0);
+        if (g == 0 && (threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s0;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double t = 0.0;
+            for (int q = 0; q < ROWS / 64; ++q) t += part[q];
+            partial[2 * blockIdx.x] = t;
             partial[2 * blockIdx.x + 1] = 0.0;
         }
     }
@@ -382,12 +465,14 @@ static void dot_many_cols(bool c, const void* V, std::size_t ld, const void* con
         const Cols Vc{table ? nullptr : static_cast<const char*>(V) + done * ld * elem, ld * elem,
                       table ? table + done : nullptr};
         const int want = (first && wnorm2) ? 1 : 0;
+        const int per = dot_columns(mc, nb);
+        const dim3 grid(static_cast<unsigned>(nb), static_cast<unsigned>(mc > 0 ? (mc + per - 1) / per : 1));
         if (c)
-            hipLaunchKernelGGL(k_dot_many<true>, dim3(static_cast<unsigned>(nb)), dim3(kThreads), 0, st, Vc, mc, w,
-                               n, rpb, part, static_cast<int>(nb), want);
+            hipLaunchKernelGGL(k_dot_many<true>, grid, dim3(kThreads), 0, st, Vc, mc, per, w, n, rpb, part,
+                               static_cast<int>(nb), want);
         else
-            hipLaunchKernelGGL(k_dot_many<false>, dim3(static_cast<unsigned>(nb)), dim3(kThreads), 0, st, Vc, mc,
-                               w, n, rpb, part, static_cast<int>(nb), want);
+            hipLaunchKernelGGL(k_dot_many<false>, grid, dim3(kThreads), 0, st, Vc, mc, per, w, n, rpb, part,
+                               static_cast<int>(nb), want);
         hipLaunchKernelGGL(k_dot_many_finish, dim3(static_cast<unsigned>(mc + want)), dim3(kThreads), 0, st, part,
                            static_cast<int>(nb), mc, coeffs + done, want ? wnorm2 : nullptr);
         done += static_cast<std::size_t>(mc);
@@ -409,7 +494,9 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
                            double sign) {
     double* part = static_cast<double*>(scratch);
     const std::size_t elem = c ? sizeof(Zd) : sizeof(double);
-    const unsigned g = grid_for(n);
+    const std::size_t rows = n <= 65536 ? 64 : 128;   // k_axpy_many_split's rows per block
+    const unsigned g = n >= kSplitRows ? grid_for(n)
+                                       : static_cast<unsigned>(std::min<std::size_t>(std::max<std::size_t>((n + rows - 1) / rows, 1), kMaxBlocks));
     std::size_t done = 0;
     do {
         const int mc = static_cast<int>((m - done) < static_cast<std::size_t>(kManyCols) ? (m - done) : kManyCols);
@@ -417,12 +504,20 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
         const int want = (last && wnorm2) ? 1 : 0;
         const Cols Vc{table ? nullptr : static_cast<const char*>(V) + done * ld * elem, ld * elem,
                       table ? table + done : nullptr};
-        if (c)
-            hipLaunchKernelGGL(k_axpy_many<true>, dim3(g), dim3(kThreads), 0, st, coeffs + done, Vc, mc, w, n, part,
+        auto go = [&](auto kernel, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(g), dim3(static_cast<unsigned>(threads)), 0, st, coeffs + done, Vc, mc, w, n, part,
                                want, sign);
-        else
-            hipLaunchKernelGGL(k_axpy_many<false>, dim3(g), dim3(kThreads), 0, st, coeffs + done, Vc, mc, w, n,
-                               part, want, sign);
+        };
+        if (n >= kSplitRows) {
+            if (c) go(k_axpy_many<true>, kThreads);
+            else go(k_axpy_many<false>, kThreads);
+        } else if (rows == 64) {
+            if (c) go(k_axpy_many_split<true, 64>, kSplitThreads);
+            else go(k_axpy_many_split<false, 64>, kSplitThreads);
+        } else {
+            if (c) go(k_axpy_many_split<true, 128>, kSplitThreads);
+            else go(k_axpy_many_split<false, 128>, kSplitThreads);
+        }
         if (want) hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), 2, wnorm2);
         done += static_cast<std::size_t>(mc);
     } while (done < m);
