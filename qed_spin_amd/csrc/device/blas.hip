@@ -85,8 +85,19 @@ template <bool C> __global__ void k_fill_gauss(void* x, std::size_t n, u64 seed)
     }
 }
 
-template <bool C> __global__ void k_axpby(Zd a, const void* x, Zd b, void* y, std::size_t n, int mode) {
+/// A coefficient's value (Coef): given by the host, or read on the device.
+__device__ __forceinline__ Zd coef_value(const Coef& c) {
+    if (c.kind == 1) return Zd{-c.p[0], 0.0};
+    if (c.kind == 2) {
+        const Zd v{c.p[0], c.p[1]};
+        return sqrt(v.re * v.re + v.im * v.im) > c.threshold ? Zd{-v.re, -v.im} : Zd{0.0, 0.0};
+    }
+    return c.a;
+}
+
+template <bool C> __global__ void k_axpby(Coef ca, const void* x, Zd b, void* y, std::size_t n, int mode) {
     // mode 0: y += a x; 1: y *= a; 2: y = a x + b y
+    const Zd a = coef_value(ca);
     for (std::size_t i = blockIdx.x * static_cast<std::size_t>(blockDim.x) + threadIdx.x; i < n;
          i += static_cast<std::size_t>(gridDim.x) * blockDim.x) {
         if (mode == 1) {
@@ -101,10 +112,23 @@ template <bool C> __global__ void k_axpby(Zd a, const void* x, Zd b, void* y, st
     }
 }
 
-// Reduction kinds: 0 dot z^H y; 1 sum |y|^2; both optionally after y += a x (fuse != 0).
+// out = w / *norm (out may be w).
+template <bool C> __global__ void k_scale_by(const void* w, const double* norm, void* out, std::size_t n) {
+    const double f = 1.0 / *norm;
+    for (std::size_t i = blockIdx.x * static_cast<std::size_t>(blockDim.x) + threadIdx.x; i < n;
+         i += static_cast<std::size_t>(gridDim.x) * blockDim.x) {
+        const Zd v = V<C>::load(w, i);
+        V<C>::store(out, i, Zd{v.re * f, v.im * f});
+    }
+}
+
+// Reduction kinds: 0 dot z^H y; 1 sum |y|^2; both optionally after y += a x (fuse != 0; a zero
+// coefficient read on the device adds nothing).
 template <bool C, int KIND>
-__global__ __launch_bounds__(kThreads) void k_reduce(Zd a, const void* x, void* y, const void* z, std::size_t n,
+__global__ __launch_bounds__(kThreads) void k_reduce(Coef ca, const void* x, void* y, const void* z, std::size_t n,
                                                      int fuse, double* partial) {
+    const Zd a = coef_value(ca);
+    if (ca.kind == 2 && a.re == 0.0 && a.im == 0.0) fuse = 0;
     double s0 = 0.0, s1 = 0.0;
     for (std::size_t i = blockIdx.x * static_cast<std::size_t>(blockDim.x) + threadIdx.x; i < n;
          i += static_cast<std::size_t>(gridDim.x) * blockDim.x) {
@@ -151,9 +175,21 @@ __device__ void finish_pairs(const double* partial, int nb, int out_kind, void* 
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_finish(const double* partial, int nb, int out_kind, void* out) {
+__global__ __launch_bounds__(kThreads) void k_finish(const double* partial, int nb, int out_kind, void* out,
+                                                     const int* gate) {
+    if (gate && !*gate) return;
     finish_pairs(partial, nb, out_kind, out);
 }
+
+// The DGKS gate of a Gram-Schmidt pass: beta = the norm it left; the pass is repeated when that is below
+// kappa of the norm it found.
+__global__ void k_cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta) {
+    const double a = sqrt(*after2);
+    *beta = a;
+    *again = a < kappa * sqrt(*before2) ? 1 : 0;
+}
+
+__global__ void k_add_pair(const Zd* a, const Zd* b, Zd* out) { *out = Zd{a->re + b->re, a->im + b->im}; }
 
 // The columns of a Gram-Schmidt block: column j at base + j stride (bytes), or table[j] when a
 // table of device pointers is given (the reference's array-of-vectors form).
@@ -180,7 +216,8 @@ constexpr int kTile = 1024;      // rows per LDS tile
 template <bool C>
 __global__ __launch_bounds__(kThreads) void k_dot_many(Cols Vb, int m, int per, const void* w,
                                                        std::size_t n, std::size_t rows_per_block, double* partial,
-                                                       int nb, int want_norm) {
+                                                       int nb, int want_norm, const int* gate) {
+    if (gate && !*gate) return;
     __shared__ Zd sw[kTile];
     __shared__ Zd acc[kManyCols + 1];
     const std::size_t r0 = blockIdx.x * rows_per_block;
@@ -244,7 +281,8 @@ inline int dot_columns(int m, std::size_t row_blocks) {
 
 // One block per column: the sum of its nb block partials (contiguous) in a fixed order.
 __global__ __launch_bounds__(kThreads) void k_dot_many_finish(const double* partial, int nb, int m, Zd* coeffs,
-                                                              double* wnorm2) {
+                                                              double* wnorm2, const int* gate) {
+    if (gate && !*gate) return;
     const int j = blockIdx.x;
     if (j < m) finish_pairs(partial + static_cast<std::size_t>(j) * nb * 2, nb, 0, coeffs + j);
     else if (wnorm2) finish_pairs(partial + static_cast<std::size_t>(j) * nb * 2, nb, 2, wnorm2);
@@ -254,7 +292,8 @@ __global__ __launch_bounds__(kThreads) void k_dot_many_finish(const double* part
 template <bool C>
 __global__ __launch_bounds__(kThreads) void k_axpy_many(const Zd* coeffs, Cols Vb, int m,
                                                         void* w, std::size_t n, double* partial, int want_norm,
-                                                        double sign) {
+                                                        double sign, const int* gate) {
+    if (gate && !*gate) return;
     __shared__ Zd sc[kManyCols];
     for (int j = threadIdx.x; j < m; j += blockDim.x) sc[j] = Zd{sign * coeffs[j].re, sign * coeffs[j].im};
     __syncthreads();
@@ -307,7 +346,8 @@ constexpr int kSplitThreads = 512;
 template <bool C, int ROWS>
 __global__ __launch_bounds__(kSplitThreads) void k_axpy_many_split(const Zd* coeffs, Cols Vb, int m, void* w,
                                                                    std::size_t n, double* partial, int want_norm,
-                                                                   double sign) {
+                                                                   double sign, const int* gate) {
+    if (gate && !*gate) return;
     constexpr int G = kSplitThreads / ROWS, U = 4;
     __shared__ Zd sc[kManyCols];
     __shared__ Zd share[G - 1][ROWS];
@@ -409,20 +449,36 @@ void fill_gaussian(bool c, void* x, std::size_t n, u64 seed, hipStream_t st) {
     else hipLaunchKernelGGL(k_fill_gauss<false>, dim3(g), dim3(kThreads), 0, st, x, n, seed);
 }
 
-static void launch_axpby(bool c, Zd a, const void* x, Zd b, void* y, std::size_t n, int mode, hipStream_t st) {
+static void launch_axpby(bool c, Coef a, const void* x, Zd b, void* y, std::size_t n, int mode, hipStream_t st) {
     if (!n) return;
     const unsigned g = grid_for(n);
     if (c) hipLaunchKernelGGL(k_axpby<true>, dim3(g), dim3(kThreads), 0, st, a, x, b, y, n, mode);
     else hipLaunchKernelGGL(k_axpby<false>, dim3(g), dim3(kThreads), 0, st, a, x, b, y, n, mode);
 }
 
-void axpy(bool c, Zd a, const void* x, void* y, std::size_t n, hipStream_t st) { launch_axpby(c, a, x, Zd{0, 0}, y, n, 0, st); }
-void scale(bool c, Zd a, void* x, std::size_t n, hipStream_t st) { launch_axpby(c, a, nullptr, Zd{0, 0}, x, n, 1, st); }
+void axpy(bool c, Zd a, const void* x, void* y, std::size_t n, hipStream_t st) { launch_axpby(c, Coef{a}, x, Zd{0, 0}, y, n, 0, st); }
+void axpy(bool c, Coef a, const void* x, void* y, std::size_t n, hipStream_t st) { launch_axpby(c, a, x, Zd{0, 0}, y, n, 0, st); }
+void scale(bool c, Zd a, void* x, std::size_t n, hipStream_t st) { launch_axpby(c, Coef{a}, nullptr, Zd{0, 0}, x, n, 1, st); }
 void axpby(bool c, Zd a, const void* x, Zd b, void* y, std::size_t n, hipStream_t st) {
-    launch_axpby(c, a, x, b, y, n, 2, st);
+    launch_axpby(c, Coef{a}, x, b, y, n, 2, st);
 }
 
-static void reduce(bool c, int kind, Zd a, const void* x, void* y, const void* z, std::size_t n, int fuse,
+void scale_by(bool c, const void* w, const double* norm, void* out, std::size_t n, hipStream_t st) {
+    if (!n) return;
+    const unsigned g = grid_for(n);
+    if (c) hipLaunchKernelGGL(k_scale_by<true>, dim3(g), dim3(kThreads), 0, st, w, norm, out, n);
+    else hipLaunchKernelGGL(k_scale_by<false>, dim3(g), dim3(kThreads), 0, st, w, norm, out, n);
+}
+
+void cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta, hipStream_t st) {
+    hipLaunchKernelGGL(k_cgs_gate, dim3(1), dim3(1), 0, st, before2, after2, kappa, again, beta);
+}
+
+void add_pair(const Zd* a, const Zd* b, Zd* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_add_pair, dim3(1), dim3(1), 0, st, a, b, out);
+}
+
+static void reduce(bool c, int kind, Coef a, const void* x, void* y, const void* z, std::size_t n, int fuse,
                    void* scratch, int out_kind, void* out, hipStream_t st) {
     const unsigned g = grid_for(n);
     double* part = static_cast<double*>(scratch);
@@ -433,25 +489,33 @@ static void reduce(bool c, int kind, Zd a, const void* x, void* y, const void* z
         if (kind == 0) hipLaunchKernelGGL((k_reduce<false, 0>), dim3(g), dim3(kThreads), 0, st, a, x, y, z, n, fuse, part);
         else hipLaunchKernelGGL((k_reduce<false, 1>), dim3(g), dim3(kThreads), 0, st, a, x, y, z, n, fuse, part);
     }
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), out_kind, out);
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), out_kind, out, static_cast<const int*>(nullptr));
 }
 
 void dot(bool c, const void* x, const void* y, std::size_t n, void* scratch, Zd* result, hipStream_t st) {
-    reduce(c, 0, Zd{0, 0}, nullptr, const_cast<void*>(y), x, n, 0, scratch, 0, result, st);
+    reduce(c, 0, Coef{}, nullptr, const_cast<void*>(y), x, n, 0, scratch, 0, result, st);
 }
 void nrm2(bool c, const void* x, std::size_t n, void* scratch, double* result, hipStream_t st) {
-    reduce(c, 1, Zd{0, 0}, nullptr, const_cast<void*>(x), nullptr, n, 0, scratch, 1, result, st);
+    reduce(c, 1, Coef{}, nullptr, const_cast<void*>(x), nullptr, n, 0, scratch, 1, result, st);
 }
 void axpy_dot(bool c, Zd a, const void* x, void* y, const void* z, std::size_t n, void* scratch, Zd* result,
+              hipStream_t st) {
+    reduce(c, 0, Coef{a}, x, y, z, n, 1, scratch, 0, result, st);
+}
+void axpy_dot(bool c, Coef a, const void* x, void* y, const void* z, std::size_t n, void* scratch, Zd* result,
               hipStream_t st) {
     reduce(c, 0, a, x, y, z, n, 1, scratch, 0, result, st);
 }
 void axpy_nrm2(bool c, Zd a, const void* x, void* y, std::size_t n, void* scratch, double* result, hipStream_t st) {
+    reduce(c, 1, Coef{a}, x, y, nullptr, n, 1, scratch, 1, result, st);
+}
+void axpy_nrm2(bool c, Coef a, const void* x, void* y, std::size_t n, void* scratch, double* result, hipStream_t st) {
     reduce(c, 1, a, x, y, nullptr, n, 1, scratch, 1, result, st);
 }
 
 static void dot_many_cols(bool c, const void* V, std::size_t ld, const void* const* table, std::size_t m,
-                          const void* w, std::size_t n, void* scratch, Zd* coeffs, double* wnorm2, hipStream_t st) {
+                          const void* w, std::size_t n, void* scratch, Zd* coeffs, double* wnorm2, hipStream_t st,
+                          const int* gate) {
     double* part = static_cast<double*>(scratch);
     const std::size_t elem = c ? sizeof(Zd) : sizeof(double);
     std::size_t done = 0;
@@ -469,29 +533,29 @@ static void dot_many_cols(bool c, const void* V, std::size_t ld, const void* con
         const dim3 grid(static_cast<unsigned>(nb), static_cast<unsigned>(mc > 0 ? (mc + per - 1) / per : 1));
         if (c)
             hipLaunchKernelGGL(k_dot_many<true>, grid, dim3(kThreads), 0, st, Vc, mc, per, w, n, rpb, part,
-                               static_cast<int>(nb), want);
+                               static_cast<int>(nb), want, gate);
         else
             hipLaunchKernelGGL(k_dot_many<false>, grid, dim3(kThreads), 0, st, Vc, mc, per, w, n, rpb, part,
-                               static_cast<int>(nb), want);
+                               static_cast<int>(nb), want, gate);
         hipLaunchKernelGGL(k_dot_many_finish, dim3(static_cast<unsigned>(mc + want)), dim3(kThreads), 0, st, part,
-                           static_cast<int>(nb), mc, coeffs + done, want ? wnorm2 : nullptr);
+                           static_cast<int>(nb), mc, coeffs + done, want ? wnorm2 : nullptr, gate);
         done += static_cast<std::size_t>(mc);
         first = false;
     } while (done < m);
 }
 
 void dot_many(bool c, const void* V, std::size_t ld, std::size_t m, const void* w, std::size_t n, void* scratch,
-              Zd* coeffs, double* wnorm2, hipStream_t st) {
-    dot_many_cols(c, V, ld, nullptr, m, w, n, scratch, coeffs, wnorm2, st);
+              Zd* coeffs, double* wnorm2, hipStream_t st, const int* gate) {
+    dot_many_cols(c, V, ld, nullptr, m, w, n, scratch, coeffs, wnorm2, st, gate);
 }
 void dot_many_table(bool c, const void* const* table, std::size_t m, const void* w, std::size_t n, void* scratch,
                     Zd* coeffs, hipStream_t st) {
-    if (m) dot_many_cols(c, nullptr, 0, table, m, w, n, scratch, coeffs, nullptr, st);
+    if (m) dot_many_cols(c, nullptr, 0, table, m, w, n, scratch, coeffs, nullptr, st, nullptr);
 }
 
 static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t ld, const void* const* table,
                            std::size_t m, void* w, std::size_t n, void* scratch, double* wnorm2, hipStream_t st,
-                           double sign) {
+                           double sign, const int* gate, bool root) {
     double* part = static_cast<double*>(scratch);
     const std::size_t elem = c ? sizeof(Zd) : sizeof(double);
     const std::size_t rows = n <= 65536 ? 64 : 128;   // k_axpy_many_split's rows per block
@@ -506,7 +570,7 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
                       table ? table + done : nullptr};
         auto go = [&](auto kernel, int threads) {
             hipLaunchKernelGGL(kernel, dim3(g), dim3(static_cast<unsigned>(threads)), 0, st, coeffs + done, Vc, mc, w, n, part,
-                               want, sign);
+                               want, sign, gate);
         };
         if (n >= kSplitRows) {
             if (c) go(k_axpy_many<true>, kThreads);
@@ -518,18 +582,19 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
             if (c) go(k_axpy_many_split<true, 128>, kSplitThreads);
             else go(k_axpy_many_split<false, 128>, kSplitThreads);
         }
-        if (want) hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), 2, wnorm2);
+        if (want) hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), root ? 1 : 2,
+                                     wnorm2, gate);
         done += static_cast<std::size_t>(mc);
     } while (done < m);
 }
 
 void axpy_many(bool c, const Zd* coeffs, const void* V, std::size_t ld, std::size_t m, void* w, std::size_t n,
-               void* scratch, double* wnorm2, hipStream_t st, double sign) {
-    axpy_many_cols(c, coeffs, V, ld, nullptr, m, w, n, scratch, wnorm2, st, sign);
+               void* scratch, double* wnorm2, hipStream_t st, double sign, const int* gate, bool root) {
+    axpy_many_cols(c, coeffs, V, ld, nullptr, m, w, n, scratch, wnorm2, st, sign, gate, root);
 }
 void axpy_many_table(bool c, const Zd* coeffs, const void* const* table, std::size_t m, void* w, std::size_t n,
                      hipStream_t st) {
-    if (m) axpy_many_cols(c, coeffs, nullptr, 0, table, m, w, n, nullptr, nullptr, st, 1.0);
+    if (m) axpy_many_cols(c, coeffs, nullptr, 0, table, m, w, n, nullptr, nullptr, st, 1.0, nullptr, false);
 }
 
 void block_rotate(bool c, const void* Vm, std::size_t ld, std::size_t mm, const double* S, std::size_t cols, void* out,

@@ -143,11 +143,11 @@ void sell_fill(const u64* row_ptr, const u32* col, const void* vals, int value_b
 
 /// Workgroups of sell_lanczos on A (its partial buffer holds two doubles per workgroup).
 unsigned sell_lanczos_blocks(const CsrView& A);
-/// The first pass of a Lanczos step in the SELL SpMV's epilogue: w = A v - beta v_prev (v_prev null:
-/// w = A v), and <v, w> into alpha (device) through partial (2 sell_lanczos_blocks(A) doubles), summed
-/// in a fixed order. false (nothing launched) without the SELL layout, or real vectors on complex
+/// The first pass of a Lanczos step in the SELL SpMV's epilogue: w = A v - *beta v_prev (v_prev null:
+/// w = A v; beta on the device), and <v, w> into alpha (device) through partial (2 sell_lanczos_blocks(A)
+/// doubles), summed in a fixed order. false (nothing launched) without the SELL layout, or real vectors on complex
 /// values.
-bool sell_lanczos(const CsrView& A, bool real, const void* v, const void* vprev, double beta, void* w,
+bool sell_lanczos(const CsrView& A, bool real, const void* v, const void* vprev, const double* beta, void* w,
                   double* partial, Zd* alpha, hipStream_t st);
 
 // ---- blas.hip (vectors of T = double or Zd; n entries) -------------------------------------------
@@ -159,7 +159,25 @@ void fill_zero(bool cplx, void* x, std::size_t n, hipStream_t st);
 /// x[i] = standard normal entries (complex: both parts) from a counter hash of (seed, i): test and
 /// benchmark vectors, not the FTLM samples.
 void fill_gaussian(bool cplx, void* x, std::size_t n, u64 seed, hipStream_t st);
+/// A coefficient of an update: a value the host knows, or one that lies on the device (no
+/// synchronisation to read it): kind 1 -p[0]; kind 2 -(p[0], p[1]) when its modulus exceeds threshold,
+/// else zero (the update is then left out).
+struct Coef {
+    Zd a{0.0, 0.0};
+    const double* p = nullptr;
+    int kind = 0;
+    double threshold = 0.0;
+};
+inline Coef minus(const double* p) { return Coef{Zd{0.0, 0.0}, p, 1, 0.0}; }
+inline Coef minus_above(const Zd* p, double threshold) { return Coef{Zd{0.0, 0.0}, &p->re, 2, threshold}; }
 void axpy(bool cplx, Zd a, const void* x, void* y, std::size_t n, hipStream_t st);
+void axpy(bool cplx, Coef a, const void* x, void* y, std::size_t n, hipStream_t st);
+/// out = w / *norm (device; out may be w).
+void scale_by(bool cplx, const void* w, const double* norm, void* out, std::size_t n, hipStream_t st);
+/// *beta = sqrt(*after2); *again = that is below kappa sqrt(*before2) (all on the device).
+void cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta, hipStream_t st);
+/// *out = *a + *b (device scalars).
+void add_pair(const Zd* a, const Zd* b, Zd* out, hipStream_t st);
 void scale(bool cplx, Zd a, void* x, std::size_t n, hipStream_t st);
 void axpby(bool cplx, Zd a, const void* x, Zd b, void* y, std::size_t n, hipStream_t st);
 /// result (device, one Zd) = x^H y.
@@ -169,17 +187,22 @@ void nrm2(bool cplx, const void* x, std::size_t n, void* scratch, double* result
 /// y += a x; result = z^H y.
 void axpy_dot(bool cplx, Zd a, const void* x, void* y, const void* z, std::size_t n, void* scratch, Zd* result,
               hipStream_t st);
+void axpy_dot(bool cplx, Coef a, const void* x, void* y, const void* z, std::size_t n, void* scratch, Zd* result,
+              hipStream_t st);
 /// y += a x; result = ||y||.
 void axpy_nrm2(bool cplx, Zd a, const void* x, void* y, std::size_t n, void* scratch, double* result,
                hipStream_t st);
+void axpy_nrm2(bool cplx, Coef a, const void* x, void* y, std::size_t n, void* scratch, double* result,
+               hipStream_t st);
 /// coeffs[j] = V_j^H w for the m columns of the block V (column j at V + j ld); also ||w||^2 into
-/// *wnorm2 when non-null.
+/// *wnorm2 when non-null. gate (device, or null): nothing is done or written when it holds 0.
 void dot_many(bool cplx, const void* V, std::size_t ld, std::size_t m, const void* w, std::size_t n, void* scratch,
-              Zd* coeffs, double* wnorm2, hipStream_t st);
-/// w += sign sum_j coeffs[j] V_j (coeffs in device memory); ||w||^2 after the update into *wnorm2
-/// when non-null.
+              Zd* coeffs, double* wnorm2, hipStream_t st, const int* gate = nullptr);
+/// w += sign sum_j coeffs[j] V_j (coeffs in device memory); ||w||^2 (root: ||w||) after the update into
+/// *wnorm2 when non-null. gate as above.
 void axpy_many(bool cplx, const Zd* coeffs, const void* V, std::size_t ld, std::size_t m, void* w, std::size_t n,
-               void* scratch, double* wnorm2, hipStream_t st, double sign = 1.0);
+               void* scratch, double* wnorm2, hipStream_t st, double sign = 1.0, const int* gate = nullptr,
+               bool root = false);
 
 /// dot_many / axpy_many over columns given as a device array of m device pointers (the reference's
 /// array-of-vectors form, BasicBackend::dot_many / axpy_many). axpy_many_table: w += sum_j c_j V_j.

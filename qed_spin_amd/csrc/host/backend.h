@@ -78,60 +78,57 @@ public:
         return read_double(0);
     }
 
-    /// One classical Gram-Schmidt pass against the m columns of the contiguous block V (column j
-    /// at V + j ld): w -= V (V^H w). Returns (||w|| before, ||w|| after). The coefficients stay on
-    /// the device (the host never needs them).
-    std::pair<double, double> cgs_pass(const Scalar* V, std::size_t ld, std::size_t m, Scalar* w, std::size_t n) const {
-        if (coeff_.bytes() < m * sizeof(dev::Zd)) coeff_.reset(std::max<std::size_t>(m, 64) * 2 * sizeof(dev::Zd));
-        double* norms = result_.get<double>() + 4;
-        dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), coeff_.get<dev::Zd>(), norms, st());
-        dev::axpy_many(kComplex, coeff_.get<dev::Zd>(), V, ld, m, w, n, scratch_.get(), norms + 1, st(), -1.0);
-        double h[2];
-        QSA_HIP(hipMemcpyAsync(h, norms, 16, hipMemcpyDeviceToHost, st()));
-        QSA_HIP(hipStreamSynchronize(st()));
-        return {std::sqrt(h[0]), std::sqrt(h[1])};
+    // ---- steps whose scalars stay on the device (nothing here waits) -------------------------------
+    /// y += a x
+    void axpy(dev::Coef a, const Scalar* x, Scalar* y, std::size_t n) const { dev::axpy(kComplex, a, x, y, n, st()); }
+    /// *result = x^H y
+    void dot(const Scalar* x, const Scalar* y, std::size_t n, dev::Zd* result) const {
+        dev::dot(kComplex, x, y, n, scratch_.get(), result, st());
     }
-
-    /// Two unconditional classical Gram-Schmidt passes of w against the m >= 1 contiguous columns
-    /// of V. Returns the coefficient of the last column summed over both passes (V_{m-1}^H w as w
-    /// was) and ||w|| after, read back together in one synchronisation.
-    std::pair<Scalar, double> cgs2_tail(const Scalar* V, std::size_t ld, std::size_t m, Scalar* w, std::size_t n) const {
-        if (coeff_.bytes() < 2 * m * sizeof(dev::Zd)) coeff_.reset(std::max<std::size_t>(m, 64) * 2 * sizeof(dev::Zd));
-        dev::Zd* c1 = coeff_.get<dev::Zd>();
+    /// y += a x; *result = z^H y
+    void axpy_dot(dev::Coef a, const Scalar* x, Scalar* y, const Scalar* zz, std::size_t n, dev::Zd* result) const {
+        dev::axpy_dot(kComplex, a, x, y, zz, n, scratch_.get(), result, st());
+    }
+    /// y += a x; *result = ||y||
+    void axpy_nrm2(dev::Coef a, const Scalar* x, Scalar* y, std::size_t n, double* result) const {
+        dev::axpy_nrm2(kComplex, a, x, y, n, scratch_.get(), result, st());
+    }
+    /// out = w / *norm
+    void scale_by(const Scalar* w, const double* norm, Scalar* out, std::size_t n) const {
+        dev::scale_by(kComplex, w, norm, out, n, st());
+    }
+    /// One classical Gram-Schmidt pass of w against the m columns of the contiguous block V (column j at
+    /// V + j ld), w -= V (V^H w), and a second one where the first left less than kappa of ||w||:
+    /// *beta = ||w|| after.
+    void cgs_gated(const Scalar* V, std::size_t ld, std::size_t m, Scalar* w, std::size_t n, double kappa,
+                   double* beta) const {
+        dev::Zd* c = coefficients(m);
+        double* norms = result_.get<double>() + 4;
+        int* again = reinterpret_cast<int*>(result_.get<double>() + 6);
+        dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c, norms, st());
+        dev::axpy_many(kComplex, c, V, ld, m, w, n, scratch_.get(), norms + 1, st(), -1.0);
+        dev::cgs_gate(norms, norms + 1, kappa, again, beta, st());
+        dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c, nullptr, st(), again);
+        dev::axpy_many(kComplex, c, V, ld, m, w, n, scratch_.get(), beta, st(), -1.0, again, true);
+    }
+    /// Two unconditional classical Gram-Schmidt passes of w against the m >= 1 columns of V: *tail =
+    /// the last column's coefficient summed over both, *norm = ||w|| after.
+    void cgs2(const Scalar* V, std::size_t ld, std::size_t m, Scalar* w, std::size_t n, dev::Zd* tail, double* norm) const {
+        dev::Zd* c1 = coefficients(2 * m);
         dev::Zd* c2 = c1 + m;
-        double* norm = result_.get<double>() + 8;
         dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c1, nullptr, st());
         dev::axpy_many(kComplex, c1, V, ld, m, w, n, scratch_.get(), nullptr, st(), -1.0);
         dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c2, nullptr, st());
-        dev::axpy_many(kComplex, c2, V, ld, m, w, n, scratch_.get(), norm, st(), -1.0);
-        dev::Zd tail[2];
-        double nn = 0.0;
-        QSA_HIP(hipMemcpyAsync(&tail[0], c1 + (m - 1), sizeof(dev::Zd), hipMemcpyDeviceToHost, st()));
-        QSA_HIP(hipMemcpyAsync(&tail[1], c2 + (m - 1), sizeof(dev::Zd), hipMemcpyDeviceToHost, st()));
-        QSA_HIP(hipMemcpyAsync(&nn, norm, sizeof(double), hipMemcpyDeviceToHost, st()));
-        QSA_HIP(hipStreamSynchronize(st()));
-        return {from_z(dev::Zd{tail[0].re + tail[1].re, tail[0].im + tail[1].im}), std::sqrt(nn)};
+        dev::axpy_many(kComplex, c2, V, ld, m, w, n, scratch_.get(), norm, st(), -1.0, nullptr, true);
+        dev::add_pair(c1 + (m - 1), c2 + (m - 1), tail, st());
     }
 
-    /// coeffs_out[j] = V_j^H v for the m columns of V (host result).
-    void dot_many_block(const Scalar* V, std::size_t ld, std::size_t m, const Scalar* v, std::size_t n,
-                        Scalar* coeffs_out) const {
-        if (coeff_.bytes() < m * sizeof(dev::Zd)) coeff_.reset(std::max<std::size_t>(m, 64) * 2 * sizeof(dev::Zd));
-        dev::dot_many(kComplex, V, ld, m, v, n, scratch_.get(), coeff_.get<dev::Zd>(), nullptr, st());
-        std::vector<dev::Zd> h(m);
-        QSA_HIP(hipMemcpyAsync(h.data(), coeff_.get(), m * sizeof(dev::Zd), hipMemcpyDeviceToHost, st()));
-        QSA_HIP(hipStreamSynchronize(st()));
-        for (std::size_t j = 0; j < m; ++j) coeffs_out[j] = from_z(h[j]);
-    }
-    /// v += sum_j coeffs[j] V_j (host coefficients).
-    void axpy_many_block(const Scalar* coeffs, const Scalar* V, std::size_t ld, std::size_t m, Scalar* v,
-                         std::size_t n) const {
-        if (coeff_.bytes() < m * sizeof(dev::Zd)) coeff_.reset(std::max<std::size_t>(m, 64) * 2 * sizeof(dev::Zd));
-        std::vector<dev::Zd> h(m);
-        for (std::size_t j = 0; j < m; ++j) h[j] = z(coeffs[j]);
-        QSA_HIP(hipMemcpyAsync(coeff_.get(), h.data(), m * sizeof(dev::Zd), hipMemcpyHostToDevice, st()));
-        dev::axpy_many(kComplex, coeff_.get<dev::Zd>(), V, ld, m, v, n, scratch_.get(), nullptr, st());
-        QSA_HIP(hipStreamSynchronize(st()));
+    /// Two unconditional classical Gram-Schmidt passes of w against the m >= 1 contiguous columns of V;
+    /// ||w|| after, read back.
+    double cgs2_norm(const Scalar* V, std::size_t ld, std::size_t m, Scalar* w, std::size_t n) const {
+        double* norm = result_.get<double>() + 8;
+        cgs2(V, ld, m, w, n, result_.get<dev::Zd>() + 5, norm);
+        return read_double(8);
     }
 
     void synchronize() const { QSA_HIP(hipStreamSynchronize(st())); }
@@ -145,6 +142,11 @@ private:
     static Scalar from_z(dev::Zd v) {
         if constexpr (kComplex) return Scalar(v.re, v.im);
         else return v.re;
+    }
+    /// Room for m coefficients.
+    dev::Zd* coefficients(std::size_t m) const {
+        if (coeff_.bytes() < m * sizeof(dev::Zd)) coeff_.reset(std::max<std::size_t>(m, 64) * 2 * sizeof(dev::Zd));
+        return coeff_.get<dev::Zd>();
     }
     Scalar read_scalar() const {
         dev::Zd h;

@@ -179,6 +179,8 @@ public:
         Q_ = be.make_zero_vector(n * (mid_ + m_ + 1));
         w_ = be.make_zero_vector(n);
         keep_ = be.make_zero_vector(n * m_);
+        diag_.reset(m_ * sizeof(dev::Zd));
+        norm_.reset(m_ * sizeof(double));
     }
 
     /// Runs to k locked levels (verified against missed degenerate copies) or the apply budget.
@@ -253,11 +255,12 @@ private:
         --locked_;
     }
 
-    /// Columns [mid_ - locked_, mid_ + j) as one block: the locked vectors and active columns < j.
-    std::pair<Scalar, double> orthogonalize(Scalar* x, std::size_t j) {
+    /// x orthogonalised against the locked vectors and the active columns < j, one block of columns
+    /// [mid_ - locked_, mid_ + j); its norm after.
+    double orthogonalize(Scalar* x, std::size_t j) {
         const std::size_t cols = locked_ + j;
-        if (cols == 0) return {Scalar(0), be_.nrm2(x, n_)};
-        return be_.cgs2_tail(lowest_locked(), n_, cols, x, n_);
+        if (cols == 0) return be_.nrm2(x, n_);
+        return be_.cgs2_norm(lowest_locked(), n_, cols, x, n_);
     }
 
     /// Lock `want` more levels starting from the vector in active column 0. With a finite give_up,
@@ -266,7 +269,7 @@ private:
         const std::size_t target = locked_ + want;
         bool first_cycle = true;
         {
-            const double nrm = orthogonalize(col(0), 0).second;
+            const double nrm = orthogonalize(col(0), 0);
             if (nrm < 1e-12) return Search::kNullStart;
             be_.scale(Scalar(1.0 / nrm), col(0), n_);
         }
@@ -284,20 +287,29 @@ private:
             }
             std::size_t size = m;
             double tail = 0.0;
+            // the cycle's steps, their scalars on the device; read when all are enqueued, and cut at
+            // the step that found an invariant subspace (what lies past it is not used)
             for (std::size_t j = kept; j < m; ++j) {
                 H_(col(j), w_.get());
+                be_.cgs2(lowest_locked(), n_, locked_ + j + 1, w_.get(), n_, diag_.get<dev::Zd>() + j,
+                         norm_.get<double>() + j);
+                be_.scale_by(w_.get(), norm_.get<double>() + j, col(j + 1), n_);
+            }
+            QSA_HIP(hipGetLastError());
+            std::vector<dev::Zd> diag(m);
+            std::vector<double> norm(m);
+            copy_to_host(diag.data() + kept, diag_.get<dev::Zd>() + kept, (m - kept) * sizeof(dev::Zd));
+            copy_to_host(norm.data() + kept, norm_.get<double>() + kept, (m - kept) * sizeof(double));
+            for (std::size_t j = kept; j < m; ++j) {
                 ++applies_;
-                const auto [diag, beta] = orthogonalize(w_.get(), j + 1);
-                T[j * m + j] = std::real(diag);
-                if (beta <= s_.breakdown_tol || j + 1 == n_ - locked_) {   // invariant subspace
+                T[j * m + j] = diag[j].re;
+                if (norm[j] <= s_.breakdown_tol || j + 1 == n_ - locked_) {   // invariant subspace
                     size = j + 1;
                     tail = 0.0;
                     break;
                 }
-                if (j + 1 < m) T[j * m + j + 1] = T[(j + 1) * m + j] = beta;
-                be_.copy(w_.get(), col(j + 1), n_);
-                be_.scale(Scalar(1.0 / beta), col(j + 1), n_);
-                tail = beta;
+                if (j + 1 < m) T[j * m + j + 1] = T[(j + 1) * m + j] = norm[j];
+                tail = norm[j];
             }
             std::vector<double> Ts(size * size);
             for (std::size_t c = 0; c < size; ++c)
@@ -365,6 +377,7 @@ private:
     std::size_t n_, k_ = 1, m_ = 1, mid_ = 2, locked_ = 0, applies_ = 0;
     Settings s_;
     typename HipBackend<Scalar>::UniqueVec Q_, w_, keep_;
+    DeviceBuffer diag_, norm_;   // a cycle's diagonal entries and norms
     std::vector<double> value_;
 };
 

@@ -500,19 +500,15 @@ void SectorOperator::apply(const void* in, void* out, bool complex_vectors) cons
     apply_multi(ins, outs, 1, complex_vectors);
 }
 
-bool SectorOperator::lanczos_first_pass(const void* v, const void* vprev, double beta, void* w, bool complex_vectors,
-                                        cplx* alpha) const {
+bool SectorOperator::lanczos_first_pass(const void* v, const void* vprev, const double* beta, void* w,
+                                        bool complex_vectors, dev::Zd* alpha, DeviceBuffer& scratch) const {
     if (lane_ != kLaneCsr || !sell() || !same()) return false;
     const dev::CsrView A = csr_view(false, true);
-    const hipStream_t st = engine_stream();
-    DeviceBuffer partial(static_cast<std::size_t>(dev::sell_lanczos_blocks(A)) * 2 * sizeof(double) + sizeof(dev::Zd));
-    dev::Zd* a = reinterpret_cast<dev::Zd*>(partial.get<char>() + partial.bytes() - sizeof(dev::Zd));
-    if (!dev::sell_lanczos(A, real_ && !complex_vectors, v, vprev, beta, w, partial.get<double>(), a, st)) return false;
+    const std::size_t need = static_cast<std::size_t>(dev::sell_lanczos_blocks(A)) * 2 * sizeof(double);
+    if (scratch.bytes() < need) scratch.reset(need);
+    if (!dev::sell_lanczos(A, real_ && !complex_vectors, v, vprev, beta, w, scratch.get<double>(), alpha, engine_stream()))
+        return false;
     QSA_HIP(hipGetLastError());
-    dev::Zd h{};
-    QSA_HIP(hipMemcpyAsync(&h, a, sizeof(h), hipMemcpyDeviceToHost, st));
-    QSA_HIP(hipStreamSynchronize(st));
-    *alpha = cplx(h.re, h.im);
     return true;
 }
 

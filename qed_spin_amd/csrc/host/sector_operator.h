@@ -55,10 +55,11 @@ public:
     /// on the engine stream.
     void apply(const void* in, void* out, bool complex_vectors = false) const;
     /// The first pass of a Lanczos step fused into the apply (the SELL layout only): w = H v -
-    /// beta v_prev (v_prev null: w = H v) and <v, w> into *alpha. false (nothing done) when the
+    /// *beta v_prev (v_prev null: w = H v) and <v, w> into *alpha, the scalars on the device, nothing
+    /// waited for; scratch holds the partial sums and grows as needed. false (nothing done) when the
     /// operator cannot (no SELL layout, not square): the caller applies and forms alpha itself.
-    bool lanczos_first_pass(const void* v, const void* vprev, double beta, void* w, bool complex_vectors,
-                            cplx* alpha) const;
+    bool lanczos_first_pass(const void* v, const void* vprev, const double* beta, void* w, bool complex_vectors,
+                            dev::Zd* alpha, DeviceBuffer& scratch) const;
     /// outs[i] = O ins[i], i < k (k-vector applies equal k single applies bit for bit).
     void apply_multi(const void* const* ins, void* const* outs, int k, bool complex_vectors = false) const;
     /// Block-interleaved vectors: X[row * nv + i] (nv in 1, 2, 4, 8); CSR lane only.
@@ -141,12 +142,9 @@ template <class Scalar> struct OperatorMatvec {
     const SectorOperator& op;
     bool complex_vectors;
     void operator()(const Scalar* in, Scalar* out) const { op.apply(in, out, complex_vectors); }
-    bool first_pass(const Scalar* v, const Scalar* vprev, double beta, Scalar* w, Scalar& alpha) const {
-        cplx a;
-        if (!op.lanczos_first_pass(v, vprev, beta, w, complex_vectors, &a)) return false;
-        if constexpr (std::is_same_v<Scalar, double>) alpha = a.real();
-        else alpha = a;
-        return true;
+    bool first_pass(const Scalar* v, const Scalar* vprev, const double* beta, Scalar* w, dev::Zd* alpha,
+                    DeviceBuffer& scratch) const {
+        return op.lanczos_first_pass(v, vprev, beta, w, complex_vectors, alpha, scratch);
     }
 };
 
