@@ -455,18 +455,77 @@ __global__ __launch_bounds__(kFinishThreads) void k_lanczos_finish(const double*
     if (threadIdx.x == 0) *alpha = Zd{sr[0], si[0]};
 }
 
-// Block-interleaved vectors X[row * NV + k] on the SELL layout. ACC lanes share a row, lane l
-// taking entries k = l, l + ACC, ... in order (the single-vector kernel's partial sums), combined
-// by the xor butterfly whose order is that kernel's tree: the same bits as single applies.
-template <int WIDTH, bool VREAL, bool REAL, bool LD, int NV, int ACC>
-__global__ __launch_bounds__(1024) void k_sell_block(CsrView A, const void* X, void* Y) {
+// Block-interleaved vectors X[row * NV + k] on the SELL layout: LR lanes share a row, each holding 16
+// bytes of its vectors (one complex or two real) in the single-vector kernel's ACC partial sums and
+// tree, so the same bits as single applies. What bounds a gather is the vector cache's one line a
+// clock among adjacent lanes, so lanes side by side read the two to eight pieces of one row of X
+// rather than each lane all pieces of its own row; the row's entries are read by its lanes from the
+// same addresses. us a launch, each lane all pieces / so: 1.43 million rows, 4 complex 367 / 335 (19
+// million L2 misses at 7.2 TB/s of 128-byte lines); 400,023 rows, complex 2, 4, 8: 37 / 36, 57 / 53,
+// 118 / 79; 2.7 million, real 8: 293 / 245. (4 complex at 1.43 million rows:
+// eight entries a round 352, the next group's entries prefetched 357, a row's sums on twice the lanes
+// 373: more registers or rows further apart in flight.)
+struct alignas(8) Two {
+    double a, b;
+};
+
+template <int WIDTH, bool VREAL, bool REAL, bool LD, int LR, int ACC>
+__global__ __launch_bounds__(1024) void k_sell_block(CsrView A, const Two* X, Two* Y) {
     const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
+    const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
+    const i64 row = gid / LR;
+    const u32 lane = static_cast<u32>(gid % LR);
+    if (row >= A.rows) return;
+    const u32 n = A.nt ? __builtin_nontemporal_load(A.sell_len + row) : A.sell_len[row];
+    const u64 first = A.sell_ptr[row >> 6] + static_cast<u64>(row & 63) * 4;
+    double s0[ACC], s1[ACC];
+#pragma unroll
+    for (int j = 0; j < ACC; ++j) s0[j] = s1[j] = 0.0;
+    auto accumulate = [&](int j, const Two& x, double vr, double vi) {
+        if constexpr (REAL) {
+            s0[j] += vr * x.a;
+            s1[j] += vr * x.b;
+        } else {
+            s0[j] += vr * x.a - vi * x.b;
+            s1[j] += vr * x.b + vi * x.a;
+        }
+    };
+    u32 k = 0;
+    for (; k + 4 <= n; k += 4) {
+        u32 c[4];
+        double vr[4], vi[4] = {0.0, 0.0, 0.0, 0.0};
+        Two x[4];
+        load_quad<WIDTH, VREAL, LD>(A, d, first + static_cast<u64>(k / 4) * 256, c, vr, vi);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = X[static_cast<u64>(c[u]) * LR + lane];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) accumulate(u % ACC, x[u], vr[u], vi[u]);
+    }
+    if (k < n) {   // the last group, entries below n
+        u32 c[4];
+        double vr[4], vi[4] = {0.0, 0.0, 0.0, 0.0};
+        load_quad<WIDTH, VREAL, LD>(A, d, first + static_cast<u64>(k / 4) * 256, c, vr, vi);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + static_cast<u32>(u) < n) accumulate(u % ACC, X[static_cast<u64>(c[u]) * LR + lane], vr[u], vi[u]);
+    }
+    Y[static_cast<u64>(row) * LR + lane] = Two{tree<ACC>(s0), tree<ACC>(s1)};
+}
+
+// The same for 2 and 4 real vectors: ACC lanes share a row, lane l taking entries l, l + ACC, ..., their
+// sums combined by the xor butterfly in the tree's order. With 16 or 32 bytes a row of X, fewer rows in
+// flight weigh more than the cache's lines where a sector's columns scatter (1.43 million rows of a
+// momentum sector, 2 and 4 vectors: 103 and 143 us, one lane or two per row 113 and 150; 400,023 rows,
+// 4 vectors: 36 and 37), though not without a lattice symmetry (705,432 rows: 31 and 41, there 24 and 35).
+template <int WIDTH, bool LD, int NV, int ACC>
+__global__ __launch_bounds__(1024) void k_sell_block_rows(CsrView A, const double* X, double* Y) {
+    const Dict<LD> d = stage_dict<WIDTH, true, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / ACC;
     const int lane = static_cast<int>(gid % ACC);
-    double ar[NV], ai[NV];
+    double ar[NV];
 #pragma unroll
-    for (int q = 0; q < NV; ++q) ar[q] = ai[q] = 0.0;
+    for (int q = 0; q < NV; ++q) ar[q] = 0.0;
     if (row < A.rows) {
         const u32 n = A.sell_len[row];
         const u64 slice = A.sell_ptr[row >> 6];
@@ -474,34 +533,20 @@ __global__ __launch_bounds__(1024) void k_sell_block(CsrView A, const void* X, v
         for (u32 k = static_cast<u32>(lane); k < n; k += ACC) {
             u32 c32;
             double vr, vi = 0.0;
-            load_entry<WIDTH, VREAL, LD>(A, d, sell_at(slice, j, k), c32, vr, vi);
-            const u64 c = c32;
+            load_entry<WIDTH, true, LD>(A, d, sell_at(slice, j, k), c32, vr, vi);
+            const double* x = X + static_cast<u64>(c32) * NV;
 #pragma unroll
-            for (int q = 0; q < NV; ++q) {
-                if constexpr (REAL) {
-                    ar[q] += vr * static_cast<const double*>(X)[c * NV + q];
-                } else {
-                    const Zd x = static_cast<const Zd*>(X)[c * NV + q];
-                    ar[q] += vr * x.re - vi * x.im;
-                    ai[q] += vr * x.im + vi * x.re;
-                }
-            }
+            for (int q = 0; q < NV; ++q) ar[q] += vr * x[q];
         }
     }
 #pragma unroll
     for (int off = ACC / 2; off > 0; off >>= 1) {
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            ar[q] += __shfl_xor(ar[q], off, ACC);
-            if constexpr (!REAL) ai[q] += __shfl_xor(ai[q], off, ACC);
-        }
+        for (int q = 0; q < NV; ++q) ar[q] += __shfl_xor(ar[q], off, ACC);
     }
     if (row < A.rows && lane == 0) {
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            if constexpr (REAL) static_cast<double*>(Y)[row * NV + q] = ar[q];
-            else static_cast<Zd*>(Y)[row * NV + q] = Zd{ar[q], ai[q]};
-        }
+        for (int q = 0; q < NV; ++q) Y[row * NV + q] = ar[q];
     }
 }
 
@@ -570,15 +615,34 @@ inline CsrView block_view(const CsrView& A) {
 template <int WIDTH, bool VREAL, bool REAL, int ACC>
 void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
     const CsrView B = block_view(A);
-    const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(block_threads(B));
+    if constexpr (REAL) {
+        if (nv <= 4) {
+            const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(block_threads(B));
+            by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+                constexpr bool LD = decltype(in_lds)::value;
+                const double* x = static_cast<const double*>(X);
+                double* y = static_cast<double*>(Y);
+                if (nv == 2) hipLaunchKernelGGL((k_sell_block_rows<WIDTH, LD, 2, ACC>), grid, block, lds, st, B, x, y);
+                else hipLaunchKernelGGL((k_sell_block_rows<WIDTH, LD, 4, ACC>), grid, block, lds, st, B, x, y);
+            });
+            return;
+        }
+    }
+    const int lanes = REAL ? nv / 2 : nv;   // 16 bytes each
+    const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * static_cast<u64>(lanes))), block(block_threads(B));
     by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
-#define QSA_SELL_BLOCK(NV) hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, LD, NV, ACC>), grid, block, lds, st, B, X, Y)
-        switch (nv) {
-        case 1: QSA_SELL_BLOCK(1); break;
-        case 2: QSA_SELL_BLOCK(2); break;
+#define QSA_SELL_BLOCK(LR)                                                                                     \
+    hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, LD, LR, ACC>), grid, block, lds, st, B,               \
+                       static_cast<const Two*>(X), static_cast<Two*>(Y))
+        switch (lanes) {
+        case 2:
+            if constexpr (!REAL) QSA_SELL_BLOCK(2);
+            break;
         case 4: QSA_SELL_BLOCK(4); break;
-        case 8: QSA_SELL_BLOCK(8); break;
+        case 8:
+            if constexpr (!REAL) QSA_SELL_BLOCK(8);
+            break;
         default: break;
         }
 #undef QSA_SELL_BLOCK
@@ -586,7 +650,13 @@ void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hip
 }
 template <int WIDTH, bool VREAL, bool REAL>
 void launch_sell_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    if (A.sell_acc == 4) launch_sell_block_acc<WIDTH, VREAL, REAL, 4>(A, nv, X, Y, st);
+    if (nv == 1) {   // one vector: the single apply
+        VecSet v;
+        v.k = 1;
+        v.in[0] = X;
+        v.out[0] = Y;
+        launch_sell_set<WIDTH, VREAL, REAL>(A, v, st);
+    } else if (A.sell_acc == 4) launch_sell_block_acc<WIDTH, VREAL, REAL, 4>(A, nv, X, Y, st);
     else launch_sell_block_acc<WIDTH, VREAL, REAL, 1>(A, nv, X, Y, st);
 }
 
