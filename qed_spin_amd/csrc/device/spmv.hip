@@ -769,6 +769,28 @@ __global__ __launch_bounds__(256) void k_sell_lengths(const u64* row_ptr, i64 ro
 // diag_first (a square operator): a row's diagonal entry, when it has one, moves to its first slot,
 // the others keeping their order -- the k = 0 loads of a wavefront then read x[row] for 64
 // consecutive rows, one coalesced line instead of 64 gathers.
+// A lane gathers four entries of its row and writes the group whole, zeros past the row's end: a
+// wavefront's stores are 1 KB of consecutive words (20.7 million entries: 626 us an entry at a time
+// into cleared memory, 182 so). What the slice holds past a row's last group is never read.
+template <class T, int V> struct alignas(sizeof(T) * V) Group {
+    T v[V];
+};
+
+template <class T, class G>
+__device__ __forceinline__ void sell_group(const void* vals, void* sell_vals, u64 dst, const G& source) {
+    constexpr int V = sizeof(T) >= 8 ? 16 / sizeof(T) : 4;   // 16 bytes a store at most
+#pragma unroll
+    for (int h = 0; h < 4 / V; ++h) {
+        Group<T, V> w;
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const u64 from = source(h * V + u);
+            w.v[u] = from == ~u64{0} ? T{} : static_cast<const T*>(vals)[from];
+        }
+        *reinterpret_cast<Group<T, V>*>(static_cast<T*>(sell_vals) + dst + h * V) = w;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_sell_fill(const u64* row_ptr, const u32* col, const void* vals, int vb,
                                                    i64 rows, const u64* sell_ptr, u32* sell_col, void* sell_vals,
                                                    int diag_first, int packed) {
@@ -781,15 +803,19 @@ __global__ __launch_bounds__(256) void k_sell_fill(const u64* row_ptr, const u32
     if (diag_first)
         for (u64 k = 0; k < n && diag == n; ++k)
             if ((packed ? (col[e0 + k] & 0xFFFFFFu) : col[e0 + k]) == static_cast<u32>(r)) diag = k;
-    for (u64 k = 0; k < n; ++k) {
+    for (u64 k0 = 0; k0 < n; k0 += 4) {
         // slot k takes the diagonal first, then the row's other entries in order
-        const u64 from = diag == n ? k : (k == 0 ? diag : (k <= diag ? k - 1 : k));
-        const u64 dst = sell_at(slice, j, static_cast<u32>(k)), src = e0 + from;
-        sell_col[dst] = col[src];
-        if (vb == 1) static_cast<u8*>(sell_vals)[dst] = static_cast<const u8*>(vals)[src];
-        else if (vb == 2) static_cast<u16*>(sell_vals)[dst] = static_cast<const u16*>(vals)[src];
-        else if (vb == 8) static_cast<double*>(sell_vals)[dst] = static_cast<const double*>(vals)[src];
-        else if (vb == 16) static_cast<Zd*>(sell_vals)[dst] = static_cast<const Zd*>(vals)[src];
+        auto source = [&](int u) -> u64 {
+            const u64 k = k0 + static_cast<u64>(u);
+            if (k >= n) return ~u64{0};
+            return e0 + (diag == n ? k : (k == 0 ? diag : (k <= diag ? k - 1 : k)));
+        };
+        const u64 dst = sell_at(slice, j, static_cast<u32>(k0));
+        sell_group<u32>(col, sell_col, dst, source);
+        if (vb == 1) sell_group<u8>(vals, sell_vals, dst, source);
+        else if (vb == 2) sell_group<u16>(vals, sell_vals, dst, source);
+        else if (vb == 8) sell_group<double>(vals, sell_vals, dst, source);
+        else if (vb == 16) sell_group<Zd>(vals, sell_vals, dst, source);
     }
 }
 

@@ -399,8 +399,6 @@ bool SectorOperator::build_sell(bool diag_first) {
     const int vb = packed_ ? 0 : (csr_.width == 1 || csr_.width == 2) ? csr_.width : (real_ ? 8 : 16);
     sell_col_.reset(std::max<std::uint64_t>(total, 1) * 4);
     if (vb) sell_vals_.reset(std::max<std::uint64_t>(total, 1) * static_cast<std::size_t>(vb));
-    QSA_HIP(hipMemsetAsync(sell_col_.get(), 0, sell_col_.bytes(), st));
-    if (vb) QSA_HIP(hipMemsetAsync(sell_vals_.get(), 0, sell_vals_.bytes(), st));
     dev::sell_fill(row_ptr_.get<std::uint64_t>(), col_.get<std::uint32_t>(), vals_.get(), vb, rows,
                    sell_ptr_.get<std::uint64_t>(), sell_col_.get<std::uint32_t>(), sell_vals_.get(),
                    sell_diag_first_ && same(), packed_, st);
