@@ -770,7 +770,7 @@ __global__ __launch_bounds__(256) void k_sell_lengths(const u64* row_ptr, i64 ro
 // the others keeping their order -- the k = 0 loads of a wavefront then read x[row] for 64
 // consecutive rows, one coalesced line instead of 64 gathers.
 // A lane gathers four entries of its row and writes the group whole, zeros past the row's end: a
-// wavefront's stores are 1 KB of consecutive words (20.7 million entries: 626 us an entry at a time
+// wavefront's stores are 1 KB of consecutive words (716,000 rows, 10.4 million entries: 626 us an entry at a time
 // into cleared memory, 182 so). What the slice holds past a row's last group is never read.
 template <class T, int V> struct alignas(sizeof(T) * V) Group {
     T v[V];
