@@ -200,7 +200,7 @@ __global__ __launch_bounds__(1024) void k_spmv(CsrView A, Ptrs<NV> v) {
 
 // Block-interleaved vectors: X[row * NV + k].
 template <int WIDTH, bool VREAL, bool REAL, bool LD, int L, int NV>
-__global__ __launch_bounds__(1024) void k_spmv_block(CsrView A, const void* X, void* Y) {
+__global__ __launch_bounds__(256) void k_spmv_block(CsrView A, const void* X, void* Y) {
     const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / L;
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(1024) void k_sell_block(CsrView A, const Two* X, Tw
 // momentum sector, 2 and 4 vectors: 103 and 143 us, one lane or two per row 113 and 150; 400,023 rows,
 // 4 vectors: 36 and 37), though not without a lattice symmetry (705,432 rows: 31 and 41, there 24 and 35).
 template <int WIDTH, bool LD, int NV, int ACC>
-__global__ __launch_bounds__(1024) void k_sell_block_rows(CsrView A, const double* X, double* Y) {
+__global__ __launch_bounds__(256) void k_sell_block_rows(CsrView A, const double* X, double* Y) {
     const Dict<LD> d = stage_dict<WIDTH, true, LD>(A);
     const i64 gid = row_block(A) * blockDim.x + threadIdx.x;
     const i64 row = gid / ACC;
@@ -604,21 +604,26 @@ template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& 
     });
 }
 
-/// Workgroup of the block kernels: 256 threads, or 1024 where a workgroup's copy of the dictionary is
-/// worth more than a few of its rows (2 KB).
-inline CsrView block_view(const CsrView& A) {
+/// The block kernels' workgroup and whether a dictionary of u16 ids is staged (one of u8 ids always is).
+/// A row's entries are looked up once for all its vectors, so the more vectors the less a copy in LDS
+/// saves. On the SELL layout complex vectors stage it, in workgroups of 1024 where it is over 2 KB
+/// (4 of 1.43 million rows: 399 us from global memory, 367 so); on the CSR layout 2 vectors do, in
+/// workgroups of 256 (32,065 rows: 6.2 and 5.4 us), while 8 in 1024 threads took 16.1 against 9.4 us
+/// on 9225 rows and 73 against 58 on 112,640.
+inline CsrView block_view(const CsrView& A, bool stage_u16, bool large) {
     CsrView B = A;
-    B.wg = dict_in_lds(A) && dict_lds_bytes(A) > 2048 ? 1024 : 256;
+    if (A.dict_n > 256 && !stage_u16) B.lds_dict = 0;
+    B.wg = large && dict_in_lds(B) && dict_lds_bytes(A) > 2048 ? 1024 : 256;
     return B;
 }
 
 template <int WIDTH, bool VREAL, bool REAL, int ACC>
 void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    const CsrView B = block_view(A);
     if constexpr (REAL) {
         if (nv <= 4) {
+            const CsrView B = block_view(A, false, false);
             const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(block_threads(B));
-            by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+            by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
                 constexpr bool LD = decltype(in_lds)::value;
                 const double* x = static_cast<const double*>(X);
                 double* y = static_cast<double*>(Y);
@@ -629,8 +634,9 @@ void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hip
         }
     }
     const int lanes = REAL ? nv / 2 : nv;   // 16 bytes each
+    const CsrView B = block_view(A, true, true);
     const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * static_cast<u64>(lanes))), block(block_threads(B));
-    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+    by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
 #define QSA_SELL_BLOCK(LR)                                                                                     \
     hipLaunchKernelGGL((k_sell_block<WIDTH, VREAL, REAL, LD, LR, ACC>), grid, block, lds, st, B,               \
@@ -688,9 +694,9 @@ template <int WIDTH, bool VREAL, bool REAL> void pick_lanes(const CsrView& A, co
 
 template <int WIDTH, bool VREAL, bool REAL, int L>
 void launch_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    const CsrView B = block_view(A);
+    const CsrView B = block_view(A, nv <= 2 && dict_lds_bytes(A) <= 16 * 1024, false);
     const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * L)), block(block_threads(B));
-    by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
+    by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
 #define QSA_SPMV_BLOCK(NV) hipLaunchKernelGGL((k_spmv_block<WIDTH, VREAL, REAL, LD, L, NV>), grid, block, lds, st, B, X, Y)
         switch (nv) {
@@ -770,7 +776,7 @@ __global__ __launch_bounds__(256) void k_sell_lengths(const u64* row_ptr, i64 ro
 // the others keeping their order -- the k = 0 loads of a wavefront then read x[row] for 64
 // consecutive rows, one coalesced line instead of 64 gathers.
 // A lane gathers four entries of its row and writes the group whole, zeros past the row's end: a
-// wavefront's stores are 1 KB of consecutive words (716,000 rows, 10.4 million entries: 626 us an entry at a time
+// wavefront's stores are 1 KB of consecutive words (716,000 rows, 20.7 million entries: 626 us an entry at a time
 // into cleared memory, 182 so). What the slice holds past a row's last group is never read.
 template <class T, int V> struct alignas(sizeof(T) * V) Group {
     T v[V];
