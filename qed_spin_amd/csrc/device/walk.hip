@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256) void k_csr_stage_dict(i64 rows_n, const u32* r
 
 // The CSR from the stage: columns, and value ids (width 1 / 2) or full values (width 0). An id is four
 // loads one after the other (value, fingerprint, the value kept there, its id), so a thread looks four
-// entries of its row up side by side; a probe past the first slot goes on by itself. 716,000 rows of 14.5
+// entries of its row up side by side; a probe past the first slot goes on by itself. 716,000 rows of 29
 // entries, u16 ids: one entry at a time 921 us, 450 so.
 template <int WIDTH, bool REAL>
 __global__ __launch_bounds__(256) void k_csr_compact(i64 rows_n, const u64* __restrict__ row_ptr,

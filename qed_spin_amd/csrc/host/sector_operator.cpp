@@ -436,8 +436,8 @@ void SectorOperator::autotune() {
     // mean row length gives and an apply does not depend on timing noise.
     // On the SELL-64 copy one lane owns a row, so no choice changes a sum.
     // The workgroup size first, at the middle depth, then the depth at the best size, two launches each:
-    // the two hardly depend on each other, and all pairs four times over were 3.2 ms of the 17 that a
-    // streamed block of 720,000 rows takes, against 1.0.
+    // the two hardly depend on each other, and all pairs four times over were 3.2 ms of the 16 that a
+    // streamed block of 716,000 rows takes, against 1.0.
     const std::vector<int> depths = sell() ? std::vector<int>{8, 4, 16} : std::vector<int>{4, 2, 8};
     const std::vector<int> groups = sell() ? std::vector<int>{256, 512, 1024} : std::vector<int>{512, 1024};
     auto launch = [&] {
