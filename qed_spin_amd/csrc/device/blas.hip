@@ -181,12 +181,10 @@ __global__ __launch_bounds__(kThreads) void k_finish(const double* partial, int 
     finish_pairs(partial, nb, out_kind, out);
 }
 
-// The DGKS gate of a Gram-Schmidt pass: beta = the norm it left; the pass is repeated when that is below
-// kappa of the norm it found.
-__global__ void k_cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta) {
-    const double a = sqrt(*after2);
-    *beta = a;
-    *again = a < kappa * sqrt(*before2) ? 1 : 0;
+// The DGKS gate of a Gram-Schmidt pass: it is repeated when the norm it left is below kappa of the norm
+// it found.
+__global__ void k_cgs_gate(const double* before2, const double* after2, double kappa, int* again) {
+    *again = sqrt(*after2) < kappa * sqrt(*before2) ? 1 : 0;
 }
 
 __global__ void k_add_pair(const Zd* a, const Zd* b, Zd* out) { *out = Zd{a->re + b->re, a->im + b->im}; }
@@ -335,68 +333,48 @@ __global__ __launch_bounds__(kThreads) void k_axpy_many(const Zd* coeffs, Cols V
     }
 }
 
-// axpy_many below kSplitRows rows: a block takes ROWS rows and its 512 / ROWS wavefront groups a share of
-// the columns each (column j to group j mod groups, four loads in flight per thread), the shares added
-// in group order. One thread per four rows and all columns, as above, is a chain of m / 4 rounds of
-// loads on n / 1024 blocks: 44 us for 9252 rows and 100 columns (so 7), 18 us for 112,632 complex rows and
-// 25 (so 9.6). From 2^19 rows on the threads alone keep enough loads in flight.
+// axpy_many below kSplitRows rows: a wavefront takes 64 rows, a thread one row and all columns, sixteen loads
+// in flight, added in column order as above (the same bits). One thread per four rows with four loads in
+// flight left the card idle: 44 us for 9252 rows and 100 columns. From 2^19 rows on the threads alone keep
+// enough loads in flight.
 constexpr std::size_t kSplitRows = std::size_t{1} << 19;
-constexpr int kSplitThreads = 512;
+constexpr int kSplitThreads = 64;
 
-template <bool C, int ROWS>
+template <bool C>
 __global__ __launch_bounds__(kSplitThreads) void k_axpy_many_split(const Zd* coeffs, Cols Vb, int m, void* w,
                                                                    std::size_t n, double* partial, int want_norm,
                                                                    double sign, const int* gate) {
     if (gate && !*gate) return;
-    constexpr int G = kSplitThreads / ROWS, U = 4;
+    constexpr int U = 16;
     __shared__ Zd sc[kManyCols];
-    __shared__ Zd share[G - 1][ROWS];
-    __shared__ double part[ROWS / 64];
     for (int j = threadIdx.x; j < m; j += kSplitThreads) sc[j] = Zd{sign * coeffs[j].re, sign * coeffs[j].im};
     __syncthreads();
-    const int row = static_cast<int>(threadIdx.x % ROWS), g = static_cast<int>(threadIdx.x / ROWS);
     double s0 = 0.0;
-    for (std::size_t base = blockIdx.x * static_cast<std::size_t>(ROWS); base < n;
-         base += static_cast<std::size_t>(gridDim.x) * ROWS) {
-        const std::size_t i = base + row;
-        const bool in = i < n;
-        Zd acc{0.0, 0.0};
-        if (in) {
-            int j = g;
-            for (; j + (U - 1) * G < m; j += U * G) {
-                Zd v[U];
+    for (std::size_t i = blockIdx.x * static_cast<std::size_t>(kSplitThreads) + threadIdx.x; i < n;
+         i += static_cast<std::size_t>(gridDim.x) * kSplitThreads) {
+        Zd acc = V<C>::load(w, i);
+        int j = 0;
+        for (; j + U <= m; j += U) {
+            Zd v[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = V<C>::load(Vb.at(j + u * G), i);
+            for (int u = 0; u < U; ++u) v[u] = V<C>::load(Vb.at(j + u), i);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if constexpr (C) acc = cadd(acc, cmul(sc[j + u * G], v[u]));
-                    else acc.re += sc[j + u * G].re * v[u].re;
-                }
-            }
-            for (; j < m; j += G) {
-                const Zd vj = V<C>::load(Vb.at(j), i);
-                acc = C ? cadd(acc, cmul(sc[j], vj)) : Zd{acc.re + sc[j].re * vj.re, 0.0};
+            for (int u = 0; u < U; ++u) {
+                if constexpr (C) acc = cadd(acc, cmul(sc[j + u], v[u]));
+                else acc.re += sc[j + u].re * v[u].re;
             }
         }
-        if (g > 0) share[g - 1][row] = acc;
-        __syncthreads();
-        if (g == 0 && in) {
-            acc = cadd(V<C>::load(w, i), acc);
-#pragma unroll
-            for (int q = 0; q < G - 1; ++q) acc = cadd(acc, share[q][row]);
-            V<C>::store(w, i, acc);
-            s0 += acc.re * acc.re + (C ? acc.im * acc.im : 0.0);
+        for (; j < m; ++j) {
+            const Zd vj = V<C>::load(Vb.at(j), i);
+            acc = C ? cadd(acc, cmul(sc[j], vj)) : Zd{acc.re + sc[j].re * vj.re, 0.0};
         }
-        __syncthreads();   // before the next rows' shares
+        V<C>::store(w, i, acc);
+        s0 += acc.re * acc.re + (C ? acc.im * acc.im : 0.0);
     }
-    if (want_norm) {   // the rows' threads are the first ROWS / 64 wavefronts
+    if (want_norm) {
         s0 = wave_sum(s0);
-        if (g == 0 && (threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s0;
-        __syncthreads();
         if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int q = 0; q < ROWS / 64; ++q) t += part[q];
-            partial[2 * blockIdx.x] = t;
+            partial[2 * blockIdx.x] = s0;
             partial[2 * blockIdx.x + 1] = 0.0;
         }
     }
@@ -470,8 +448,8 @@ void scale_by(bool c, const void* w, const double* norm, void* out, std::size_t 
     else hipLaunchKernelGGL(k_scale_by<false>, dim3(g), dim3(kThreads), 0, st, w, norm, out, n);
 }
 
-void cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta, hipStream_t st) {
-    hipLaunchKernelGGL(k_cgs_gate, dim3(1), dim3(1), 0, st, before2, after2, kappa, again, beta);
+void cgs_gate(const double* before2, const double* after2, double kappa, int* again, hipStream_t st) {
+    hipLaunchKernelGGL(k_cgs_gate, dim3(1), dim3(1), 0, st, before2, after2, kappa, again);
 }
 
 void add_pair(const Zd* a, const Zd* b, Zd* out, hipStream_t st) {
@@ -558,9 +536,9 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
                            double sign, const int* gate, bool root) {
     double* part = static_cast<double*>(scratch);
     const std::size_t elem = c ? sizeof(Zd) : sizeof(double);
-    const std::size_t rows = n <= 65536 ? 64 : 128;   // k_axpy_many_split's rows per block
-    const unsigned g = n >= kSplitRows ? grid_for(n)
-                                       : static_cast<unsigned>(std::min<std::size_t>(std::max<std::size_t>((n + rows - 1) / rows, 1), kMaxBlocks));
+    const unsigned g = n >= kSplitRows
+                           ? grid_for(n)
+                           : static_cast<unsigned>(std::min<std::size_t>(std::max<std::size_t>((n + 63) / 64, 1), kMaxBlocks));
     std::size_t done = 0;
     do {
         const int mc = static_cast<int>((m - done) < static_cast<std::size_t>(kManyCols) ? (m - done) : kManyCols);
@@ -575,12 +553,10 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
         if (n >= kSplitRows) {
             if (c) go(k_axpy_many<true>, kThreads);
             else go(k_axpy_many<false>, kThreads);
-        } else if (rows == 64) {
-            if (c) go(k_axpy_many_split<true, 64>, kSplitThreads);
-            else go(k_axpy_many_split<false, 64>, kSplitThreads);
+        } else if (c) {
+            go(k_axpy_many_split<true>, kSplitThreads);
         } else {
-            if (c) go(k_axpy_many_split<true, 128>, kSplitThreads);
-            else go(k_axpy_many_split<false, 128>, kSplitThreads);
+            go(k_axpy_many_split<false>, kSplitThreads);
         }
         if (want) hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), root ? 1 : 2,
                                      wnorm2, gate);

@@ -174,8 +174,8 @@ void axpy(bool cplx, Zd a, const void* x, void* y, std::size_t n, hipStream_t st
 void axpy(bool cplx, Coef a, const void* x, void* y, std::size_t n, hipStream_t st);
 /// out = w / *norm (device; out may be w).
 void scale_by(bool cplx, const void* w, const double* norm, void* out, std::size_t n, hipStream_t st);
-/// *beta = sqrt(*after2); *again = that is below kappa sqrt(*before2) (all on the device).
-void cgs_gate(const double* before2, const double* after2, double kappa, int* again, double* beta, hipStream_t st);
+/// *again = sqrt(*after2) is below kappa sqrt(*before2) (all on the device).
+void cgs_gate(const double* before2, const double* after2, double kappa, int* again, hipStream_t st);
 /// *out = *a + *b (device scalars).
 void add_pair(const Zd* a, const Zd* b, Zd* out, hipStream_t st);
 void scale(bool cplx, Zd a, void* x, std::size_t n, hipStream_t st);

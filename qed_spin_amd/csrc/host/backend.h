@@ -107,9 +107,10 @@ public:
         int* again = reinterpret_cast<int*>(result_.get<double>() + 6);
         dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c, norms, st());
         dev::axpy_many(kComplex, c, V, ld, m, w, n, scratch_.get(), norms + 1, st(), -1.0);
-        dev::cgs_gate(norms, norms + 1, kappa, again, beta, st());
+        dev::cgs_gate(norms, norms + 1, kappa, again, st());
         dev::dot_many(kComplex, V, ld, m, w, n, scratch_.get(), c, nullptr, st(), again);
-        dev::axpy_many(kComplex, c, V, ld, m, w, n, scratch_.get(), beta, st(), -1.0, again, true);
+        dev::axpy_many(kComplex, c, V, ld, m, w, n, scratch_.get(), nullptr, st(), -1.0, again);
+        dev::nrm2(kComplex, w, n, scratch_.get(), beta, st());
     }
     /// Two unconditional classical Gram-Schmidt passes of w against the m >= 1 columns of V: *tail =
     /// the last column's coefficient summed over both, *norm = ||w|| after.
