@@ -143,6 +143,7 @@ BlockEstimate estimate_lowest(const HipBackend<Scalar>& be, Matvec&& H, std::siz
     o.max_iter = std::min<std::size_t>(40, n);
     o.reorth = Reorth::None;
     o.keep_basis = false;
+    o.random_start = true;
     auto v0 = be.make_zero_vector(n);
     device_gaussian(v0.get(), n, kEstimateStartSeed);
     const auto run = lanczos_run(be, H, n, v0.get(), o);
@@ -289,11 +290,13 @@ private:
             double tail = 0.0;
             // the cycle's steps, their scalars on the device; read when all are enqueued, and cut at
             // the step that found an invariant subspace (what lies past it is not used)
+            detail::StepsInFlight flight(n_);
             for (std::size_t j = kept; j < m; ++j) {
                 H_(col(j), w_.get());
                 be_.cgs2(lowest_locked(), n_, locked_ + j + 1, w_.get(), n_, diag_.get<dev::Zd>() + j,
                          norm_.get<double>() + j);
                 be_.scale_by(w_.get(), norm_.get<double>() + j, col(j + 1), n_);
+                flight.step();
             }
             QSA_HIP(hipGetLastError());
             std::vector<dev::Zd> diag(m);

@@ -38,6 +38,7 @@ template <class Scalar> struct LanczosOptions {
     std::function<bool(const std::vector<double>&, const std::vector<double>&)> convergence_check;
     std::size_t convergence_check_interval = 0;
     double local_ortho_threshold = 1.49011611938476562e-08;
+    bool random_start = false;   ///< a start that lies in no small invariant subspace: no early look
 };
 
 /// Seconds of a run: apply_s, reorth_s and vector_s from events around the phases of every eighth of its
@@ -104,6 +105,35 @@ private:
     std::vector<hipEvent_t> ev_;
 };
 
+/// Bounds the steps that lie enqueued and not yet run: after a step, waits for the one `stride` to
+/// 2 stride before it (an event every stride steps, two in turn), so the device always has the next
+/// ones while a release on another thread, which waits for all that every engine stream holds
+/// (fence_engine_streams), and the short kernels of streams that share a hardware queue wait for a few
+/// steps and not for a run.
+class StepsInFlight {
+public:
+    explicit StepsInFlight(std::size_t n)
+        : stride_(n < (std::size_t{1} << 19) ? 4 : n < (std::size_t{1} << 22) ? 2 : 1) {}
+    ~StepsInFlight() {
+        for (auto& e : ev_)
+            if (e) (void)hipEventDestroy(e);
+    }
+    StepsInFlight(const StepsInFlight&) = delete;
+    StepsInFlight& operator=(const StepsInFlight&) = delete;
+    /// A step has been enqueued.
+    void step() {
+        if (++count_ % stride_) return;
+        const std::size_t s = count_ / stride_ % 2;
+        if (!ev_[s]) QSA_HIP(hipEventCreateWithFlags(&ev_[s], hipEventDisableTiming));
+        QSA_HIP(hipEventRecord(ev_[s], engine_stream()));
+        if (ev_[s ^ 1]) QSA_HIP(hipEventSynchronize(ev_[s ^ 1]));
+    }
+
+private:
+    std::size_t stride_, count_ = 0;
+    hipEvent_t ev_[2] = {nullptr, nullptr};
+};
+
 }  // namespace detail
 
 template <class Scalar, class Matvec>
@@ -126,63 +156,71 @@ LanczosResult<Scalar> lanczos_run(const HipBackend<Scalar>& be, Matvec&& matvec,
     const double n0 = be.nrm2(col(0), n);
     if (!(n0 > 0.0)) throw Error(kInvalid, "lanczos: initial vector has non-positive norm");
     be.scale(Scalar(1.0 / n0), col(0), n);
-    // alpha_j (complex), beta_{j+1}, the local overlap; the SELL first pass's partial sums
-    DeviceBuffer scalars((cap + 1) * (sizeof(dev::Zd) + sizeof(double)) + sizeof(dev::Zd)), sums;
-    dev::Zd* const alpha = scalars.get<dev::Zd>();
-    dev::Zd* const overlap = alpha + cap;
-    double* const beta = reinterpret_cast<double*>(overlap + 1);   // beta[j + 1]
+    // alpha_j (complex) and beta_{j+1} of each step, side by side for one copy; the local overlap; the SELL
+    // first pass's partial sums
+    struct Step {
+        dev::Zd alpha;
+        double beta, unused;
+    };
+    DeviceBuffer scalars((cap + 1) * sizeof(Step)), sums;
+    Step* const step = scalars.get<Step>();
+    dev::Zd* const overlap = &step[cap].alpha;
     const bool check = o.convergence_check && o.convergence_check_interval > 0;
-    // steps enqueued before the host looks: without a check enough to hide the look; with one a few,
-    // the smaller the costlier a step that turns out not to be needed
+    // steps enqueued before the host looks: without a check enough to hide the look (some 60 us), fewer at
+    // first where the run may break down early; with one a few, the smaller the costlier a step that
+    // turns out not to be needed
     const std::size_t look = check ? (n < (std::size_t{1} << 16) ? 8 : n < (std::size_t{1} << 19) ? 3 : 1)
                                    : (n < (std::size_t{1} << 19) ? 64 : 16);
+    const std::size_t first = check || o.random_start ? look : look / 4;
     detail::StepClock phases(cap);
-    std::vector<dev::Zd> ha(cap);
-    std::vector<double> hb(cap);
+    detail::StepsInFlight flight(n);
+    std::vector<Step> host(cap);
     std::size_t timed_steps = 0;
     bool done = false;
     for (std::size_t j0 = 0; j0 < cap && !done;) {
-        const std::size_t j1 = std::min(cap, j0 + look);
+        const std::size_t j1 = std::min(cap, j0 + (j0 == 0 ? first : look));
         for (std::size_t j = j0; j < j1; ++j) {
             const Scalar* v = col(j);
             const Scalar* prev = j > 0 ? col(j - 1) : nullptr;
+            const double* beta = j > 0 ? &step[j - 1].beta : nullptr;
+            dev::Zd* const alpha = &step[j].alpha;
+            double* const norm = &step[j].beta;
             Scalar* w = cgs ? work.get() : col(j + 1);
             phases.mark(j);
             // alpha_j = <v_j, H v_j - beta_j v_{j-1}>: in the apply's epilogue when the matvec offers it
             bool fused = false;
             if constexpr (HasFirstPass<std::decay_t<Matvec>, Scalar>::value)
-                fused = matvec.first_pass(v, prev, beta + j, w, alpha + j, sums);
+                fused = matvec.first_pass(v, prev, beta, w, alpha, sums);
             if (!fused) matvec(v, w);
             phases.mark(j);
             if (!fused) {
-                if (prev) be.axpy_dot(dev::minus(beta + j), prev, w, v, n, alpha + j);
-                else be.dot(v, w, n, alpha + j);
+                if (prev) be.axpy_dot(dev::minus(beta), prev, w, v, n, alpha);
+                else be.dot(v, w, n, alpha);
             }
-            const dev::Coef by_alpha = dev::minus(&alpha[j].re);
+            const dev::Coef by_alpha = dev::minus(&alpha->re);
             if (cgs) {
                 be.axpy(by_alpha, v, w, n);
                 phases.mark(j);
-                be.cgs_gated(block.get(), n, j + 1, w, n, kDgksKappa, beta + j + 1);
+                be.cgs_gated(block.get(), n, j + 1, w, n, kDgksKappa, norm);
             } else if (o.reorth == Reorth::LocalDGKS3 && j > 0) {
                 be.axpy_dot(by_alpha, v, w, v, n, overlap);
                 phases.mark(j);
-                be.axpy_nrm2(dev::minus_above(overlap, o.local_ortho_threshold), v, w, n, beta + j + 1);
+                be.axpy_nrm2(dev::minus_above(overlap, o.local_ortho_threshold), v, w, n, norm);
             } else {
-                be.axpy_nrm2(by_alpha, v, w, n, beta + j + 1);
+                be.axpy_nrm2(by_alpha, v, w, n, norm);
                 phases.mark(j);
             }
             phases.mark(j);
-            if (j + 1 < cap) be.scale_by(w, beta + j + 1, col(j + 1), n);
+            if (j + 1 < cap) be.scale_by(w, norm, col(j + 1), n);
+            flight.step();
         }
         QSA_HIP(hipGetLastError());
-        QSA_HIP(hipMemcpyAsync(ha.data() + j0, alpha + j0, (j1 - j0) * sizeof(dev::Zd), hipMemcpyDeviceToHost, engine_stream()));
-        QSA_HIP(hipMemcpyAsync(hb.data() + j0, beta + j0 + 1, (j1 - j0) * sizeof(double), hipMemcpyDeviceToHost, engine_stream()));
-        be.synchronize();
+        copy_to_host(host.data() + j0, step + j0, (j1 - j0) * sizeof(Step));
         timed_steps = j1;
         for (std::size_t j = j0; j < j1 && !done; ++j) {
-            R.alpha.push_back(ha[j].re);
-            R.beta.push_back(hb[j]);
-            if (hb[j] < o.breakdown_tol) done = true;
+            R.alpha.push_back(host[j].alpha.re);
+            R.beta.push_back(host[j].beta);
+            if (host[j].beta < o.breakdown_tol) done = true;
             else if (check && (j + 1) % o.convergence_check_interval == 0) done = o.convergence_check(R.alpha, R.beta);
         }
         j0 = j1;

@@ -222,6 +222,7 @@ Curves ftlm_block(const HipBackend<cplx>& be, Matvec&& H, std::size_t n, const F
     if (o.breakdown_tol > 0.0) lo.breakdown_tol = o.breakdown_tol;
     lo.reorth = Reorth::LocalDGKS3;
     lo.keep_basis = false;
+    lo.random_start = true;
     for (std::size_t s = 0; s < o.samples; ++s) {
         std::mt19937 gen = sample_engine(o.seed, s);
         const std::vector<cplx> h = gaussian_vector(n, gen);
