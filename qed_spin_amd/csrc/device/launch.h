@@ -112,7 +112,8 @@ struct CsrView {
     int xcd = 0;                   // contiguous row ranges per XCD (grid padded to a multiple of 8)
     int unroll = 1;                // single-vector SpMV: gathers issued 4 or 8 entries at a time (same sums)
     int dict_n = 0;                // dictionary entries (u8 / u16 ids)
-    int lds_dict = 1;              // stage the dictionary in LDS when it fits there
+    int lds_dict = 1;              // stage the dictionary in LDS when it fits there and pays
+    double mean_row = 0.0;         // entries per row
     int wg = 256;                  // single-vector SpMV: threads per workgroup (256, 512, 1024)
     // SELL-64 layout (sell_ptr non-null): col / vals hold the entries slice by slice in groups of
     // four, entry k of row 64 s + j at sell_ptr[s] + 256 (k / 4) + 4 j + k % 4 (slices padded to
@@ -141,6 +142,9 @@ void sell_scan(const u64* slice_words, i64 n_slices, u64* sell_ptr, void* temp, 
 void sell_fill(const u64* row_ptr, const u32* col, const void* vals, int value_bytes, i64 rows, const u64* sell_ptr,
                u32* sell_col, void* sell_vals, bool diag_first, bool packed, hipStream_t st);
 
+/// Whether single applies of A run in workgroups of one size whatever wg says (a staged dictionary
+/// above 16 KB).
+bool spmv_workgroup_fixed(const CsrView& A);
 /// Workgroups of sell_lanczos on A (its partial buffer holds two doubles per workgroup).
 unsigned sell_lanczos_blocks(const CsrView& A);
 /// The first pass of a Lanczos step in the SELL SpMV's epilogue: w = A v - *beta v_prev (v_prev null:

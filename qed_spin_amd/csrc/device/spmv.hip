@@ -37,8 +37,9 @@ extern __shared__ __align__(16) double lds_dict[];
 inline std::size_t dict_lds_bytes(const CsrView& A) {
     return A.width == 0 ? 0 : static_cast<std::size_t>(A.dict_n) * (A.values_real ? 8 : 16);
 }
-/// The largest staged dictionary: with 1024-thread workgroups two copies per compute unit, 32 waves.
-constexpr std::size_t kLdsDictMax = 64 * 1024;
+/// The largest staged dictionary: with the kernels' own arrays (256 bytes in k_sell_lanczos) within 64 KB
+/// a workgroup.
+constexpr std::size_t kLdsDictMax = 64 * 1024 - 512;
 inline bool dict_in_lds(const CsrView& A) { return A.lds_dict && dict_lds_bytes(A) <= kLdsDictMax; }
 
 template <int WIDTH, bool VREAL, bool LD> __device__ __forceinline__ Dict<LD> stage_dict(const CsrView& A) {
@@ -104,6 +105,25 @@ __device__ __forceinline__ i64 row_block(const CsrView& A) {
 inline unsigned block_threads(const CsrView& A) {
     if (dict_in_lds(A) && dict_lds_bytes(A) > 16 * 1024) return 1024;
     return (A.wg == 512 || A.wg == 1024) ? A.wg : 256;
+}
+
+/// A as a launch of `vectors` with `lanes` threads per row reads it: more than 256 values (u16 ids) are
+/// staged only where a workgroup looks up enough of them to pay for its copy: 7/10 of the dictionary's
+/// size below 2^18 rows (a few workgroups per compute unit, bound by the chain of loads); from there on,
+/// where the loads themselves bound it, its size, and 9/4 of it for one vector of a real operator (one
+/// load a lookup saved, not two). us an apply from global memory / staged, lookups over values: 32,066
+/// rows, 3637 real 7.7 / 6.7 at 0.8; 32,065, 3841 complex 10.3 / 7.6 at 0.8; 9252, 1890 real 4.3 / 3.9 at
+/// 0.7; 3432, 1730 real, four vectors 4.1 / 4.3 at 0.6; 112,720, 7683 real 23.0 / 23.7 at 0.4, four vectors
+/// 55 / 59; 5.17 million, 996 real 707 / 773 at 1.0, 719 / 727 at 2.1, four vectors 2170 / 2070 at 1.0; 1.43
+/// million, 804 real 169 / 162 at 2.4, 892 complex 222 / 208 at 1.1.
+inline CsrView staged(const CsrView& A, unsigned lanes, int vectors) {
+    CsrView B = A;
+    if (A.dict_n > 256 && dict_in_lds(A)) {
+        const double rows = std::min<double>(static_cast<double>(A.rows), block_threads(A) / lanes);
+        const double least = A.rows < (i64{1} << 18) ? 0.7 : A.values_real && vectors == 1 ? 2.25 : 1.0;
+        if (rows * A.mean_row < least * A.dict_n) B.lds_dict = 0;
+    }
+    return B;
 }
 
 inline unsigned grid_blocks(const CsrView& A, u64 threads) {
@@ -583,7 +603,8 @@ template <class F> void by_vectors(const VecSet& v, F&& go) {
     }
 }
 
-template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& A, const VecSet& v, hipStream_t st) {
+template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& V, const VecSet& v, hipStream_t st) {
+    const CsrView A = staged(V, 1, v.k);
     const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows))), block(block_threads(A));
     by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
@@ -609,11 +630,14 @@ template <int WIDTH, bool VREAL, bool REAL> void launch_sell_set(const CsrView& 
 /// saves. On the SELL layout complex vectors stage it, in workgroups of 1024 where it is over 2 KB
 /// (4 of 1.43 million rows: 399 us from global memory, 367 so); on the CSR layout 2 vectors do, in
 /// workgroups of 256 (32,065 rows: 6.2 and 5.4 us), while 8 in 1024 threads took 16.1 against 9.4 us
-/// on 9225 rows and 73 against 58 on 112,640.
-inline CsrView block_view(const CsrView& A, bool stage_u16, bool large) {
+/// on 9225 rows and 73 against 58 on 112,640. Of those that stage it, a launch with too few lookups for
+/// its copy does not (staged).
+inline CsrView block_view(const CsrView& A, bool stage_u16, bool large, unsigned lanes, int nv) {
     CsrView B = A;
     if (A.dict_n > 256 && !stage_u16) B.lds_dict = 0;
     B.wg = large && dict_in_lds(B) && dict_lds_bytes(A) > 2048 ? 1024 : 256;
+    B = staged(B, lanes, nv);
+    if (!dict_in_lds(B)) B.wg = 256;
     return B;
 }
 
@@ -621,7 +645,7 @@ template <int WIDTH, bool VREAL, bool REAL, int ACC>
 void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
     if constexpr (REAL) {
         if (nv <= 4) {
-            const CsrView B = block_view(A, false, false);
+            const CsrView B = block_view(A, false, false, ACC, nv);
             const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * ACC)), block(block_threads(B));
             by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
                 constexpr bool LD = decltype(in_lds)::value;
@@ -634,7 +658,7 @@ void launch_sell_block_acc(const CsrView& A, int nv, const void* X, void* Y, hip
         }
     }
     const int lanes = REAL ? nv / 2 : nv;   // 16 bytes each
-    const CsrView B = block_view(A, true, true);
+    const CsrView B = block_view(A, true, true, static_cast<unsigned>(lanes), nv);
     const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * static_cast<u64>(lanes))), block(block_threads(B));
     by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
@@ -666,7 +690,8 @@ void launch_sell_block(const CsrView& A, int nv, const void* X, void* Y, hipStre
     else launch_sell_block_acc<WIDTH, VREAL, REAL, 1>(A, nv, X, Y, st);
 }
 
-template <int WIDTH, bool VREAL, bool REAL, int L> void launch_set(const CsrView& A, const VecSet& v, hipStream_t st) {
+template <int WIDTH, bool VREAL, bool REAL, int L> void launch_set(const CsrView& V, const VecSet& v, hipStream_t st) {
+    const CsrView A = staged(V, L, v.k);
     const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows) * L)), block(block_threads(A));
     by_dict<WIDTH>(A, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
@@ -694,7 +719,7 @@ template <int WIDTH, bool VREAL, bool REAL> void pick_lanes(const CsrView& A, co
 
 template <int WIDTH, bool VREAL, bool REAL, int L>
 void launch_block(const CsrView& A, int nv, const void* X, void* Y, hipStream_t st) {
-    const CsrView B = block_view(A, nv <= 2 && dict_lds_bytes(A) <= 16 * 1024, false);
+    const CsrView B = block_view(A, nv <= 2 && dict_lds_bytes(A) <= 16 * 1024, false, L, nv);
     const dim3 grid(grid_blocks(B, static_cast<u64>(A.rows) * L)), block(block_threads(B));
     by_dict<WIDTH>(B, [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
@@ -870,11 +895,17 @@ void csr_spmv_block(const CsrView& A, bool real, int nv, const void* X, void* Y,
     dispatch<true>(A, A.values_real, real, nullptr, nv, X, Y, st);
 }
 
-unsigned sell_lanczos_blocks(const CsrView& A) { return grid_blocks(A, static_cast<u64>(A.rows)); }
+bool spmv_workgroup_fixed(const CsrView& A) {
+    const CsrView B = staged(A, A.sell_ptr ? 1u : static_cast<unsigned>(A.lanes), 1);
+    return dict_in_lds(B) && dict_lds_bytes(B) > 16 * 1024;
+}
 
-bool sell_lanczos(const CsrView& A, bool real, const void* v, const void* vprev, const double* beta, void* w,
+unsigned sell_lanczos_blocks(const CsrView& A) { return grid_blocks(staged(A, 1, 1), static_cast<u64>(A.rows)); }
+
+bool sell_lanczos(const CsrView& V, bool real, const void* v, const void* vprev, const double* beta, void* w,
                   double* partial, Zd* alpha, hipStream_t st) {
-    if (!A.sell_ptr || A.rows == 0 || (real && !A.values_real)) return false;
+    if (!V.sell_ptr || V.rows == 0 || (real && !V.values_real)) return false;
+    const CsrView A = staged(V, 1, 1);
     const unsigned nb = sell_lanczos_blocks(A);
     const dim3 grid(nb), block(block_threads(A));
     Ptrs<1> p;

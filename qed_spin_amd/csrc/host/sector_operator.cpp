@@ -462,7 +462,11 @@ void SectorOperator::autotune() {
     unroll_ = u1;
     wg_ = w1;
     launch();   // (the first one reads everything from HBM)
-    for (int WG : groups) consider(depths[0], WG);
+    for (int WG : groups) {
+        wg_ = WG;
+        if (dev::spmv_workgroup_fixed(csr_view(false, sell())) && best < 1e30f) continue;   // the same launch again
+        consider(depths[0], WG);
+    }
     const int group = w1;
     for (std::size_t i = 1; i < depths.size(); ++i) consider(depths[i], group);
     (void)hipEventDestroy(a);
@@ -496,6 +500,7 @@ dev::CsrView SectorOperator::csr_view(bool block, bool sell) const {
     A.unroll = unroll_;
     A.dict_n = static_cast<int>(csr_.dict);
     A.lds_dict = global_dict_ ? 0 : 1;
+    A.mean_row = A.rows > 0 ? static_cast<double>(csr_.nnz) / static_cast<double>(A.rows) : 0.0;
     A.wg = wg_;
     return A;
 }
