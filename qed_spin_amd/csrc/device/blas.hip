@@ -333,47 +333,57 @@ __global__ __launch_bounds__(kThreads) void k_axpy_many(const Zd* coeffs, Cols V
     }
 }
 
-// axpy_many below kSplitRows rows: a wavefront takes 64 rows, a thread one row and all columns, sixteen loads
-// in flight, added in column order as above (the same bits). One thread per four rows with four loads in
-// flight left the card idle: 44 us for 9252 rows and 100 columns. From 2^19 rows on the threads alone keep
-// enough loads in flight.
+// axpy_many below kSplitRows rows: a thread takes one row and all columns, sixteen loads in flight (then
+// four, then one), added in column order as above (the same bits). One thread per four rows with four
+// loads in flight left the card idle: 44 us for 9252 rows and 100 columns. Workgroups of one wavefront up
+// to 2^16 rows, so that these spread over the compute units, of four above, a row a thread up to
+// kSplitRows: at most 2048 of them (400,000 rows, a call with its 40 us of host work: 20 real columns 60
+// us and 100 complex 167; 61 and 163 by the kernel above, 69 and 176 with 1024 workgroups of one wavefront
+// at most and the last columns one at a time).
+// From 2^19 rows on the threads of the kernel above keep enough loads in flight.
 constexpr std::size_t kSplitRows = std::size_t{1} << 19;
-constexpr int kSplitThreads = 64;
+inline int split_threads(std::size_t n) { return n <= (std::size_t{1} << 16) ? 64 : 256; }
+
+template <bool C, int U>
+__device__ __forceinline__ void add_columns(const Cols& Vb, const Zd* sc, int m, std::size_t i, int& j, Zd& acc) {
+    for (; j + U <= m; j += U) {
+        Zd v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = V<C>::load(Vb.at(j + u), i);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if constexpr (C) acc = cadd(acc, cmul(sc[j + u], v[u]));
+            else acc.re += sc[j + u].re * v[u].re;
+        }
+    }
+}
 
 template <bool C>
-__global__ __launch_bounds__(kSplitThreads) void k_axpy_many_split(const Zd* coeffs, Cols Vb, int m, void* w,
-                                                                   std::size_t n, double* partial, int want_norm,
-                                                                   double sign, const int* gate) {
+__global__ __launch_bounds__(kThreads) void k_axpy_many_split(const Zd* coeffs, Cols Vb, int m, void* w,
+                                                              std::size_t n, double* partial, int want_norm,
+                                                              double sign, const int* gate) {
     if (gate && !*gate) return;
-    constexpr int U = 16;
     __shared__ Zd sc[kManyCols];
-    for (int j = threadIdx.x; j < m; j += kSplitThreads) sc[j] = Zd{sign * coeffs[j].re, sign * coeffs[j].im};
+    __shared__ double wave[kWaves];
+    for (int j = threadIdx.x; j < m; j += blockDim.x) sc[j] = Zd{sign * coeffs[j].re, sign * coeffs[j].im};
     __syncthreads();
     double s0 = 0.0;
-    for (std::size_t i = blockIdx.x * static_cast<std::size_t>(kSplitThreads) + threadIdx.x; i < n;
-         i += static_cast<std::size_t>(gridDim.x) * kSplitThreads) {
+    const std::size_t i = blockIdx.x * static_cast<std::size_t>(blockDim.x) + threadIdx.x;
+    if (i < n) {
         Zd acc = V<C>::load(w, i);
         int j = 0;
-        for (; j + U <= m; j += U) {
-            Zd v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = V<C>::load(Vb.at(j + u), i);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if constexpr (C) acc = cadd(acc, cmul(sc[j + u], v[u]));
-                else acc.re += sc[j + u].re * v[u].re;
-            }
-        }
-        for (; j < m; ++j) {
-            const Zd vj = V<C>::load(Vb.at(j), i);
-            acc = C ? cadd(acc, cmul(sc[j], vj)) : Zd{acc.re + sc[j].re * vj.re, 0.0};
-        }
+        add_columns<C, 16>(Vb, sc, m, i, j, acc);
+        add_columns<C, 4>(Vb, sc, m, i, j, acc);
+        add_columns<C, 1>(Vb, sc, m, i, j, acc);
         V<C>::store(w, i, acc);
-        s0 += acc.re * acc.re + (C ? acc.im * acc.im : 0.0);
+        s0 = acc.re * acc.re + (C ? acc.im * acc.im : 0.0);
     }
-    if (want_norm) {
+    if (want_norm) {   // the wavefronts' sums in order
         s0 = wave_sum(s0);
+        if ((threadIdx.x & 63u) == 0) wave[threadIdx.x >> 6] = s0;
+        __syncthreads();
         if (threadIdx.x == 0) {
+            for (unsigned q = 1; q < blockDim.x / 64; ++q) s0 += wave[q];
             partial[2 * blockIdx.x] = s0;
             partial[2 * blockIdx.x + 1] = 0.0;
         }
@@ -408,7 +418,7 @@ __global__ __launch_bounds__(256) void k_block_rotate(const void* Vb, std::size_
 
 std::size_t blas_scratch_bytes(std::size_t max_cols) {
     (void)max_cols;
-    const std::size_t red = 2 * kMaxBlocks * sizeof(double);
+    const std::size_t red = 2 * std::max<std::size_t>(kMaxBlocks, kSplitRows / 256) * sizeof(double);
     const std::size_t many = static_cast<std::size_t>(kMaxBlocks) * (kManyCols + 1) * 2 * sizeof(double);
     return red > many ? red : many;
 }
@@ -536,9 +546,9 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
                            double sign, const int* gate, bool root) {
     double* part = static_cast<double*>(scratch);
     const std::size_t elem = c ? sizeof(Zd) : sizeof(double);
-    const unsigned g = n >= kSplitRows
-                           ? grid_for(n)
-                           : static_cast<unsigned>(std::min<std::size_t>(std::max<std::size_t>((n + 63) / 64, 1), kMaxBlocks));
+    const bool split = n < kSplitRows;
+    const std::size_t threads = split ? static_cast<std::size_t>(split_threads(n)) : kThreads;
+    const unsigned g = split ? static_cast<unsigned>(std::max<std::size_t>((n + threads - 1) / threads, 1)) : grid_for(n);
     std::size_t done = 0;
     do {
         const int mc = static_cast<int>((m - done) < static_cast<std::size_t>(kManyCols) ? (m - done) : kManyCols);
@@ -546,18 +556,14 @@ static void axpy_many_cols(bool c, const Zd* coeffs, const void* V, std::size_t 
         const int want = (last && wnorm2) ? 1 : 0;
         const Cols Vc{table ? nullptr : static_cast<const char*>(V) + done * ld * elem, ld * elem,
                       table ? table + done : nullptr};
-        auto go = [&](auto kernel, int threads) {
+        auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(g), dim3(static_cast<unsigned>(threads)), 0, st, coeffs + done, Vc, mc, w, n, part,
                                want, sign, gate);
         };
-        if (n >= kSplitRows) {
-            if (c) go(k_axpy_many<true>, kThreads);
-            else go(k_axpy_many<false>, kThreads);
-        } else if (c) {
-            go(k_axpy_many_split<true>, kSplitThreads);
-        } else {
-            go(k_axpy_many_split<false>, kSplitThreads);
-        }
+        if (split && c) go(k_axpy_many_split<true>);
+        else if (split) go(k_axpy_many_split<false>);
+        else if (c) go(k_axpy_many<true>);
+        else go(k_axpy_many<false>);
         if (want) hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, static_cast<int>(g), root ? 1 : 2,
                                      wnorm2, gate);
         done += static_cast<std::size_t>(mc);
