@@ -115,6 +115,25 @@ __device__ __forceinline__ BlockDict stage_block_dict(const BatchView& B, u32 bl
 
 extern __shared__ __align__(16) Zd batch_dict[];
 
+// Entry e of one block's own CSR: its column, its dictionary id (width 1 / 2 / 3), its value.
+__device__ __forceinline__ u32 entry_column(const CsrView& A, u64 e) {
+    const u32 w = A.col[e];
+    return A.width == 3 ? (w & 0xFFFFFFu) : w;
+}
+__device__ __forceinline__ u32 entry_id(const CsrView& A, u64 e) {
+    if (A.width == 3) return A.col[e] >> 24;
+    return A.width == 1 ? static_cast<u32>(static_cast<const u8*>(A.vals)[e])
+                        : static_cast<u32>(static_cast<const u16*>(A.vals)[e]);
+}
+__device__ __forceinline__ Zd csr_value(const CsrView& A, u64 e) {
+    if (A.width != 0) {
+        const u32 id = entry_id(A, e);
+        return Zd{A.dict_re[id], A.values_real ? 0.0 : A.dict_im[id]};
+    }
+    if (A.values_real) return Zd{static_cast<const double*>(A.vals)[e], 0.0};
+    return static_cast<const Zd*>(A.vals)[e];
+}
+
 // ar + i ai += v x, by fused multiply-adds.
 __device__ __forceinline__ void zfma(Zd v, Zd x, double& ar, double& ai) {
     ar = __builtin_fma(v.re, x.re, ar);
@@ -281,7 +300,13 @@ __global__ __launch_bounds__(kGroupThreads) void k_batch_spmv_group(BatchView B,
 // took 0.906 ms; with the dictionary in LDS and four entries in flight 0.785 ms, in level order
 // (L2 misses 26.7M -> 10.7M lines) 0.769 ms: latency, every row being a chain of loads for a couple of
 // entries per lane. So: 0.626 ms.
-template <bool LD>
+//
+// Where an entry's value comes from: kOneFull in full; kOneLds ids, every block's dictionary staged;
+// kOneMixed ids, a dictionary above kBatchDictMax values read from global memory and the others staged,
+// so that one large dictionary costs the other blocks nothing and no block 20 bytes an entry for 6.
+enum OneValues { kOneFull, kOneLds, kOneMixed };
+
+template <OneValues MODE>
 __global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, const Zd* Vprev,
                                                                    const Zd* Vcur, Zd* W, const double* beta,
                                                                    double* partial, const double* sprev,
@@ -296,7 +321,13 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, 
     const bool on = r < t.row_end && pair_live(B, t.block, 0);
     const u32 n = on ? S.len[r] : 0u;
     const u64 at = S.ptr[static_cast<u64>(w.tile) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] + (threadIdx.x & 63u) * 4u;
-    if constexpr (LD) {
+    bool lds = MODE == kOneLds;   // the same for the whole workgroup
+    u32 d0 = 0;
+    if constexpr (MODE == kOneMixed) {
+        d0 = B.dict_begin[t.block];
+        lds = B.dict_begin[t.block + 1] - d0 <= static_cast<u32>(kBatchDictMax);
+    }
+    if (lds) {
         (void)stage_block_dict(B, t.block, batch_dict);
         __syncthreads();
     }
@@ -309,7 +340,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, 
         for (int g = 0; g < 2; ++g) {
             const u64 e = at + static_cast<u64>(k / 4 + static_cast<u32>(g)) * 256;
             c[g] = *reinterpret_cast<const u32x4*>(S.col + e);
-            if constexpr (LD) {
+            if constexpr (MODE != kOneFull) {
                 id[g] = *reinterpret_cast<const u16x4*>(S.vid + e);
             } else {
 #pragma unroll
@@ -318,9 +349,22 @@ __global__ __launch_bounds__(kThreads) void k_batch_spmv_one_fused(BatchView B, 
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) x[u] = Vcur[c[u / 4][u % 4]];
+        if constexpr (MODE == kOneMixed) {
+            if (!lds) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {   // (past the row's end: id 0, counted as zero)
+                    const u32 i = d0 + id[u / 4][u % 4];
+                    const Zd q{B.dict_re[i], B.dict_im[i]};
+                    v[u] = k + static_cast<u32>(u) < n ? q : Zd{0.0, 0.0};
+                }
+            }
+        }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            if constexpr (LD) v[u] = batch_dict[id[u / 4][u % 4]];
+            if constexpr (MODE == kOneLds) v[u] = batch_dict[id[u / 4][u % 4]];
+            if constexpr (MODE == kOneMixed) {
+                if (lds) v[u] = batch_dict[id[u / 4][u % 4]];
+            }
             if (u < 4) zfma(v[u], x[u], ar, ai);
             else zfma(v[u], x[u], br, bi);
         }
@@ -379,14 +423,17 @@ __global__ __launch_bounds__(kThreads) void k_one_lengths(BatchView B, u32* len,
         slice[static_cast<u64>(blockIdx.x) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] = static_cast<u64>((n + 7u) & ~7u) * 64;
 }
 
-__global__ __launch_bounds__(kThreads) void k_one_fill(BatchView B, const u64* slice, u32* col, u16* vid, Zd* val) {
-    const Tile t = B.tiles[blockIdx.x];
-    const u64 r = t.row_begin + threadIdx.x;
-    if (r >= t.row_end) return;
-    const u64 from = B.row_ptr[r];
-    const u32 n = static_cast<u32>(B.row_ptr[r + 1] - from), end = (n + 7u) & ~7u;
-    const u64 at = slice[static_cast<u64>(blockIdx.x) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] + (threadIdx.x & 63u) * 4u;
-    const u32 d0 = vid ? B.dict_begin[t.block] : 0u, zero = vid ? B.dict_begin[t.block + 1] - d0 : 0u;
+// One block's entries into the slices, from its own CSR: its tile blockIdx.x (the packed tile tile0 +
+// blockIdx.x), packed row p holding row order[p] (null: p) and column c at place[c]; ids count from the
+// block's first.
+__global__ __launch_bounds__(kThreads) void k_one_fill(CsrView A, u64 row0, u32 tile0, const u32* order, const u32* place,
+                                                       const u64* slice, u32* col, u16* vid, Zd* val, u32 zero) {
+    const u64 q = blockIdx.x * static_cast<u64>(kBatchTileRows) + threadIdx.x;
+    if (q >= static_cast<u64>(A.rows)) return;
+    const u64 p = row0 + q, r = order ? order[p] - row0 : q;
+    const u64 from = A.row_ptr[r];
+    const u32 n = static_cast<u32>(A.row_ptr[r + 1] - from), end = (n + 7u) & ~7u;
+    const u64 at = slice[static_cast<u64>(tile0 + blockIdx.x) * (kBatchTileRows / 64) + (threadIdx.x >> 6)] + (threadIdx.x & 63u) * 4u;
     for (u32 k = 0; k < end; k += 4) {
         u32x4 c;
         u16x4 id;
@@ -394,9 +441,11 @@ __global__ __launch_bounds__(kThreads) void k_one_fill(BatchView B, const u64* s
 #pragma unroll
         for (u32 u = 0; u < 4; ++u) {
             const bool in = k + u < n;
-            c[u] = in ? B.col[from + k + u] : static_cast<u32>(r);
-            if (vid) id[u] = static_cast<u16>(in ? B.vid[from + k + u] - d0 : zero);
-            else v[u] = in ? entry_value(B, from + k + u) : Zd{0.0, 0.0};
+            const u64 e = from + (in ? k + u : 0u);
+            const u64 to = row0 + entry_column(A, e);
+            c[u] = in ? (place ? place[to] : static_cast<u32>(to)) : static_cast<u32>(p);
+            if (vid) id[u] = static_cast<u16>(in ? entry_id(A, e) : zero);
+            else v[u] = in ? csr_value(A, e) : Zd{0.0, 0.0};
         }
         const u64 e = at + static_cast<u64>(k / 4) * 256;
         *reinterpret_cast<u32x4*>(col + e) = c;
@@ -672,26 +721,8 @@ __global__ void k_order_invert(const u32* order, u64 n, u32* place) {
 
 __global__ void k_order_lengths(const u64* row_ptr, const u32* order, u64 n, u32* len) {
     for (u64 i = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * blockDim.x) {
-        const u64 r = order ? order[i] : i;
+        const u64 r = order[i];
         len[i] = static_cast<u32>(row_ptr[r + 1] - row_ptr[r]);
-    }
-}
-
-// Row i of the new matrix is row order[i] of the old one (null: i), its entries in the same order, their
-// columns moved to place[column] (null: kept); eight lanes per row.
-__global__ __launch_bounds__(kThreads) void k_order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val,
-                                                         const u32* order, const u32* place, u64 n, const u64* new_ptr,
-                                                         u32* new_col, u16* new_vid, Zd* new_val) {
-    const u64 stride = static_cast<u64>(gridDim.x) * (kThreads / 8);
-    for (u64 i = blockIdx.x * static_cast<u64>(kThreads / 8) + (threadIdx.x >> 3); i < n; i += stride) {
-        const u64 r = order ? order[i] : i;
-        const u64 from = row_ptr[r], m = row_ptr[r + 1] - from, to = new_ptr[i];
-        for (u64 k = threadIdx.x & 7u; k < m; k += 8) {
-            const u32 c = col[from + k];
-            new_col[to + k] = place ? place[c] : c;
-            if (vid) new_vid[to + k] = vid[from + k];
-            else new_val[to + k] = val[from + k];
-        }
     }
 }
 
@@ -738,42 +769,40 @@ __global__ void k_csr_to_dense(CsrView A, Zd* out) {
     }
 }
 
-// Pack one block's CSR into the global one: rows shifted by row_off, columns by col_off, values
-// expanded from the dictionary (width 1 / 2 / 3) or copied (width 0; double when real) -- or, with a
-// packed dictionary, the ids offset by the block's first entry in it.
-__global__ void k_pack_csr(CsrView A, u64 row_off, u64 col_off, u64 nnz_off, u64* row_ptr, u32* col, Zd* val,
-                           u16* vid, u32 dict_off) {
-    const u64 r = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x;
-    if (r > static_cast<u64>(A.rows)) return;
-    row_ptr[row_off + r] = nnz_off + A.row_ptr[r];
-    if (r == static_cast<u64>(A.rows)) return;
-    for (u64 e = A.row_ptr[r]; e < A.row_ptr[r + 1]; ++e) {
-        const u32 w = A.col[e];
-        col[nnz_off + e] = static_cast<u32>(col_off + (A.width == 3 ? (w & 0xFFFFFFu) : w));
-        if (vid) {   // the caller checked that the block has ids and the offset ids fit 16 bits
-            const u32 id = A.width == 3 ? (w >> 24)
-                           : A.width == 1 ? static_cast<u32>(static_cast<const u8*>(A.vals)[e])
-                                          : static_cast<u32>(static_cast<const u16*>(A.vals)[e]);
-            vid[nnz_off + e] = static_cast<u16>(dict_off + id);
-            continue;
+// One block's CSR into the packed one, eight lanes per row, each row's entries in their order. Rows: at
+// row_off + r and nnz_off, the row pointers written here, or (row_place set) at row_place[row_off + r],
+// whose first entry row_ptr already holds. Columns (col null: the row pointers alone): col_off + c, or
+// col_place[col_off + c]. Values: in full into val, or the ids offset by the block's first entry in the
+// packed dictionary into vid (the caller checked that the block has ids and the offset ids fit 16 bits),
+// or neither.
+__global__ __launch_bounds__(kThreads) void k_pack_csr(CsrView A, u64 row_off, const u32* row_place, u64 col_off,
+                                                       const u32* col_place, u64 nnz_off, u64* row_ptr, u32* col, Zd* val,
+                                                       u16* vid, u32 dict_off) {
+    const u64 rows = static_cast<u64>(A.rows), stride = static_cast<u64>(gridDim.x) * (kThreads / 8);
+    const u32 lane = threadIdx.x & 7u;
+    for (u64 r = blockIdx.x * static_cast<u64>(kThreads / 8) + (threadIdx.x >> 3); r < rows; r += stride) {
+        const u64 from = A.row_ptr[r], end = A.row_ptr[r + 1];
+        u64 to = nnz_off + from;
+        if (row_place) {
+            to = row_ptr[row_place[row_off + r]];
+        } else if (lane == 0) {
+            row_ptr[row_off + r] = to;
+            if (r + 1 == rows) row_ptr[row_off + rows] = nnz_off + end;
         }
-        Zd v;
-        if (A.width == 3) {
-            const u32 id = w >> 24;
-            v = Zd{A.dict_re[id], A.values_real ? 0.0 : A.dict_im[id]};
-        } else if (A.width == 1) {
-            const u32 id = static_cast<const u8*>(A.vals)[e];
-            v = Zd{A.dict_re[id], A.values_real ? 0.0 : A.dict_im[id]};
-        } else if (A.width == 2) {
-            const u32 id = static_cast<const u16*>(A.vals)[e];
-            v = Zd{A.dict_re[id], A.values_real ? 0.0 : A.dict_im[id]};
-        } else if (A.values_real) {
-            v = Zd{static_cast<const double*>(A.vals)[e], 0.0};
-        } else {
-            v = static_cast<const Zd*>(A.vals)[e];
+        if (!col) continue;
+        for (u64 k = lane; k < end - from; k += 8) {
+            const u64 c = col_off + entry_column(A, from + k);
+            col[to + k] = col_place ? col_place[c] : static_cast<u32>(c);
+            if (vid) vid[to + k] = static_cast<u16>(dict_off + entry_id(A, from + k));
+            else if (val) val[to + k] = csr_value(A, from + k);
         }
-        val[nnz_off + e] = v;
     }
+}
+
+// The row lengths of one block at its rows' places.
+__global__ void k_place_lengths(CsrView A, u64 row_off, const u32* place, u32* len) {
+    const u64 r = blockIdx.x * static_cast<u64>(blockDim.x) + threadIdx.x;
+    if (r < static_cast<u64>(A.rows)) len[place[row_off + r]] = static_cast<u32>(A.row_ptr[r + 1] - A.row_ptr[r]);
 }
 
 // Whether block b takes a Gram-Schmidt pass: it is fully reorthogonalised and, with per-pair flags,
@@ -967,15 +996,10 @@ unsigned grid_for(u64 n) {
 
 }  // namespace
 
+namespace {
+/// Whether every block's dictionary fits the SpMV's LDS.
 bool batch_dict_in_lds(const BatchView& B) {
     return B.dict_begin && B.dict_max > 0 && B.dict_max <= static_cast<u32>(kBatchDictMax);
-}
-
-namespace {
-/// f(whether the blocks' dictionaries fit LDS one at a time, the dynamic LDS bytes).
-template <class F> void by_block_dict(const BatchView& B, bool ids, F&& f) {
-    if (ids && batch_dict_in_lds(B)) f(std::true_type{}, (static_cast<std::size_t>(B.dict_max) + 1) * sizeof(Zd));
-    else f(std::false_type{}, std::size_t{0});
 }
 
 template <bool FUSED>
@@ -983,7 +1007,7 @@ void launch_group(const BatchView& B, const Zd* Vprev, const Zd* X, Zd* Y, const
                   const double* sprev, const double* scur, hipStream_t st) {
     const int chunks = batch_chunks(B.R);
     const dim3 grid(B.sched ? B.n_sched : B.n_tiles * static_cast<u32>(chunks)), block(kGroupThreads);
-    by_block_dict(B, B.vid != nullptr, [&](auto in_lds, std::size_t lds) {
+    auto go = [&](auto in_lds, std::size_t lds) {
         constexpr bool LD = decltype(in_lds)::value;
 #define QSA_GROUP(RP)                                                                                                  \
     hipLaunchKernelGGL((k_batch_spmv_group<RP, LD, FUSED>), grid, block, lds, st, B, chunks, Vprev, X, Y, beta, partial, \
@@ -992,7 +1016,9 @@ void launch_group(const BatchView& B, const Zd* Vprev, const Zd* X, Zd* Y, const
         else if (B.R <= 4) QSA_GROUP(4);
         else QSA_GROUP(8);
 #undef QSA_GROUP
-    });
+    };
+    if (B.vid && batch_dict_in_lds(B)) go(std::true_type{}, (static_cast<std::size_t>(B.dict_max) + 1) * sizeof(Zd));
+    else go(std::false_type{}, std::size_t{0});
 }
 }  // namespace
 
@@ -1003,24 +1029,33 @@ void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st) {
 void batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
                       hipStream_t st, const double* sprev, const double* scur) {
     if (!B.n_tiles) return;
-    if (B.R > 1) {
+    if (!B.one.ptr) {
         launch_group<true>(B, Vprev, Vcur, W, beta, partial, sprev, scur, st);
         return;
     }
     const dim3 grid(B.sched ? B.n_sched : B.n_tiles), block(kThreads);
-    by_block_dict(B, B.one.vid != nullptr, [&](auto in_lds, std::size_t lds) {
-        constexpr bool LD = decltype(in_lds)::value;
-        hipLaunchKernelGGL((k_batch_spmv_one_fused<LD>), grid, block, lds, st, B, Vprev, Vcur, W, beta, partial,
-                           sprev, scur);
-    });
+    const std::size_t lds = (std::min<std::size_t>(B.dict_max, kBatchDictMax) + 1) * sizeof(Zd);
+#define QSA_ONE(MODE, LDS)                                                                                            \
+    hipLaunchKernelGGL((k_batch_spmv_one_fused<MODE>), grid, block, LDS, st, B, Vprev, Vcur, W, beta, partial, sprev, \
+                       scur)
+    if (!B.one.vid) QSA_ONE(kOneFull, 0);
+    else if (batch_dict_in_lds(B)) QSA_ONE(kOneLds, lds);
+    else QSA_ONE(kOneMixed, lds);
+#undef QSA_ONE
 }
 
 void one_lengths(const BatchView& B, u32* len, u64* slice, hipStream_t st) {
     if (B.n_tiles) hipLaunchKernelGGL(k_one_lengths, dim3(B.n_tiles), dim3(kThreads), 0, st, B, len, slice);
 }
 
-void one_fill(const BatchView& B, const u64* slice, u32* col, u16* vid, Zd* val, hipStream_t st) {
-    if (B.n_tiles) hipLaunchKernelGGL(k_one_fill, dim3(B.n_tiles), dim3(kThreads), 0, st, B, slice, col, vid, val);
+void one_fill(const CsrView& A, u64 row0, u32 tile0, const u32* order, const u32* place, const u64* slice, u32* col,
+              u16* vid, Zd* val, hipStream_t st) {
+    static_assert(kThreads == kBatchTileRows, "a thread per row of a tile");
+    if (!A.rows) return;
+    // the zero after a staged dictionary's last value; a dictionary in global memory counts the padding out
+    const u32 zero = A.dict_n <= kBatchDictMax ? static_cast<u32>(A.dict_n) : 0u;
+    hipLaunchKernelGGL(k_one_fill, dim3(static_cast<unsigned>((static_cast<u64>(A.rows) + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, st, A, row0, tile0, order, place, slice, col, vid, val, zero);
 }
 
 void batch_vec(const BatchView& B, int mode, const Zd* Vcur, Zd* W, const double* coef, const Zd* zcoef,
@@ -1085,13 +1120,6 @@ void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hip
     if (rows) hipLaunchKernelGGL(k_order_lengths, dim3(grid_for(rows)), dim3(256), 0, st, row_ptr, order, rows, len);
 }
 
-void order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val, const u32* order, const u32* place,
-                u64 rows, const u64* new_ptr, u32* new_col, u16* new_vid, Zd* new_val, hipStream_t st) {
-    if (rows)
-        hipLaunchKernelGGL(k_order_rows, dim3(grid_for(rows * 8)), dim3(kThreads), 0, st, row_ptr, col, vid, val, order,
-                           place, rows, new_ptr, new_col, new_vid, new_val);
-}
-
 void csr_to_dense(const CsrView& A, Zd* out, hipStream_t st) {
     const u64 n = static_cast<u64>(A.rows);
     if (!n) return;
@@ -1151,11 +1179,17 @@ void batch_fill_zero(Zd* x, u64 n, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_zd, dim3(grid_for(n)), dim3(256), 0, st, x, n);
 }
 
-void pack_csr(const CsrView& A, u64 row_off, u64 col_off, u64 nnz_off, u64* row_ptr, u32* col, Zd* val, u16* vid,
-              u32 dict_off, hipStream_t st) {
-    const u64 n = static_cast<u64>(A.rows) + 1;
-    hipLaunchKernelGGL(k_pack_csr, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, A, row_off,
-                       col_off, nnz_off, row_ptr, col, val, vid, dict_off);
+void place_lengths(const CsrView& A, u64 row_off, const u32* place, u32* len, hipStream_t st) {
+    if (!A.rows) return;
+    hipLaunchKernelGGL(k_place_lengths, dim3(static_cast<unsigned>((static_cast<u64>(A.rows) + 255) / 256)), dim3(256), 0, st,
+                       A, row_off, place, len);
+}
+
+void pack_csr(const CsrView& A, u64 row_off, const u32* row_place, u64 col_off, const u32* col_place, u64 nnz_off,
+              u64* row_ptr, u32* col, Zd* val, u16* vid, u32 dict_off, hipStream_t st) {
+    if (!A.rows) return;
+    hipLaunchKernelGGL(k_pack_csr, dim3(grid_for(static_cast<u64>(A.rows) * 8)), dim3(kThreads), 0, st, A, row_off, row_place,
+                       col_off, col_place, nnz_off, row_ptr, col, val, vid, dict_off);
 }
 
 }  // namespace qsa::dev

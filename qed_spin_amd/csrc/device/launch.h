@@ -274,12 +274,13 @@ constexpr int kBatchMaxR = 64;
 /// Work items of a tile in the SpMV: one up to eight vectors, above that one per run of eight.
 constexpr int batch_chunks(int R) { return R > 8 ? (R + 7) / 8 : 1; }
 void batch_spmv(const BatchView& B, const Zd* X, Zd* Y, hipStream_t st);
-/// Whether a block's dictionary fits the SpMV's LDS (else the R = 1 layout holds full values).
-bool batch_dict_in_lds(const BatchView& B);
 /// The R = 1 layout (OneView) of a packed matrix: the rows' lengths and the slices' entries
-/// (kBatchTileRows / 64 per tile; sell_scan gives their offsets), then the entries (vid or val null).
+/// (kBatchTileRows / 64 per tile; sell_scan gives their offsets), then one block's entries at a time from
+/// its own CSR, rows and columns in the engine's order (order and place null: the states'); vid or val
+/// null, and ids only when the block has them.
 void one_lengths(const BatchView& B, u32* len, u64* slice, hipStream_t st);
-void one_fill(const BatchView& B, const u64* slice, u32* col, u16* vid, Zd* val, hipStream_t st);
+void one_fill(const CsrView& A, u64 row0, u32 tile0, const u32* order, const u32* place, const u64* slice, u32* col,
+              u16* vid, Zd* val, hipStream_t st);
 /// W = H V_cur - beta V_prev with the partials of <V_cur, W>. sprev / scur: per-pair factors of the
 /// stored vectors (V = stored times factor), or null (1).
 void batch_spmv_fused(const BatchView& B, const Zd* Vprev, const Zd* Vcur, Zd* W, const double* beta, double* partial,
@@ -313,11 +314,8 @@ std::size_t level_sort_temp_bytes(u64 rows);
 /// key, key2, row: rows words each.
 void level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
                  std::size_t temp_bytes, hipStream_t st);
-/// A packed matrix with its rows in `order` (null: kept) and its columns at `place` (null: kept), each
-/// row's entries in their order: the new rows' lengths, then (new_ptr from their scan) the entries.
+/// len[i] = the length of the row that `order` puts at place i.
 void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hipStream_t st);
-void order_rows(const u64* row_ptr, const u32* col, const u16* vid, const Zd* val, const u32* order, const u32* place,
-                u64 rows, const u64* new_ptr, u32* new_col, u16* new_vid, Zd* new_val, hipStream_t st);
 void batch_fill_zero(Zd* x, u64 n, hipStream_t st);
 
 // ---- sample.hip ------------------------------------------------------------------------------
@@ -327,10 +325,15 @@ void batch_fill_zero(Zd* x, u64 n, hipStream_t st);
 /// `vectors` workgroups. Not normalised.
 void sample_gauss(Zd* V, int R, const u64* row_begin, const u64* dims, const u32* seeds, u32 vectors,
                   const u32* place, hipStream_t st);
-/// One block's CSR into the packed one: rows and columns offset, values in full into val, or (vid
-/// set, the block's CSR holding dictionary ids) the ids offset by dict_off into vid.
-void pack_csr(const CsrView& A, u64 row_off, u64 col_off, u64 nnz_off, u64* row_ptr, u32* col, Zd* val, u16* vid,
-              u32 dict_off, hipStream_t st);
+/// One block's CSR into the packed one, each row's entries in their order. Rows offset by row_off, the row
+/// pointers (from nnz_off on) written; or, with row_place, moved to row_place[row_off + r], the row
+/// pointers there given (place_lengths and row_scan). Columns at col_off + c or col_place[col_off + c];
+/// values in full into val, or (vid set, the block holding ids) the ids offset by dict_off into vid. col
+/// null: the row pointers alone; val and vid null: no values.
+void pack_csr(const CsrView& A, u64 row_off, const u32* row_place, u64 col_off, const u32* col_place, u64 nnz_off,
+              u64* row_ptr, u32* col, Zd* val, u16* vid, u32 dict_off, hipStream_t st);
+/// len[place[row_off + r]] = the length of the block's row r.
+void place_lengths(const CsrView& A, u64 row_off, const u32* place, u32* len, hipStream_t st);
 void batch_advance(const BatchView& B, hipStream_t st);
 /// One classical Gram-Schmidt pass of the batch vectors W against kept layers 0 .. K-1 (layer k at
 /// basis + k * layer entries, the batch layout), only for the blocks whose full[b] is set and, with

@@ -57,6 +57,23 @@ template <class T> void put(DeviceBuffer& b, const std::vector<T>& h, hipStream_
     QSA_HIP(hipStreamSynchronize(st));
 }
 
+/// Bytes that the row order and the R = 1 slices may take beyond the packed CSR
+/// (QED_SPIN_AMD_BATCH_EXTRA_BYTES; without it, what can be allocated).
+std::uint64_t extra_bytes() {
+    const char* e = std::getenv("QED_SPIN_AMD_BATCH_EXTRA_BYTES");
+    return e ? std::strtoull(e, nullptr, 10) : ~std::uint64_t{0};
+}
+
+/// fn(), or false when it ran out of device memory.
+template <class Fn> bool if_it_fits(Fn&& fn) {
+    try {
+        return fn();
+    } catch (const Error& e) {
+        if (e.code != kResourceLimit) throw;
+        return false;
+    }
+}
+
 /// A pooled stream at the default priority (graph capture needs a stream other than the null one).
 struct OwnStream {
     hipStream_t s = nullptr;
@@ -88,8 +105,6 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     nnz_ = nnz_off.back();
     if (rows_ >= (std::uint64_t{1} << 32)) throw Error(kInvalid, "batched lanczos: more than 2^32 rows in one batch");
     const hipStream_t st = engine_stream();
-    row_ptr_.reset((rows_ + 1) * 8);
-    col_.reset(std::max<std::uint64_t>(nnz_, 1) * 4);
     // Values: when every block stores dictionary ids and the dictionaries hold at most 2^16 values
     // together, 16-bit ids into their concatenation (2 bytes per entry instead of 16); else in full.
     std::vector<std::uint32_t> dict_off(ops_.size() + 1, 0);
@@ -110,7 +125,6 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
         dict_n_ = static_cast<std::uint32_t>(dict_total);
         dict_off.back() = dict_n_;
         put(dict_begin_, dict_off, st);
-        vid_.reset(std::max<std::uint64_t>(nnz_, 1) * 2);
         dict_re_.reset(dict_total * 8);
         dict_im_.reset(dict_total * 8);
         for (std::size_t b = 0; b < ops_.size(); ++b) {
@@ -122,14 +136,7 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
             else
                 QSA_HIP(hipMemcpyAsync(dict_im_.get<double>() + dict_off[b], A.dict_im, n, hipMemcpyDeviceToDevice, st));
         }
-    } else {
-        val_.reset(std::max<std::uint64_t>(nnz_, 1) * sizeof(dev::Zd));
     }
-    for (std::size_t b = 0; b < ops_.size(); ++b)
-        dev::pack_csr(ops_[b]->device_csr(), row_off_[b], row_off_[b], nnz_off[b], row_ptr_.get<std::uint64_t>(),
-                      col_.get<std::uint32_t>(), ids ? nullptr : val_.get<dev::Zd>(),
-                      ids ? vid_.get<std::uint16_t>() : nullptr, dict_off[b], st);
-    QSA_HIP(hipGetLastError());
     // Tiles: every block cut into runs of at most kBatchTileRows rows, blocks in order.
     tile_begin_.assign(1, 0);
     for (std::size_t b = 0; b < ops_.size(); ++b) {
@@ -144,9 +151,46 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
     }
     put(tiles_d_, tiles_, st);
     put(tile_begin_d_, tile_begin_, st);
+    // The matrix: the row pointers, and (where rows will move) the columns that the order is found from;
+    // then the entries, straight from the blocks to where they stay, so that no second copy exists at
+    // any time. R = 1: into slices, unless these do not fit.
+    std::vector<std::uint8_t> reorder(ops_.size(), 0);
+    bool any = false;
+    const std::uint64_t wide = static_cast<std::uint64_t>(std::min(R_, 8)) * sizeof(dev::Zd);
+    for (std::size_t b = 0; b < ops_.size(); ++b) {
+        reorder[b] = dim(static_cast<int>(b)) * wide > kOrderMinBytes ? 1 : 0;
+        any = any || reorder[b];
+    }
+    const bool slices = R_ == 1;
+    row_ptr_.reset((rows_ + 1) * 8);
+    auto room = [&] {
+        col_.reset(std::max<std::uint64_t>(nnz_, 1) * 4);
+        if (ids) vid_.reset(std::max<std::uint64_t>(nnz_, 1) * 2);
+        else val_.reset(std::max<std::uint64_t>(nnz_, 1) * sizeof(dev::Zd));
+    };
+    auto pack = [&](std::size_t b, const std::uint32_t* place, bool values) {
+        dev::pack_csr(ops_[b]->device_csr(), row_off_[b], place, row_off_[b], place, nnz_off[b], row_ptr_.get<std::uint64_t>(),
+                      col_.get<std::uint32_t>(), values && !ids ? val_.get<dev::Zd>() : nullptr,
+                      values && ids ? vid_.get<std::uint16_t>() : nullptr, dict_off[b], st);
+    };
+    if (!slices) room();
+    else if (any) col_.reset(std::max<std::uint64_t>(nnz_, 1) * 4);
+    for (std::size_t b = 0; b < ops_.size(); ++b) pack(b, nullptr, !slices && !reorder[b]);
+    QSA_HIP(hipGetLastError());
     const auto t_order = clock_t_::now();
-    order_rows();
-    if (R_ == 1) slice_rows();
+    if (any && !if_it_fits([&] { return order_rows(reorder); })) {
+        order_.release();
+        place_.release();
+    }
+    if (slices) {
+        col_.release();
+        one_ = if_it_fits([&] { return slice_rows(ids); });
+        if (!one_) room();
+    }
+    for (std::size_t b = 0; b < ops_.size() && !one_; ++b)
+        if (slices || reorder[b]) pack(b, place_.get<std::uint32_t>(), true);
+    order_.release();
+    QSA_HIP(hipGetLastError());
     const char* pinned = std::getenv("QED_SPIN_AMD_BATCH_SCHEDULE");   // 0 or 1
     set_schedule(pinned ? (std::atoi(pinned) == 1 ? 1 : 0) : 1);
     order_s_ = secs(t_order, clock_t_::now());
@@ -181,15 +225,9 @@ BatchedLanczos::BatchedLanczos(std::vector<std::shared_ptr<const SectorOperator>
 // (Rows of a level by their least column of the level before, so that neighbours share columns in the
 // L1, took a fifth of the L1's misses at R = 1 for 2% of the step, and made the J1-J2 rings' step at
 // R = 4 9% slower.)
-void BatchedLanczos::order_rows() {
-    const std::uint64_t wide = static_cast<std::uint64_t>(std::min(R_, 8)) * sizeof(dev::Zd);
-    std::vector<std::uint8_t> reorder(ops_.size(), 0);
-    bool any = false;
-    for (std::size_t b = 0; b < ops_.size(); ++b) {
-        reorder[b] = dim(static_cast<int>(b)) * wide > kOrderMinBytes ? 1 : 0;
-        any = any || reorder[b];
-    }
-    if (!any || ops_.size() >= (std::size_t{1} << 24)) return;
+bool BatchedLanczos::order_rows(const std::vector<std::uint8_t>& reorder) {
+    // (the sort and the scan count rows in 32 bits; 33 bytes a row and the sort's own at the peak)
+    if (rows_ >= (std::uint64_t{1} << 31) || ops_.size() >= (std::size_t{1} << 24) || rows_ * 33 > extra_bytes()) return false;
     const hipStream_t st = engine_stream();
     dev::BatchView B = view();
     DeviceBuffer flags, level(rows_), marked(256 * 4);
@@ -217,54 +255,47 @@ void BatchedLanczos::order_rows() {
                          st);
         QSA_HIP(hipGetLastError());
     }
-    reorder_matrix(rows_, order_.get<std::uint32_t>(), place_.get<std::uint32_t>(), row_ptr_, col_, vid_, val_);
+    DeviceBuffer len(rows_ * 4), ptr((rows_ + 1) * 8);
+    dev::order_lengths(row_ptr_.get<std::uint64_t>(), order_.get<std::uint32_t>(), rows_, len.get<std::uint32_t>(), st);
+    const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows_));
+    DeviceBuffer temp(tb ? tb : 8);
+    dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), ptr.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(hipGetLastError());
+    row_ptr_ = std::move(ptr);   // the old one is freed on this stream, after the kernels that read it
+    return true;
 }
 
-/// The packed matrix in the R = 1 layout, in place of the CSR.
-void BatchedLanczos::slice_rows() {
+/// The matrix in the R = 1 layout, straight from the blocks, in place of the row pointers; false when
+/// rows of very different lengths would fill it to more than twice the entries.
+bool BatchedLanczos::slice_rows(bool ids) {
     const hipStream_t st = engine_stream();
     const dev::BatchView B = view();
     const std::int64_t slices = static_cast<std::int64_t>(tiles_.size()) * (dev::kBatchTileRows / 64);
     DeviceBuffer words(static_cast<std::size_t>(slices + 1) * 8);
-    one_len_.reset(rows_ * 4);
-    one_ptr_.reset(static_cast<std::size_t>(slices + 1) * 8);
+    DeviceBuffer len(rows_ * 4), ptr(static_cast<std::size_t>(slices + 1) * 8);
     dev::fill_zero(false, words.get(), static_cast<std::size_t>(slices + 1), st);
-    dev::one_lengths(B, one_len_.get<std::uint32_t>(), words.get<std::uint64_t>(), st);
+    dev::one_lengths(B, len.get<std::uint32_t>(), words.get<std::uint64_t>(), st);
     const std::size_t tb = dev::sell_scan_temp_bytes(slices);
     DeviceBuffer temp(tb ? tb : 8);
-    dev::sell_scan(words.get<std::uint64_t>(), slices, one_ptr_.get<std::uint64_t>(), temp.get(), tb, st);
+    dev::sell_scan(words.get<std::uint64_t>(), slices, ptr.get<std::uint64_t>(), temp.get(), tb, st);
     QSA_HIP(hipGetLastError());
     std::uint64_t total = 0;
-    copy_to_host(&total, one_ptr_.get<std::uint64_t>() + slices, 8);
-    const bool ids = B.vid && dev::batch_dict_in_lds(B);
-    DeviceBuffer col(std::max<std::uint64_t>(total, 1) * 4), vid(ids ? total * 2 : 0),
+    copy_to_host(&total, ptr.get<std::uint64_t>() + slices, 8);
+    const std::uint64_t least = rows_ * 8;   // (short rows fill whole groups of eight)
+    if (total > 2 * std::max(nnz_, least) || total * 6 > extra_bytes()) return false;
+    DeviceBuffer col(std::max<std::uint64_t>(total, 1) * 4), vid(ids ? std::max<std::uint64_t>(total, 1) * 2 : 0),
         val(ids ? 0 : std::max<std::uint64_t>(total, 1) * sizeof(dev::Zd));
-    dev::one_fill(B, one_ptr_.get<std::uint64_t>(), col.get<std::uint32_t>(), vid.get<std::uint16_t>(), val.get<dev::Zd>(), st);
+    for (std::size_t b = 0; b < ops_.size(); ++b)
+        dev::one_fill(ops_[b]->device_csr(), row_off_[b], tile_begin_[b], order_.get<std::uint32_t>(), place_.get<std::uint32_t>(),
+                      ptr.get<std::uint64_t>(), col.get<std::uint32_t>(), vid.get<std::uint16_t>(), val.get<dev::Zd>(), st);
     QSA_HIP(hipGetLastError());
+    one_ptr_ = std::move(ptr);
+    one_len_ = std::move(len);
     col_ = std::move(col);
     vid_ = std::move(vid);
     val_ = std::move(val);
     row_ptr_.release();
-    one_ = true;
-}
-
-void reorder_matrix(std::uint64_t rows, const std::uint32_t* order, const std::uint32_t* place, DeviceBuffer& row_ptr,
-                    DeviceBuffer& col, DeviceBuffer& vid, DeviceBuffer& val) {
-    const hipStream_t st = engine_stream();
-    DeviceBuffer len(rows * 4), ptr((rows + 1) * 8);
-    dev::order_lengths(row_ptr.get<std::uint64_t>(), order, rows, len.get<std::uint32_t>(), st);
-    const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows));
-    DeviceBuffer temp(tb ? tb : 8);
-    dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows), ptr.get<std::uint64_t>(), temp.get(), tb, st);
-    DeviceBuffer ncol(col.bytes()), nvid(vid.bytes()), nval(val.bytes());
-    dev::order_rows(row_ptr.get<std::uint64_t>(), col.get<std::uint32_t>(), vid.get<std::uint16_t>(), val.get<dev::Zd>(), order,
-                    place, rows, ptr.get<std::uint64_t>(), ncol.get<std::uint32_t>(), nvid.get<std::uint16_t>(),
-                    nval.get<dev::Zd>(), st);
-    QSA_HIP(hipGetLastError());
-    row_ptr = std::move(ptr);   // the old ones are freed on this stream, after the kernels that read them
-    col = std::move(ncol);
-    vid = std::move(nvid);
-    val = std::move(nval);
+    return true;
 }
 
 void BatchedLanczos::set_schedule(int kind) {

@@ -74,15 +74,13 @@ public:
     int schedule() const { return sched_kind_; }
     /// Host seconds the row order and the schedule took.
     double order_seconds() const { return order_s_; }
-    /// The engine's row order (device, rows() words each, null: the states' order): the packed row of
-    /// the states' order at place i, and the place of each such row.
-    const std::uint32_t* order() const { return order_.get<std::uint32_t>(); }
+    /// The engine's row order (device, rows() words, null: the states' order): the place of each row.
     const std::uint32_t* place() const { return place_.get<std::uint32_t>(); }
 
 private:
     dev::BatchView view() const;
-    void order_rows();
-    void slice_rows();
+    bool order_rows(const std::vector<std::uint8_t>& reorder);
+    bool slice_rows(bool ids);
     /// Blocks whose vectors (eight at most) take more than this are stored in level order: half an
     /// XCD's L2.
     static constexpr std::uint64_t kOrderMinBytes = 2u << 20;
@@ -106,11 +104,6 @@ private:
         tol_d_;
     friend struct BatchedAccess;
 };
-
-/// A packed matrix with its rows in `order` (null: kept) and its columns moved to `place` (null: kept),
-/// each row's entries in their order; vid or val may be empty.
-void reorder_matrix(std::uint64_t rows, const std::uint32_t* order, const std::uint32_t* place, DeviceBuffer& row_ptr,
-                    DeviceBuffer& col, DeviceBuffer& vid, DeviceBuffer& val);
 
 struct BatchedFtlmOptions {
     int samples = 40, krylov = 100;

@@ -24,7 +24,7 @@ double since(clk::time_point a) { return std::chrono::duration<double>(clk::now(
 class PackedProbe {
 public:
     PackedProbe(const std::vector<const SectorOperator*>& probes, const std::vector<std::uint64_t>& row_off,
-                const std::vector<std::uint64_t>& col_off, int R, const std::uint32_t* row_order,
+                const std::vector<std::uint64_t>& col_off, int R, const std::uint32_t* row_place,
                 const std::uint32_t* col_place)
         : R_(R) {
         const hipStream_t st = engine_stream();
@@ -37,14 +37,20 @@ public:
         row_ptr_.reset((rows_ + 1) * 8);
         col_.reset(std::max<std::uint64_t>(nnz_off.back(), 1) * 4);
         val_.reset(std::max<std::uint64_t>(nnz_off.back(), 1) * sizeof(dev::Zd));
-        for (std::size_t c = 0; c < probes.size(); ++c)
-            dev::pack_csr(probes[c]->device_csr(), row_off[c], col_off[c], nnz_off[c], row_ptr_.get<std::uint64_t>(),
-                          col_.get<std::uint32_t>(), val_.get<dev::Zd>(), nullptr, 0, st);
-        QSA_HIP(hipGetLastError());
-        if (row_order || col_place) {   // into the engines' row orders
-            DeviceBuffer no_ids;
-            reorder_matrix(rows_, row_order, col_place, row_ptr_, col_, no_ids, val_);
+        // into the engines' row orders
+        if (row_place) {
+            DeviceBuffer len(rows_ * 4);
+            for (std::size_t c = 0; c < probes.size(); ++c)
+                dev::place_lengths(probes[c]->device_csr(), row_off[c], row_place, len.get<std::uint32_t>(), st);
+            const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows_));
+            DeviceBuffer temp(tb ? tb : 8);
+            dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), row_ptr_.get<std::uint64_t>(), temp.get(),
+                          tb, st);
         }
+        for (std::size_t c = 0; c < probes.size(); ++c)
+            dev::pack_csr(probes[c]->device_csr(), row_off[c], row_place, col_off[c], col_place, nnz_off[c],
+                          row_ptr_.get<std::uint64_t>(), col_.get<std::uint32_t>(), val_.get<dev::Zd>(), nullptr, 0, st);
+        QSA_HIP(hipGetLastError());
         std::vector<dev::Tile> tiles;
         std::vector<std::uint32_t> begin(1, 0);
         for (std::size_t c = 0; c < probes.size(); ++c) {
@@ -274,7 +280,7 @@ DynWalkResult ftlm_dynamics_walk(const std::vector<std::shared_ptr<const SectorO
                     full_c.push_back(static_cast<std::size_t>(channels[c].H->dim()) <= full_limit ? 1 : 0);
                 }
                 BatchedLanczos T(wtgt, R);
-                const PackedProbe P(probes, crow, colo, R, T.order(), S.place());
+                const PackedProbe P(probes, crow, colo, R, T.place(), S.place());
                 P.apply(Vs, reinterpret_cast<dev::Zd*>(T.start_buffer()));
                 T.normalize(&n2);
                 std::vector<int> live(nc * static_cast<std::size_t>(R));
