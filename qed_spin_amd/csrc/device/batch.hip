@@ -1106,14 +1106,18 @@ std::size_t level_sort_temp_bytes(u64 rows) {
     return bytes;
 }
 
-void level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
-                 std::size_t temp_bytes, hipStream_t st) {
-    if (!B.n_tiles) return;
+hipError_t level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
+                       std::size_t temp_bytes, hipStream_t st) {
+    if (!B.n_tiles) return hipSuccess;
+    if (B.rows >> 32 != 0) return hipErrorInvalidValue;   // rows are 32-bit words
     hipLaunchKernelGGL(k_level_keys, dim3(B.n_tiles), dim3(kThreads), 0, st, B, level, key, row);
     int bits = 8;
     while (bits < 32 && (static_cast<u64>(B.n_blocks) >> (bits - 8)) != 0) ++bits;
-    (void)hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, key, key2, row, order, static_cast<unsigned>(B.rows), 0, bits, st);
+    const hipError_t e = hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, key, key2, row, order,
+                                                            static_cast<unsigned>(B.rows), 0, bits, st);
+    if (e != hipSuccess) return e;   // (order is no index then)
     hipLaunchKernelGGL(k_order_invert, dim3(grid_for(B.rows)), dim3(256), 0, st, order, B.rows, place);
+    return hipSuccess;
 }
 
 void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hipStream_t st) {

@@ -62,7 +62,7 @@ void csr_stage_dict(i64 rows, const u32* row_len, const Zd* stage_val, const Dic
 void csr_compact(i64 rows, const u64* row_ptr, const u32* stage_col, const Zd* stage_val, u32* col, void* vals,
                  int width, bool real, const DictTable& D, hipStream_t st);
 std::size_t row_scan_temp_bytes(i64 rows);
-void row_scan(const u32* row_len, i64 rows, u64* row_ptr, void* temp, std::size_t temp_bytes, hipStream_t st);
+[[nodiscard]] hipError_t row_scan(const u32* row_len, i64 rows, u64* row_ptr, void* temp, std::size_t temp_bytes, hipStream_t st);
 
 // ---- irrep.hip -------------------------------------------------------------------------------
 /// masks[r * words + w] bit b: element 64 w + b fixes representative r (words = ceil(G / 64)).
@@ -137,7 +137,7 @@ void pack_col_ids(u32* col, const u8* id, u64 nnz, hipStream_t st);
 /// (value_bytes 0: none, 1, 2, 8 or 16) into the slices.
 void sell_lengths(const u64* row_ptr, i64 rows, u16* sell_len, u64* slice_words, u32* too_long, hipStream_t st);
 std::size_t sell_scan_temp_bytes(i64 n_slices);
-void sell_scan(const u64* slice_words, i64 n_slices, u64* sell_ptr, void* temp, std::size_t temp_bytes,
+[[nodiscard]] hipError_t sell_scan(const u64* slice_words, i64 n_slices, u64* sell_ptr, void* temp, std::size_t temp_bytes,
                hipStream_t st);
 void sell_fill(const u64* row_ptr, const u32* col, const void* vals, int value_bytes, i64 rows, const u64* sell_ptr,
                u32* sell_col, void* sell_vals, bool diag_first, bool packed, hipStream_t st);
@@ -312,7 +312,7 @@ void level_sweep(const BatchView& B, const u8* reorder, u32 l, u8* level, u32* m
 std::size_t level_sort_temp_bytes(u64 rows);
 /// order[i] = the row at place i when every block's rows go by level, then by row; place: its inverse.
 /// key, key2, row: rows words each.
-void level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
+[[nodiscard]] hipError_t level_order(const BatchView& B, const u8* level, u32* key, u32* key2, u32* row, u32* order, u32* place, void* temp,
                  std::size_t temp_bytes, hipStream_t st);
 /// len[i] = the length of the row that `order` puts at place i.
 void order_lengths(const u64* row_ptr, const u32* order, u64 rows, u32* len, hipStream_t st);

@@ -866,8 +866,10 @@ std::size_t sell_scan_temp_bytes(i64 n_slices) {
     return bytes;
 }
 
-void sell_scan(const u64* slice_words, i64 n_slices, u64* sell_ptr, void* temp, std::size_t temp_bytes, hipStream_t st) {
-    (void)hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, slice_words, sell_ptr, static_cast<int>(n_slices + 1), st);
+hipError_t sell_scan(const u64* slice_words, i64 n_slices, u64* sell_ptr, void* temp, std::size_t temp_bytes,
+                     hipStream_t st) {
+    if (n_slices < 0 || n_slices >= (i64{1} << 31) - 1) return hipErrorInvalidValue;   // (counted in 32 bits)
+    return hipcub::DeviceScan::ExclusiveSum(temp, temp_bytes, slice_words, sell_ptr, static_cast<int>(n_slices + 1), st);
 }
 
 void sell_fill(const u64* row_ptr, const u32* col, const void* vals, int value_bytes, i64 rows, const u64* sell_ptr,

@@ -703,6 +703,7 @@ void walk_gather(const SectorView& R, const SectorView& C, bool same, const Prog
 
 
 namespace {
+constexpr i64 kScanMax = (i64{1} << 31) - 1;   // the scan counts in 32 bits
 struct ToU64 {
     __host__ __device__ u64 operator()(u32 x) const { return static_cast<u64>(x); }
 };
@@ -711,16 +712,18 @@ struct ToU64 {
 std::size_t row_scan_temp_bytes(i64 rows) {
     std::size_t bytes = 0;
     hipcub::TransformInputIterator<u64, ToU64, const u32*> it(nullptr, ToU64{});
-    hipcub::DeviceScan::InclusiveSum(nullptr, bytes, it, static_cast<u64*>(nullptr), static_cast<int>(rows));
+    if (rows > kScanMax) return 0;   // row_scan refuses it
+    (void)hipcub::DeviceScan::InclusiveSum(nullptr, bytes, it, static_cast<u64*>(nullptr), static_cast<int>(rows));
     return bytes;
 }
 
 // row_ptr[0] = 0, row_ptr[r + 1] = sum of row_len[0..r].
-void row_scan(const u32* row_len, i64 rows, u64* row_ptr, void* temp, std::size_t temp_bytes, hipStream_t st) {
-    hipMemsetAsync(row_ptr, 0, sizeof(u64), st);
-    if (rows == 0) return;
+hipError_t row_scan(const u32* row_len, i64 rows, u64* row_ptr, void* temp, std::size_t temp_bytes, hipStream_t st) {
+    if (rows < 0 || rows > kScanMax) return hipErrorInvalidValue;
+    const hipError_t e = hipMemsetAsync(row_ptr, 0, sizeof(u64), st);
+    if (e != hipSuccess || rows == 0) return e;
     hipcub::TransformInputIterator<u64, ToU64, const u32*> it(row_len, ToU64{});
-    hipcub::DeviceScan::InclusiveSum(temp, temp_bytes, it, row_ptr + 1, static_cast<int>(rows), st);
+    return hipcub::DeviceScan::InclusiveSum(temp, temp_bytes, it, row_ptr + 1, static_cast<int>(rows), st);
 }
 
 }  // namespace qsa::dev

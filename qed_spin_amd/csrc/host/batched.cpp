@@ -250,16 +250,16 @@ bool BatchedLanczos::order_rows(const std::vector<std::uint8_t>& reorder) {
         DeviceBuffer key(rows_ * 4), key2(rows_ * 4), row(rows_ * 4);
         const std::size_t tb = dev::level_sort_temp_bytes(rows_);
         DeviceBuffer temp(tb ? tb : 8);
-        dev::level_order(B, level.get<std::uint8_t>(), key.get<std::uint32_t>(), key2.get<std::uint32_t>(),
+        QSA_HIP(dev::level_order(B, level.get<std::uint8_t>(), key.get<std::uint32_t>(), key2.get<std::uint32_t>(),
                          row.get<std::uint32_t>(), order_.get<std::uint32_t>(), place_.get<std::uint32_t>(), temp.get(), tb,
-                         st);
+                         st));
         QSA_HIP(hipGetLastError());
     }
     DeviceBuffer len(rows_ * 4), ptr((rows_ + 1) * 8);
     dev::order_lengths(row_ptr_.get<std::uint64_t>(), order_.get<std::uint32_t>(), rows_, len.get<std::uint32_t>(), st);
     const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows_));
     DeviceBuffer temp(tb ? tb : 8);
-    dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), ptr.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), ptr.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     row_ptr_ = std::move(ptr);   // the old one is freed on this stream, after the kernels that read it
     return true;
@@ -277,7 +277,7 @@ bool BatchedLanczos::slice_rows(bool ids) {
     dev::one_lengths(B, len.get<std::uint32_t>(), words.get<std::uint64_t>(), st);
     const std::size_t tb = dev::sell_scan_temp_bytes(slices);
     DeviceBuffer temp(tb ? tb : 8);
-    dev::sell_scan(words.get<std::uint64_t>(), slices, ptr.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::sell_scan(words.get<std::uint64_t>(), slices, ptr.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     std::uint64_t total = 0;
     copy_to_host(&total, ptr.get<std::uint64_t>() + slices, 8);

@@ -44,8 +44,8 @@ public:
                 dev::place_lengths(probes[c]->device_csr(), row_off[c], row_place, len.get<std::uint32_t>(), st);
             const std::size_t tb = dev::row_scan_temp_bytes(static_cast<std::int64_t>(rows_));
             DeviceBuffer temp(tb ? tb : 8);
-            dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), row_ptr_.get<std::uint64_t>(), temp.get(),
-                          tb, st);
+            QSA_HIP(dev::row_scan(len.get<std::uint32_t>(), static_cast<std::int64_t>(rows_), row_ptr_.get<std::uint64_t>(), temp.get(),
+                          tb, st));
         }
         for (std::size_t c = 0; c < probes.size(); ++c)
             dev::pack_csr(probes[c]->device_csr(), row_off[c], row_place, col_off[c], col_place, nnz_off[c],

@@ -193,7 +193,7 @@ void SectorOperator::build_csr(std::uint64_t budget) {
     row_ptr_.reset(static_cast<std::size_t>(rows + 1) * 8);
     const std::size_t tb = dev::row_scan_temp_bytes(rows);
     DeviceBuffer temp(tb ? tb : 8);
-    dev::row_scan(row_len.get<std::uint32_t>(), rows, row_ptr_.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::row_scan(row_len.get<std::uint32_t>(), rows, row_ptr_.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     std::uint64_t nnz = 0;
     unsigned cnt[2] = {0, 0};
@@ -311,7 +311,7 @@ void SectorOperator::build_csr_irrep(std::uint64_t budget) {
     row_ptr_.reset(static_cast<std::size_t>(rows + 1) * 8);
     const std::size_t tb = dev::row_scan_temp_bytes(rows);
     DeviceBuffer temp(tb ? tb : 8);
-    dev::row_scan(row_len.get<std::uint32_t>(), rows, row_ptr_.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::row_scan(row_len.get<std::uint32_t>(), rows, row_ptr_.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     std::uint64_t nnz = 0;
     QSA_HIP(hipMemcpyAsync(&nnz, row_ptr_.get<std::uint64_t>() + rows, 8, hipMemcpyDeviceToHost, st));
@@ -332,7 +332,7 @@ void SectorOperator::build_csr_irrep(std::uint64_t budget) {
                         row_len.get<std::uint32_t>(), st);
     QSA_HIP(hipGetLastError());
     DeviceBuffer merged_ptr(static_cast<std::size_t>(rows + 1) * 8);
-    dev::row_scan(row_len.get<std::uint32_t>(), rows, merged_ptr.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::row_scan(row_len.get<std::uint32_t>(), rows, merged_ptr.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     QSA_HIP(hipMemcpyAsync(&nnz, merged_ptr.get<std::uint64_t>() + rows, 8, hipMemcpyDeviceToHost, st));
     QSA_HIP(hipStreamSynchronize(st));
@@ -383,7 +383,7 @@ bool SectorOperator::build_sell(bool diag_first) {
                       flag.get<std::uint32_t>(), st);
     const std::size_t tb = dev::sell_scan_temp_bytes(slices);
     DeviceBuffer temp(tb ? tb : 8);
-    dev::sell_scan(words.get<std::uint64_t>(), slices, sell_ptr_.get<std::uint64_t>(), temp.get(), tb, st);
+    QSA_HIP(dev::sell_scan(words.get<std::uint64_t>(), slices, sell_ptr_.get<std::uint64_t>(), temp.get(), tb, st));
     QSA_HIP(hipGetLastError());
     std::uint64_t total = 0;
     std::uint32_t too_long = 0;
