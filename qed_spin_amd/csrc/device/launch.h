@@ -145,10 +145,10 @@ void sell_fill(const u64* row_ptr, const u32* col, const void* vals, int value_b
 /// Whether single applies of A run in workgroups of one size whatever wg says (a staged dictionary
 /// above 16 KB).
 bool spmv_workgroup_fixed(const CsrView& A);
-/// Workgroups of sell_lanczos on A (its partial buffer holds two doubles per workgroup).
-unsigned sell_lanczos_blocks(const CsrView& A);
+/// Partial sums of sell_lanczos on A (two doubles each).
+unsigned sell_lanczos_parts(const CsrView& A);
 /// The first pass of a Lanczos step in the SELL SpMV's epilogue: w = A v - *beta v_prev (v_prev null:
-/// w = A v; beta on the device), and <v, w> into alpha (device) through partial (2 sell_lanczos_blocks(A)
+/// w = A v; beta on the device), and <v, w> into alpha (device) through partial (2 sell_lanczos_parts(A)
 /// doubles), summed in a fixed order. false (nothing launched) without the SELL layout, or real vectors on complex
 /// values.
 bool sell_lanczos(const CsrView& A, bool real, const void* v, const void* vprev, const double* beta, void* w,

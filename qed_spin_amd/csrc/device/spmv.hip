@@ -398,15 +398,17 @@ __global__ __launch_bounds__(1024) void k_sell(CsrView A, Ptrs<NV> v) {
 }
 
 // The Lanczos step's first pass in the SpMV's epilogue: w = H v - beta v_prev (v_prev null at the
-// first step) written, and the workgroup's partial of <v, w> (the wavefronts' xor trees, then the
-// wavefronts in order) into partial[workgroup] -- the apply followed by axpy_dot, without writing
-// and reading w in between. k_lanczos_finish sums the partials in workgroup order.
+// first step) written, and the partial of <v, w> of each kLanczosPart rows (the wavefronts' xor trees,
+// then the wavefronts in order) into partial -- the apply followed by axpy_dot, without writing and
+// reading w in between. k_lanczos_finish sums the partials in row order, so alpha's bits do not depend on
+// the workgroup size that the tuner picked.
+constexpr int kLanczosPart = 256;
 template <int WIDTH, bool VREAL, bool REAL, bool LD, int U, int ACC>
 __global__ __launch_bounds__(1024) void k_sell_lanczos(CsrView A, Ptrs<1> v, const void* vprev,
                                                        const double* betap, double* partial) {
     __shared__ double wr[16], wi[16];
     const Dict<LD> d = stage_dict<WIDTH, VREAL, LD>(A);
-    const i64 row = row_block(A) * blockDim.x + threadIdx.x;
+    const i64 row0 = row_block(A) * blockDim.x, row = row0 + threadIdx.x;
     const double beta = vprev ? *betap : 0.0;
     double pr = 0.0, pi = 0.0;
     if (row < A.rows) {
@@ -440,19 +442,20 @@ __global__ __launch_bounds__(1024) void k_sell_lanczos(CsrView A, Ptrs<1> v, con
         wi[wave] = pi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    constexpr int kWaves = kLanczosPart / 64;
+    const i64 first = row0 + static_cast<i64>(threadIdx.x) * kLanczosPart;   // thread t sums the workgroup's part t
+    if (threadIdx.x < blockDim.x / kLanczosPart && first < A.rows) {
         double a = 0.0, b = 0.0;
-        for (int q = 0; q < static_cast<int>(blockDim.x >> 6); ++q) {
-            a += wr[q];
-            b += wi[q];
+        for (int q = 0; q < kWaves; ++q) {
+            a += wr[static_cast<int>(threadIdx.x) * kWaves + q];
+            b += wi[static_cast<int>(threadIdx.x) * kWaves + q];
         }
-        partial[2 * static_cast<u64>(blockIdx.x)] = a;
-        partial[2 * static_cast<u64>(blockIdx.x) + 1] = b;
+        partial[2 * (first / kLanczosPart)] = a;
+        partial[2 * (first / kLanczosPart) + 1] = b;
     }
 }
 
-// (One workgroup sums up to some ten thousand pairs: 1024 threads take 5 us for 10,106 of them, 256 took
-// 16.)
+// (One workgroup sums all pairs: 1024 threads take 5 us for 10,106 of them, 256 took 16.)
 constexpr int kFinishThreads = 1024;
 __global__ __launch_bounds__(kFinishThreads) void k_lanczos_finish(const double* partial, int nb, Zd* alpha) {
     __shared__ double sr[kFinishThreads], si[kFinishThreads];
@@ -902,14 +905,13 @@ bool spmv_workgroup_fixed(const CsrView& A) {
     return dict_in_lds(B) && dict_lds_bytes(B) > 16 * 1024;
 }
 
-unsigned sell_lanczos_blocks(const CsrView& A) { return grid_blocks(staged(A, 1, 1), static_cast<u64>(A.rows)); }
+unsigned sell_lanczos_parts(const CsrView& A) { return static_cast<unsigned>((A.rows + kLanczosPart - 1) / kLanczosPart); }
 
 bool sell_lanczos(const CsrView& V, bool real, const void* v, const void* vprev, const double* beta, void* w,
                   double* partial, Zd* alpha, hipStream_t st) {
     if (!V.sell_ptr || V.rows == 0 || (real && !V.values_real)) return false;
     const CsrView A = staged(V, 1, 1);
-    const unsigned nb = sell_lanczos_blocks(A);
-    const dim3 grid(nb), block(block_threads(A));
+    const dim3 grid(grid_blocks(A, static_cast<u64>(A.rows))), block(block_threads(A));
     Ptrs<1> p;
     p.in[0] = v;
     p.out[0] = w;
@@ -943,7 +945,7 @@ bool sell_lanczos(const CsrView& V, bool real, const void* v, const void* vprev,
     if (real) by_width(T{}, T{});
     else if (A.values_real) by_width(T{}, F{});
     else by_width(F{}, F{});
-    hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kFinishThreads), 0, st, partial, static_cast<int>(nb), alpha);
+    hipLaunchKernelGGL(k_lanczos_finish, dim3(1), dim3(kFinishThreads), 0, st, partial, static_cast<int>(sell_lanczos_parts(A)), alpha);
     return true;
 }
 

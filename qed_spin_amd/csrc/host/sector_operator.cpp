@@ -434,10 +434,10 @@ void SectorOperator::autotune() {
     // Only choices that leave every result bit unchanged are timed: the gather depth and the
     // workgroup size. The lanes per row set the summation order of a row, so they stay what the
     // mean row length gives and an apply does not depend on timing noise.
-    // On the SELL-64 copy one lane owns a row, so no choice changes a sum.
-    // The workgroup size first, at the middle depth, then the depth at the best size, two launches each:
-    // the two hardly depend on each other, and all pairs four times over were 3.2 ms of the 16 that a
-    // streamed block of 716,000 rows takes, against 1.0.
+    // On the SELL-64 copy one lane owns a row and <v, w> is summed in parts of fixed rows, so no choice
+    // changes a sum. The workgroup size first, at the middle depth, then the depth at the best size, two
+    // launches each: the two hardly depend on each other, and all pairs four times over were 3.2 ms of the
+    // 16 that building a block of 716,000 rows with tuning and estimating it takes, against 1.0.
     const std::vector<int> depths = sell() ? std::vector<int>{8, 4, 16} : std::vector<int>{4, 2, 8};
     const std::vector<int> groups = sell() ? std::vector<int>{256, 512, 1024} : std::vector<int>{512, 1024};
     auto launch = [&] {
@@ -515,7 +515,7 @@ bool SectorOperator::lanczos_first_pass(const void* v, const void* vprev, const 
                                         bool complex_vectors, dev::Zd* alpha, DeviceBuffer& scratch) const {
     if (lane_ != kLaneCsr || !sell() || !same()) return false;
     const dev::CsrView A = csr_view(false, true);
-    const std::size_t need = static_cast<std::size_t>(dev::sell_lanczos_blocks(A)) * 2 * sizeof(double);
+    const std::size_t need = static_cast<std::size_t>(dev::sell_lanczos_parts(A)) * 2 * sizeof(double);
     if (scratch.bytes() < need) scratch.reset(need);
     if (!dev::sell_lanczos(A, real_ && !complex_vectors, v, vprev, beta, w, scratch.get<double>(), alpha, engine_stream()))
         return false;
