@@ -329,8 +329,8 @@ def dynamics(H: Operator, probes, omega, *, eta: float = 0.1, T=None, sym: Optio
         for i, p in owner:
             S[p] += out[i]
             norms[p] += nsq[i]
-        engine = dict(zip(["pack_s", "steps_s", "host_s", "total_s", "applies", "rows", "nnz", "schedule", "tune_s"],
-                          stats.tolist()))
+        engine = dict(zip(["pack_s", "steps_s", "host_s", "total_s", "applies", "rows", "nnz", "schedule", "order_s"],
+                          stats.tolist()), tune_s=0.0)
     for p in range(len(probes)):
         S[p] /= float(len(states))
         norms[p] /= float(len(states))

@@ -118,3 +118,10 @@ def test_a_block_of_many_values_among_others(R):
             tol = 1e-12 * m.op.norm_bound()
             assert np.max(np.abs(a[:, i, s] - a1)) <= tol and np.max(np.abs(b[:6, i, s] - b1[1:7])) <= tol
         row += m.dim
+
+
+def test_times_go_by_their_names():
+    print("[case] names", flush=True)
+    ms = mats(14)
+    engine = th.ftlm_batched(ms, 2, 10, [1, 2, 3], np.array([1.0]))[4]
+    assert engine["tune_s"] == 0.0 and 0.0 <= engine["order_s"] <= engine["pack_s"]
