@@ -266,10 +266,11 @@ int qedh_matvec_set_lanes(qedh_matvec m, int lanes);
  * the CSR (64-row slices, one lane per row, sums in entry order) and apply through it; the lanes
  * per row then do not apply. Lanes per row (0 keeps the current) and flags:
  * non-temporal streaming of the CSR arrays, one contiguous row range per XCD, the single-vector
- * gathers issued two, four or eight entries at a time, u8-id dictionaries read from global memory
- * instead of LDS, 256 or 1024 threads per workgroup instead of 512 (every flag leaves the results
- * bit for bit unchanged). The default is XCD rows, unroll 4 (or what the autotuner found), LDS
- * dictionary, 512 threads; flags replace it. */
+ * gathers issued two, four or eight entries at a time, value dictionaries read from global memory
+ * and never from a copy in LDS, 256 or 1024 threads per workgroup instead of 512 (1024 in any case with
+ * more than 16 KB of dictionary in LDS; every flag leaves the results bit for bit unchanged). The
+ * default is XCD rows, unroll 4 (or what the autotuner found), the dictionary in LDS where that pays, 512
+ * threads; flags replace it. */
 enum {
     QEDH_TUNE_NONTEMPORAL = 1,
     QEDH_TUNE_XCD_ROWS = 2,
@@ -338,7 +339,10 @@ int qedh_cf(qedh_matvec m, const double* phi_host, int krylov, int n_omega, cons
  * start: the complex start vectors in batch layout, block b vector s at entry (off_b + i) R + s,
  * off_b = the summed dimensions of the blocks before b (normalised inside). breakdown_tol[b] per
  * block. Outputs alpha[krylov][n_blocks][R], beta[krylov][n_blocks][R] (beta of step j is
- * beta_{j+1}), steps[n_blocks][R]. timings[3] = pack s, steps s, total s (may be NULL). */
+ * beta_{j+1}), steps[n_blocks][R]. timings[3] = pack s, steps s, total s (may be NULL).
+ * Device memory of a batched engine beside the blocks' own: 48 R bytes a row for its vectors, 6 (ids) or
+ * 20 (full values) an entry for its matrix (R = 1: filled up to whole groups of eight), 8 to 16 a row, and
+ * while it is built some 40 a row for the row order, which is left out where it does not fit. */
 int qedh_batch_lanczos(const qedh_matvec* blocks, int n_blocks, int R, int krylov, const double* start,
                        const double* breakdown_tol, int reorth, int use_graph, double* alpha, double* beta,
                        int* steps, double* timings);

@@ -4,9 +4,9 @@
 // Layout: the blocks' CSRs are packed into one block-diagonal CSR (rows and columns offset by the
 // block's first row; values as 16-bit ids into the blocks' dictionaries laid end to end when every
 // block has one and they hold at most 65536 values together, else in full); a batch vector holds R
-// entries per row, X[row R + s], so the R vectors of a row are one contiguous line. Rows are cut
-// into tiles of at most kBatchTileRows rows
-// of one block, one workgroup of 256 threads per tile.
+// entries per row, X[row R + s], so the R vectors of a row are one contiguous line. Rows are cut into
+// tiles of at most kBatchTileRows rows of one block, one workgroup per tile (256 threads; the SpMV of
+// R > 1 has 512).
 //
 // Vector kernels: thread t of a tile is (slot t / R, vector t % R); the 256 / R slots take the
 // tile's rows in turn, so consecutive threads touch consecutive entries whatever R is. A
@@ -16,7 +16,7 @@
 //
 // SpMV: for R > 1 a group of 2, 4 or 8 threads per row, one vector each, that share the row's columns
 // and value ids; above 8 vectors a work item is a tile and a run of eight of its vectors. For R = 1
-// eight threads per row splitting its entries, summed by a fixed xor butterfly.
+// one thread per row of a slice layout (OneView); without room for that, the kernel of R > 1.
 //
 // The order of a block's rows is the engine's own: blocks whose vectors (eight of them at most) do not
 // fit an XCD's L2 are stored by breadth-first level of their matrix's graph, the blocks' states'

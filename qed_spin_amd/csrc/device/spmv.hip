@@ -268,8 +268,8 @@ __global__ __launch_bounds__(256) void k_spmv_block(CsrView A, const void* X, vo
 // Slice s holds rows 64 s .. 64 s + 63 in groups of four entries: entry k of row 64 s + j sits at
 // sell_ptr[s] + 256 (k / 4) + 4 j + k % 4, so one 16-byte load gives a lane four consecutive
 // entries of its row and the group loads of a wavefront's 64 rows are one contiguous kilobyte. A
-// slice is padded to its longest row, rounded up to whole groups; the padding is zero and no entry
-// beyond a row's length is used. One lane owns a row and sums its entries in CSR order: the sum
+// slice is padded to its longest row, rounded up to whole groups; a row's last group is filled up with
+// zeros, what the slice holds past it is not written, and no entry beyond a row's length is used. One lane owns a row and sums its entries in CSR order: the sum
 // depends neither on the workgroup size nor on how many gathers are in flight, and a k-vector
 // apply equals k single applies bit for bit. U entries per round: their groups first, then the U
 // gathers together, then the sums in entry order.

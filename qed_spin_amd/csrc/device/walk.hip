@@ -246,8 +246,10 @@ __global__ __launch_bounds__(1024) void k_gather_lds(SectorView R, SectorView C,
     }
 }
 
-/// LDS budget of the gather workgroup's action. Workgroups of 1024 threads (16 waves) share one copy:
-/// two of them per CU (32 waves, eight per SIMD) fit in 160 KB.
+/// LDS budget of the gather workgroup's action. Workgroups of 1024 threads (16 waves) share one copy: two
+/// copies fit a compute unit's 160 KB, and its registers where the kernel takes at most 64 (no sublattice
+/// order: 38 for one vector). With the sublattice order one vector takes 68 to 72, so one workgroup, four
+/// waves per SIMD, is all that runs there.
 constexpr std::size_t kLdsActionMax = 64 * 1024;
 /// Workgroups of the grid-stride gather: four per CU of a 256-CU device, each loading the action once.
 constexpr u64 kGatherLdsBlocks = 1024;

@@ -305,7 +305,9 @@ void BatchedLanczos::set_schedule(int kind) {
     if (kind != 1 || tiles_.empty()) return;
     // Workgroup w runs on XCD w % 8: each XCD gets one eighth of the tiles, neighbours in order, so that
     // the columns of the rows in flight share its L2; with several runs of vectors, a block's tiles
-    // take one run after the other.
+    // take one run after the other. A rule and not a trial: in level order the two are within 2% of
+    // each other (all steps, in order / in runs: N = 24, 4 samples 118.5 / 117.3 ms; continued fractions,
+    // N = 26, 155.4 / 154.4; N = 22, 40 samples 229.3 / 233.8).
     constexpr std::size_t kXcd = 8;
     const std::size_t nt = tiles_.size(), chunks = static_cast<std::size_t>(dev::batch_chunks(R_));
     const std::size_t longest = (nt + kXcd - 1) / kXcd * chunks;

@@ -6,11 +6,12 @@
 //
 // The scalars stay on the device: a step's coefficients, its norm, the gate of the second Gram-Schmidt
 // pass and of the local correction are read there by the kernels that need them, so steps are enqueued
-// one behind the other and the host looks at alpha and beta a few steps at a time (at once without a
-// convergence check). What lies past the step that ends a run (breakdown, convergence) is not
-// returned. (200 steps with full reorthogonalisation on 9252 states: 108 us a step when the host waited
-// five times a step for a scalar, 54 us so; 100 on 2.6 million, without the basis column's copy and with
-// one norm less: 815 -> 734 us.)
+// one behind the other, at most eight ahead of the device (StepsInFlight), and the host looks at alpha
+// and beta a batch of steps at a time (a few with a convergence check). What lies past the step that
+// ends a run (breakdown, convergence) is not returned. (200 steps with full reorthogonalisation on 9252
+// states: 190 us a step when the host waited five times a step for a scalar and the Gram-Schmidt
+// kernels left the card idle, 49 to 60 us so; 100 on 2.6 million, without the basis column's copy: 832
+// -> 713 us.)
 #pragma once
 
 #include <chrono>

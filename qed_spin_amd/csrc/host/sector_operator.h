@@ -75,9 +75,9 @@ public:
         csr_.lanes = lanes;
         lanes_block_ = lanes;
     }
-    /// Time the single-vector SpMV at every gather depth (2, 4, 8) and workgroup size (512, 1024) on
-    /// this matrix and keep the fastest (both leave the results bit for bit unchanged); a few tens
-    /// of milliseconds on a large sector.
+    /// Time the single-vector SpMV at every workgroup size (SELL 256, 512, 1024; CSR 512, 1024), then at
+    /// every gather depth (4, 8, 16; 2, 4, 8) with the best, on this matrix, and keep the fastest (both
+    /// leave the results bit for bit unchanged): eleven applies at most.
     void autotune();
     int lanes_block() const { return lanes_block_; }
     /// The CSR as the kernels read it (CSR lane only).
@@ -89,7 +89,7 @@ public:
     void set_xcd_rows(bool on) { xcd_ = on; }
     /// Issue the single-vector SpMV's gathers 4 or 8 entries at a time, or 1 (the sums are unchanged).
     void set_unroll(int u) { unroll_ = u; }
-    /// Read u8-id dictionaries from global memory instead of staging them in LDS.
+    /// Read value dictionaries from global memory, never from a copy in LDS.
     void set_global_dict(bool on) { global_dict_ = on; }
     /// Threads per workgroup of the single-vector SpMV (256, 512 or 1024).
     void set_workgroup(int wg) { wg_ = wg; }

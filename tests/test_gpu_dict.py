@@ -1,7 +1,7 @@
-"""Where the SpMV reads an operator's value dictionary: u8 and u16 ids from a copy in LDS, larger
-dictionaries (above 64 KB) from global memory. Both give the same bits, in the CSR and the SELL
-layout, for one vector, several, and row-interleaved ones, and match the oracle within 1e-13. Every
-case prints its name before it touches the device."""
+"""Where the SpMV reads an operator's value dictionary: u8 ids from a copy in LDS, u16 ids too where a
+workgroup's lookups pay for the copy, larger dictionaries (above 63.5 KB) from global memory. Both give the
+same bits, in the CSR and the SELL layout, for one vector, several, and row-interleaved ones, and match the
+oracle within 1e-13. Every case prints its name before it touches the device."""
 
 import sys
 

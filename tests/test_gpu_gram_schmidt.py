@@ -1,6 +1,6 @@
 """The Gram-Schmidt kernels at the sizes where their split of the work changes: rows below, at and past a
-block's rows and tile, 65536 (64 or 128 rows a block), 2^19 (one thread per row) and 2^20 (more rows than
-a block each); columns below, at and past a wavefront each, a launch's 256, and more. Against numpy in
+block's rows and tile, 65536 (workgroups of one or four wavefronts), 2^19 (a row a thread below, rows in
+strides above) and 2^20 (more rows than threads); columns below, at and past four, a launch's 256, and more. Against numpy in
 double: a sum of n products of order one rounds by less than n eps, and the results are divided by
 sqrt(n), hence 4 eps sqrt(n). dot_many_noalloc gives dot_many's bits. Every case prints its name before
 it touches the device."""

@@ -1,9 +1,9 @@
 """Where a Lanczos run ends, whatever the number of steps the device is given at a time. Two open chains of
 ka and kb spins, not coupled, one spin up in each at its end: the states reached are the ka kb placings
 of the two, and no rounding leads out of them (the other entries of every vector stay exactly zero), so
-the run breaks down at step ka kb: at one step, at, below and past a batch of 64, and where max_iter ends
-it first. What is returned of a longer run is what a run of that length returns. Every case prints its
-name before it touches the device.
+the run breaks down at step ka kb: at one step, in the first and the later batches of steps that are
+enqueued at a time, and where max_iter ends it first. What is returned of a longer run is what a run of
+that length returns. Every case prints its name before it touches the device.
 
 The last norm is rounding, below 1e-10 ||H|| while the betas before it stay above 1e-4 ||H|| (asserted);
 the Ritz values are the ka kb levels of that subspace within k ||H|| eps times the orthogonality that the

@@ -1,6 +1,5 @@
-"""The batched engine's tile schedule (which workgroup runs which tile: in order, or grouped by XCD)
-is chosen by its autotuner from timings; every schedule must give the same results bit for bit, so
-the choice never shows in a result. Pinned here through QED_SPIN_AMD_BATCH_SCHEDULE."""
+"""The batched engine's tile schedule (which workgroup runs which tile: in order, or a run of neighbouring
+tiles per XCD, the default) must never show in a result: both give the same bits. Pinned here through QED_SPIN_AMD_BATCH_SCHEDULE."""
 
 import sys
 
