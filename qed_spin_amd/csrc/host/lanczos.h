@@ -106,11 +106,14 @@ private:
     std::vector<hipEvent_t> ev_;
 };
 
-/// Bounds the steps that lie enqueued and not yet run: after a step, waits for the one `stride` to
-/// 2 stride before it (an event every stride steps, two in turn), so the device always has the next
-/// ones while a release on another thread, which waits for all that every engine stream holds
+/// Bounds the steps that lie enqueued and not yet run: every `stride` steps an event, and a wait for the
+/// event before it (two in turn), so at most 2 stride steps lie there: the device always has the next
+/// ones, while a release on another thread, which waits for all that every engine stream holds
 /// (fence_engine_streams), and the short kernels of streams that share a hardware queue wait for a few
-/// steps and not for a run.
+/// steps and not for a run. (100 mixed requests on 8 slots, mean latency: 4.73 s without a bound, 4.27
+/// with; a walk of 64 streamed blocks after them in one process 12.1 and 7.8 s.) The stride is what costs
+/// nothing: an event a step from 2^19 rows on took an estimate of 716,000 rows from 4.6 to 4.8 ms, every
+/// other step 4.65; from 2^22 on a step is long beside its event.
 class StepsInFlight {
 public:
     explicit StepsInFlight(std::size_t n)
